@@ -18,7 +18,8 @@ from . import _lib
 from . import solve as S
 from ._lib import ptr, stream_of
 
-# x: threads per row tile, or 1000 + threads for dense tiles (rows end to end)
+# x: waves with one (256) or two (1512) cells per lane; the other codes choose
+# between them by size
 X_BLOCKS = (256, 448, 512, 1256, 1512)
 # z: rows per marching segment, or an LDS tile code columns*1000 + rows
 # (8064, 4128: one cell per thread; 8096: one cell per thread with the RK

@@ -136,14 +136,13 @@ __device__ __forceinline__ double face_power(double q, int mode, PowRef* ref, bo
 __device__ __forceinline__ void flux_x_face(const double val[4],
                                             const double d3[4], double hyr,
                                             double hyt, double hv,
-                                            double F[4], int pmode = POW_PLAIN,
-                                            PowRef* ref = nullptr, bool* ok = nullptr) {
+                                            double F[4]) {
   const double rho = val[0] + hyr;
   const double ir = 1.0 / rho;
   const double u = div_rn(val[1], rho, ir);
   const double w = div_rn(val[2], rho, ir);
   const double t = div_rn(val[3] + hyt, rho, ir);
-  const double p = kC0 * face_power(rho * t, pmode, ref, ok);
+  const double p = kC0 * pow_gamma(rho * t);
   const double ru = rho * u;
   F[0] = ru - hv * d3[0];
   F[1] = (rho * (u * u) + p) - hv * d3[1];

@@ -17,13 +17,13 @@
 // receives the halo refresh of stage 1, computed from `in`) and `tmp` (the
 // reference's `state_tmp`: stage-2 interior plus the stage-3 halo refresh).
 //
-//  * x (k_dir_x<NT>): one block of NT threads per (row, tile of NT-12 cells).
-//    S, the running stage state and face fluxes live in LDS; periodic wrap
-//    replaces the halo columns at every stage. k_dir_xd<NT>: the same over
-//    the rows laid end to end, so that narrow rows fill whole blocks.
+//  * x (k_dir_x<NS>): independent waves over the rows laid end to end, K cells
+//    per lane in registers, neighbours by one-lane shifts; the periodic cells
+//    are part of the extended rows.
 //  * z, LDS tiles (k_dir_zt<CW,NT>; k_dir_zt2<CW,NR> with two cells per
-//    thread, the default): the x scheme turned on its side, CW columns per
-//    block, the wall halo rows of every stage state rebuilt from its edge row.
+//    thread): CW columns per block, S, the running stage state and the face
+//    fluxes in LDS, the wall halo rows of every stage state rebuilt from its
+//    edge row.
 //    k_dir_zt2d: the same over the column groups laid end to end.
 //  * z, marching (k_dir_z<L>): a block is three waves over 64 columns and a
 //    segment of L rows; wave s runs RK stage s+1 one row step behind the
@@ -32,6 +32,7 @@
 //    lanes past nx write the corner columns of the halo rows.
 //  * k_ens_*: the same tiles over the flattened tile list of an ensemble.
 // Block ids are remapped so that each XCD runs a contiguous range of tiles.
+#include <algorithm>
 #include <mutex>
 #include <new>
 #include <unordered_map>
@@ -93,154 +94,199 @@ __device__ __forceinline__ void wave_phase_done(int* wf, int P, int t) {
 }
 
 // ------------------------------------------------------------------ x ------
-// LDS of one x tile: S on slots 0..NT-1 (cell = i0 - 6 + slot), the running
-// stage state (S1, then S2 in place) and the face fluxes (face j between
-// slots j-1 and j).
-template <int NT>
-struct XTileLds {
-  double s0[kNv][NT];
-  double s1[kNv][NT];
-  double fl[kNv][NT];
+// The extended rows of a grid (cells -6 .. nx+5, the periodic cells the three
+// stages consume included) are laid end to end, E slots each (a multiple of K),
+// and cut into waves of W = 64 K slots every W - 12: a lane holds K cells of
+// one row in registers and runs the three stages on them. A row boundary
+// inside a wave costs no more than the wave boundary does. A slot holds a
+// correct stage-s value when it lies 2s slots inside its wave and inside its
+// own extended row (-6+2s <= cell <= nx+5-2s); values computed across a row
+// boundary are never written. The windows [6, W-6) partition the slots, so
+// every interior cell is written by one wave; halo cells are written wherever
+// they are correct (the same value). Of its neighbours a lane needs, per
+// stage, two cells before its run, one after it and the flux behind its last
+// cell: 16 doubles, shifted by one lane (DPP), no LDS traffic and no barrier.
+// The RK init S waits in the lane's own LDS slots (written once, read in
+// stages 2 and 3, no other lane looks at it), which frees 8 K registers: with
+// K = 2, 96 VGPRs instead of 114 and 5 waves per SIMD instead of 4.
+//
+// Against LDS tiles of one cell per thread (48 KB and 6 barriers per 512
+// cells; 108 doubles of LDS traffic per cell and direction, here 12) the waves
+// are bound by FP64 issue in the steady state, with the start and the tail of
+// the launch on top (2.5 of 5 waves per SIMD on average). Per launch between
+// events, 512-thread LDS tiles / these waves: 2000 x 1000 52.3 / 42.5 us,
+// 8192 x 4096 740 / 599 us (3.6 TB/s of reads and writes; a 4 GB copy reaches
+// 4.6). The cheaper power alone took the tiles from 51 to 47 us, and they
+// stayed at 42 with the power left out of a timing copy altogether.
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double x) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+  const unsigned lo =
+      (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, CTRL, 0xf, 0xf, true);
+  const unsigned hi =
+      (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+// x of lane - 1 / lane + 1 (0 at the wave's end: a state at rest)
+__device__ __forceinline__ double from_prev(double x) { return dpp_f64<0x138>(x); }
+__device__ __forceinline__ double from_next(double x) { return dpp_f64<0x130>(x); }
+
+// Two consecutive cells of a row: rows start at any multiple of 8 bytes (odd
+// nx), which a 16-byte global access takes.
+typedef double dpair __attribute__((ext_vector_type(2), aligned(8)));
+
+constexpr int kXwWaves = 4;  // waves per block (they share nothing)
+
+template <int K>
+struct XWaveLds {
+  double s[kXwWaves][K * kNv][64];
 };
 
-// The three RK stages of one x tile: row k, output cells i0 .. i0+NT-13.
-// Called by all NT threads of the block (contains barriers).
-template <int NT>
-__device__ __forceinline__ void dir_x_tile(const DirArgs& a, const Grid& g, int k, int i0,
-                                           XTileLds<NT>& sm) {
-  constexpr int H = 6, C = NT - 2 * H;
-  auto& s0 = sm.s0;
-  auto& s1 = sm.s1;
-  auto& fl = sm.fl;
-  const int nx = g.nx, prow = k + kHs, t = threadIdx.x;
-  const int cell = i0 - H + t;
-  const int cw = wrap_cell(cell, nx);
-  const long long srow = (long long)k * nx;
-  const long long rowoff = (long long)prow * g.ld;         // block-uniform
-  const unsigned bw = (unsigned)(cw + kHs) * 8u;            // byte offsets in the row
-  const unsigned bc = (unsigned)(cell + kHs) * 8u;          // (used where cell >= -2)
-  {
-    double q[4];
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) q[v] = ld_off(a.in + v * g.plane + rowoff, bw);
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) s0[v][t] = q[v];
-    if (cell == -2 || cell == -1 || cell == nx || cell == nx + 1) {
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) st_off(a.st + v * g.plane + rowoff, bc, q[v]);
-    }
-  }
-  const double hyr = a.hy_cell[prow], hyt = a.hyt_cell[prow];
-  const double src = a.src_w ? a.src_w[srow + cw] : 0.0;
-  const double id = a.id;
-  __syncthreads();
-  // face j is computed by thread j in all three stages, which keeps its
-  // stage-1 pressure power for the later stages (POW_FIRST / POW_NEXT)
-  PowRef pref;
-  // ---- stage 1: faces 2..NT-2, cells 2..NT-3, S -> s1
-  {
-    const int j = t;
-    if (j >= 2 && j <= NT - 2) {
-      double v4[4], d3[4], F[4];
-#pragma unroll
-      for (int v = 0; v < kNv; ++v)
-        recon4(s0[v][j - 2], s0[v][j - 1], s0[v][j], s0[v][j + 1], v4[v], d3[v]);
-      flux_x_face(v4, d3, hyr, hyt, a.hv, F, POW_FIRST, &pref);
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) fl[v][j] = F[v];
-    }
-  }
-  __syncthreads();
-  if (t >= 2 && t <= NT - 3) {
-    double td[4];
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) td[v] = tend_of(fl[v][t], fl[v][t + 1], a.d, id);
-    if (a.src_w) td[2] = td[2] + src;
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) s1[v][t] = s0[v][t] + a.dt1 * td[v];
-    if (a.s1 && cell >= i0 && cell < i0 + C && cell < nx) {
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) st_off(a.s1 + v * g.plane + rowoff, bc, s1[v][t]);
-    }
-  }
-  __syncthreads();
-  // ---- stage 2: faces 4..NT-4, cells 4..NT-5, s1 -> s1 (in place)
-  {
-    const int j = t;
-    bool ok = true;
-    if (j >= 4 && j <= NT - 4) {
-      double v4[4], d3[4], F[4];
-#pragma unroll
-      for (int v = 0; v < kNv; ++v)
-        recon4(s1[v][j - 2], s1[v][j - 1], s1[v][j], s1[v][j + 1], v4[v], d3[v]);
-      flux_x_face(v4, d3, hyr, hyt, a.hv, F, POW_TRY, &pref, &ok);
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) fl[v][j] = F[v];
-    }
-    if (!ok) {  // the face again with pow_pos (rare)
-      double v4[4], d3[4], F[4];
-#pragma unroll
-      for (int v = 0; v < kNv; ++v)
-        recon4(s1[v][j - 2], s1[v][j - 1], s1[v][j], s1[v][j + 1], v4[v], d3[v]);
-      flux_x_face(v4, d3, hyr, hyt, a.hv, F);
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) fl[v][j] = F[v];
-    }
-  }
-  __syncthreads();
-  if (t >= 4 && t <= NT - 5) {
-    double q[4];
+__host__ __device__ inline unsigned xw_row_slots(int nx, int K) { return (unsigned)(nx + 12 + K - 1) / K * K; }
+inline long long xw_slots(int nx, int nz, int K) { return (long long)xw_row_slots(nx, K) * nz; }
+inline int xw_blocks(int nx, int nz, int K) {
+  const long long waves = (xw_slots(nx, nz, K) - 13) / (64 * K - 12) + 1;
+  return (int)((waves + kXwWaves - 1) / kXwWaves);
+}
+
+// Wave `b` of rows rbase .. rbase+nrows-1; E = xw_row_slots(nx, K).
+template <int K>
+__device__ __forceinline__ void dir_x_wave(const DirArgs& a, const Grid& g, unsigned b,
+                                           unsigned E, int rbase, int nrows,
+                                           double (*init)[64]) {
+  constexpr int W = 64 * K, C = W - 12;
+  const int nx = g.nx, lane = threadIdx.x & 63;
+  const unsigned slot0 = b * (unsigned)C;
+  const unsigned row0 = __builtin_amdgcn_readfirstlane(slot0 / E);
+  if ((int)row0 >= nrows) return;  // the last block's spare waves
+  const unsigned rem = slot0 - row0 * E + (unsigned)(K * lane);
+  const unsigned dr0 = rem / E;
+  const int cell0 = (int)(rem - dr0 * E) - 6;
+  const bool row_ok = (int)(row0 + dr0) < nrows;  // else: past the last row, not written
+  const unsigned dr = row_ok ? dr0 : (unsigned)nrows - 1 - row0;
+  const int prow = rbase + (int)(row0 + dr) + kHs;
+  const long long rowoff = (long long)(rbase + (int)row0 + kHs) * g.ld;  // wave-uniform
+  const unsigned lrow = dr * (unsigned)g.ld + kHs;                       // the lane's row
+  const unsigned lo = (lrow + (unsigned)cell0) * 8u;
+  const bool inner = cell0 >= 0 && cell0 + K <= nx;  // no halo or padding cell
+  double s[K][4];
+  if (inner) {
 #pragma unroll
     for (int v = 0; v < kNv; ++v) {
-      const double td = tend_of(fl[v][t], fl[v][t + 1], a.d, id);
-      q[v] = td;
+      const PMW_GLOBAL char* p =
+          (const PMW_GLOBAL char*)sgpr64((unsigned long long)(a.in + v * g.plane + rowoff)) + lo;
+      if constexpr (K == 2) {
+        const dpair q = *(const PMW_GLOBAL dpair*)p;
+        s[0][v] = q.x;
+        s[K - 1][v] = q.y;
+      } else {
+        s[0][v] = *(const gdouble*)p;
+      }
     }
-    if (a.src_w) q[2] = q[2] + src;
+  } else {
 #pragma unroll
-    for (int v = 0; v < kNv; ++v) q[v] = s0[v][t] + a.dt2 * q[v];
+    for (int i = 0; i < K; ++i) {
+      const int c = cell0 + i;
+      const unsigned bw = (lrow + (unsigned)wrap_cell(c, nx)) * 8u;
 #pragma unroll
-    for (int v = 0; v < kNv; ++v) s1[v][t] = q[v];
-    // state_tmp: own cells, plus its x halos (set_bc_x of stage 3's forcing)
-    const bool own = a.tmp_interior && cell >= i0 && cell < i0 + C && cell < nx;
-    const bool halo = cell == -2 || cell == -1 || cell == nx || cell == nx + 1;
-    if (own || halo) {
+      for (int v = 0; v < kNv; ++v) s[i][v] = ld_off(a.in + v * g.plane + rowoff, bw);
+      if (row_ok && (c == -2 || c == -1 || c == nx || c == nx + 1)) {  // set_bc_x of stage 1
 #pragma unroll
-      for (int v = 0; v < kNv; ++v) st_off(a.tmp + v * g.plane + rowoff, bc, q[v]);
+        for (int v = 0; v < kNv; ++v) st_off(a.st + v * g.plane + rowoff, lo + 8u * i, s[i][v]);
+      }
     }
   }
-  __syncthreads();
-  // ---- stage 3: faces 6..NT-6, cells 6..NT-7 -> out
-  {
-    const int j = t;
-    bool ok = true;
-    if (j >= 6 && j <= NT - 6) {
-      double v4[4], d3[4], F[4];
 #pragma unroll
-      for (int v = 0; v < kNv; ++v)
-        recon4(s1[v][j - 2], s1[v][j - 1], s1[v][j], s1[v][j + 1], v4[v], d3[v]);
-      flux_x_face(v4, d3, hyr, hyt, a.hv, F, POW_TRY, &pref, &ok);
+  for (int i = 0; i < K; ++i)
 #pragma unroll
-      for (int v = 0; v < kNv; ++v) fl[v][j] = F[v];
+    for (int v = 0; v < kNv; ++v) init[i * kNv + v][lane] = s[i][v];
+  asm volatile("" ::: "memory");  // read back from LDS, not kept in registers
+  const double hyr = a.hy_cell[prow], hyt = a.hyt_cell[prow];
+  const double id = a.id;
+  const bool whole = inner && row_ok && K * lane >= 6 && K * lane + K <= W - 6;
+#pragma unroll
+  for (int stage = 0; stage < 3; ++stage) {
+    const double dts = stage == 0 ? a.dt1 : stage == 1 ? a.dt2 : a.dt3;
+    double b2[4], b1[4], nx1[4];  // cells -2, -1 and K of the lane's run
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) {
+      b1[v] = from_prev(s[K - 1][v]);
+      b2[v] = K == 1 ? from_prev(b1[v]) : from_prev(s[0][v]);
+      nx1[v] = from_next(s[0][v]);
     }
-    if (!ok) {  // the face again with pow_pos (rare)
-      double v4[4], d3[4], F[4];
+    auto update = [&](int i, const double cell[4], const double flo[4], const double fhi[4]) {
+      double td[4];
+#pragma unroll
+      for (int v = 0; v < kNv; ++v) td[v] = tend_of(flo[v], fhi[v], a.d, id);
+      if (a.src_w)
+        td[2] = td[2] + a.src_w[(long long)(prow - kHs) * nx + wrap_cell(cell0 + i, nx)];
 #pragma unroll
       for (int v = 0; v < kNv; ++v)
-        recon4(s1[v][j - 2], s1[v][j - 1], s1[v][j], s1[v][j + 1], v4[v], d3[v]);
+        s[i][v] = (stage == 0 ? cell[v] : init[i * kNv + v][lane]) + dts * td[v];
+    };
+    double F0[4], Fp[4];
+#pragma unroll
+    for (int j = 0; j < K; ++j) {  // face j, between cells j-1 and j; then cell j-1
+      double v4[4], d3[4], F[4], cur[4];
+#pragma unroll
+      for (int v = 0; v < kNv; ++v) {
+        cur[v] = s[j][v];
+        recon4(b2[v], b1[v], cur[v], j + 1 < K ? s[K - 1][v] : nx1[v], v4[v], d3[v]);
+      }
       flux_x_face(v4, d3, hyr, hyt, a.hv, F);
+      if (j == 0) {
 #pragma unroll
-      for (int v = 0; v < kNv; ++v) fl[v][j] = F[v];
+        for (int v = 0; v < kNv; ++v) F0[v] = F[v];
+      } else {
+        update(j - 1, b1, Fp, F);
+      }
+#pragma unroll
+      for (int v = 0; v < kNv; ++v) {
+        b2[v] = b1[v];
+        b1[v] = cur[v];
+        Fp[v] = F[v];
+      }
+      __builtin_amdgcn_sched_barrier(0);  // one face's values live at a time
     }
-  }
-  __syncthreads();
-  if (t >= 6 && t <= NT - 7 && cell < nx) {
-    double td[4];
+    double Fn[4];
 #pragma unroll
-    for (int v = 0; v < kNv; ++v) td[v] = tend_of(fl[v][t], fl[v][t + 1], a.d, id);
-    if (a.src_w) td[2] = td[2] + src;
+    for (int v = 0; v < kNv; ++v) Fn[v] = from_next(F0[v]);
+    update(K - 1, b1, Fp, Fn);
+    gdouble* dst = stage == 0 ? a.s1 : stage == 1 ? (a.tmp_interior ? a.tmp : nullptr) : a.out;
+    if (dst) {
+      if (whole) {
 #pragma unroll
-    for (int v = 0; v < kNv; ++v)
-      st_off(a.out + v * g.plane + rowoff, bc, s0[v][t] + a.dt3 * td[v]);
+        for (int v = 0; v < kNv; ++v) {
+          PMW_GLOBAL char* p =
+              (PMW_GLOBAL char*)sgpr64((unsigned long long)(dst + v * g.plane + rowoff)) + lo;
+          if constexpr (K == 2)
+            *(PMW_GLOBAL dpair*)p = dpair{s[0][v], s[K - 1][v]};
+          else
+            *(gdouble*)p = s[0][v];
+        }
+      } else if (row_ok) {
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+          const int c = cell0 + i, sl = K * lane + i;
+          if (sl >= 6 && sl < W - 6 && c >= 0 && c < nx) {
+#pragma unroll
+            for (int v = 0; v < kNv; ++v)
+              st_off(dst + v * g.plane + rowoff, lo + 8u * i, s[i][v]);
+          }
+        }
+      }
+    }
+    if (stage == 1 && !inner && row_ok) {  // set_bc_x of stage 3 into tmp
+#pragma unroll
+      for (int i = 0; i < K; ++i) {
+        const int c = cell0 + i, sl = K * lane + i;
+        if (sl >= 4 && sl < W - 4 && (c == -2 || c == -1 || c == nx || c == nx + 1)) {
+#pragma unroll
+          for (int v = 0; v < kNv; ++v)
+            st_off(a.tmp + v * g.plane + rowoff, lo + 8u * i, s[i][v]);
+        }
+      }
+    }
   }
 }
 
@@ -254,130 +300,27 @@ __device__ __forceinline__ void member_offset(DirArgs& a) {
   if (a.s1) a.s1 += off;
 }
 
-template <int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_dir_x(
-    DirArgs a, Grid g, int ntiles, int nreal, int per_xcd) {
-  constexpr int C = NT - 12;
-  __shared__ XTileLds<NT> sm;
+// Registers: K = 1 fits 6 waves per SIMD (78 VGPRs), K = 2 five (96).
+constexpr int xw_waves_per_simd(int K) { return K == 1 ? 6 : 5; }
+
+__device__ __forceinline__ unsigned xw_wave(int block) {
+  return __builtin_amdgcn_readfirstlane((unsigned)block * kXwWaves + (threadIdx.x >> 6));
+}
+
+// NS = slots per block: 256 (K = 1) or 512 (K = 2). A launch covers `rows`
+// rows per blockIdx.z (all of them, unless the slots would not fit 32 bits).
+template <int NS>
+__global__ __launch_bounds__(64 * kXwWaves)
+    __attribute__((amdgpu_waves_per_eu(xw_waves_per_simd(NS / 256)))) void k_dir_x(
+        DirArgs a, Grid g, unsigned E, int rows, int nreal, int per_xcd) {
+  constexpr int K = NS / 256;
+  __shared__ XWaveLds<K> sm;
   const int logical = xcd_logical(blockIdx.x, per_xcd);
-  if (logical >= nreal) return;  // whole block, before any barrier
+  if (logical >= nreal) return;
   member_offset(a);
-  dir_x_tile<NT>(a, g, logical / ntiles, (logical % ntiles) * C, sm);
-}
-
-// ---- x, dense tiles: the extended rows of a grid (cells -6 .. nx+5, E = nx+12
-// slots each, the periodic cells the three stages consume included) laid end
-// to end and cut into blocks of NT slots every NT-12. A row boundary inside a
-// block costs no more than the block boundary does, so narrow rows (200, 400
-// cells) fill the blocks instead of leaving a partial tile per row. A slot
-// holds a correct stage-s value when it lies 2s slots inside its block and
-// inside its own extended row (-6+2s <= cell <= nx+5-2s); values computed
-// across a row boundary are never written. Block windows [6, NT-6) partition
-// the slots, so every interior cell is written by one block; halo cells are
-// written wherever they are correct (the same value). Slot -> (row, cell)
-// takes one 32-bit division per thread.
-inline long long dense_x_slots(int nx, int nz) { return (long long)nz * (nx + 12); }
-inline int dense_x_blocks(int nx, int nz, int nt) {
-  return (int)((dense_x_slots(nx, nz) - 13) / (nt - 12)) + 1;
-}
-
-template <int NT>
-__device__ __forceinline__ void dir_xd_tile(const DirArgs& a, const Grid& g, int b,
-                                            XTileLds<NT>& sm) {
-  auto& s0 = sm.s0;
-  auto& s1 = sm.s1;
-  auto& fl = sm.fl;
-  const int nx = g.nx, nz = g.nz, t = threadIdx.x;
-  const unsigned E = (unsigned)nx + 12u;
-  const unsigned gs = (unsigned)b * (unsigned)(NT - 12) + (unsigned)t;
-  const int r = (int)(gs / E);
-  const int cell = (int)(gs - (unsigned)r * E) - 6;  // -6 .. nx+5
-  const bool row_ok = r < nz;
-  const int prow = (row_ok ? r : 0) + kHs;
-  const int cw = wrap_cell(cell, nx);
-  const bool own = row_ok && t >= 6 && t < NT - 6 && cell >= 0 && cell < nx;
-  const bool halo = row_ok && (cell == -2 || cell == -1 || cell == nx || cell == nx + 1);
-  {
-    double q[4] = {0.0, 0.0, 0.0, 0.0};
-    if (row_ok) {
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) q[v] = a.in[g.at(v, prow, cw + kHs)];
-    }
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) s0[v][t] = q[v];
-    if (halo) {
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) a.st[g.at(v, prow, cell + kHs)] = q[v];
-    }
-  }
-  // face j (between slots j-1 and j) is computed by thread j with its row's
-  // hydrostatic values; faces across a row boundary feed no correct cell
-  const double hyr = a.hy_cell[prow], hyt = a.hyt_cell[prow];
-  const double src = (a.src_w && row_ok) ? a.src_w[(long long)r * nx + cw] : 0.0;
-  const double id = a.id;
-  PowRef pref;  // this face's stage-1 pressure power, continued in stages 2 and 3
-  __syncthreads();
-#pragma unroll
-  for (int stage = 0; stage < 3; ++stage) {
-    const int m = 2 + 2 * stage;  // faces m..NT-m, cells m..NT-1-m
-    auto& src_s = stage == 0 ? s0 : s1;
-    bool ok = true;
-    if (t >= m && t <= NT - m) {
-      double v4[4], d3[4], F[4];
-#pragma unroll
-      for (int v = 0; v < kNv; ++v)
-        recon4(src_s[v][t - 2], src_s[v][t - 1], src_s[v][t], src_s[v][t + 1], v4[v], d3[v]);
-      flux_x_face(v4, d3, hyr, hyt, a.hv, F, stage == 0 ? POW_FIRST : POW_TRY, &pref, &ok);
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) fl[v][t] = F[v];
-    }
-    if (!ok) {  // the face again with pow_pos (rare)
-      double v4[4], d3[4], F[4];
-#pragma unroll
-      for (int v = 0; v < kNv; ++v)
-        recon4(src_s[v][t - 2], src_s[v][t - 1], src_s[v][t], src_s[v][t + 1], v4[v], d3[v]);
-      flux_x_face(v4, d3, hyr, hyt, a.hv, F);
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) fl[v][t] = F[v];
-    }
-    __syncthreads();
-    if (t >= m && t <= NT - 1 - m) {
-      const double dts = stage == 0 ? a.dt1 : stage == 1 ? a.dt2 : a.dt3;
-      double q[4];
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) q[v] = tend_of(fl[v][t], fl[v][t + 1], a.d, id);
-      if (a.src_w) q[2] = q[2] + src;
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) q[v] = s0[v][t] + dts * q[v];
-      if (stage < 2) {
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) s1[v][t] = q[v];  // in place: faces are done
-      }
-      if (stage == 0 && a.s1 && own) {
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) a.s1[g.at(v, prow, cell + kHs)] = q[v];
-      }
-      if (stage == 1 && ((own && a.tmp_interior) || halo)) {
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) a.tmp[g.at(v, prow, cell + kHs)] = q[v];
-      }
-      if (stage == 2 && own) {
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) a.out[g.at(v, prow, cell + kHs)] = q[v];
-      }
-    }
-    if (stage < 2) __syncthreads();
-  }
-}
-
-template <int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_dir_xd(
-    DirArgs a, Grid g, int nreal, int per_xcd) {
-  __shared__ XTileLds<NT> sm;
-  const int logical = xcd_logical(blockIdx.x, per_xcd);
-  if (logical >= nreal) return;  // whole block, before any barrier
-  member_offset(a);
-  dir_xd_tile<NT>(a, g, logical, sm);
+  const int rbase = (int)blockIdx.z * rows;
+  dir_x_wave<K>(a, g, xw_wave(logical), E, rbase, min(rows, g.nz - rbase),
+                sm.s[threadIdx.x >> 6]);
 }
 
 // ------------------------------------------------------------------ z ------
@@ -662,7 +605,16 @@ __global__ __launch_bounds__(192) void k_dir_z(DirArgs a, Grid g, int ncolblk, i
 }
 
 // ------------------------------------------------------------- z tiles --
-// LDS of a one-cell-per-thread z tile: the x tile's arrays and the tile
+// LDS arrays of the one-cell z tiles: S, the running stage state and the face
+// fluxes, one entry per slot.
+template <int NT>
+struct XTileLds {
+  double s0[kNv][NT];
+  double s1[kNv][NT];
+  double fl[kNv][NT];
+};
+
+// LDS of a one-cell-per-thread z tile: those arrays and the tile
 // rows' face hydrostatics (rho, rho*theta, p at the lower face of each tile
 // row), read from HBM once per tile; all CW columns of a row read one word.
 template <int NT, int NR>
@@ -1430,7 +1382,7 @@ struct MemberDev {
   double dx, dz, dt1, dt2, dt3, hvx, hvz;
   double idx, idz;       // RN(1/dx), RN(1/dz)
   int x_start, z_start;  // first work item of this member in the x / z lists
-  int x_ntiles, z_ncol;  // x tiles per row (dense x tiles: blocks of the member), z column groups
+  int x_blocks, z_ncol;  // blocks of the member's x waves, z column groups
 };
 
 __device__ __forceinline__ DirArgs member_args(const MemberDev& m, int dir, int pass,
@@ -1480,32 +1432,20 @@ __device__ __forceinline__ int member_of(const MemberDev* m, int n, int item) {
 // VGPRs live and halved the occupancy.) `pass`: bit 0 = direction of the
 // step (0: state -> work, 1: work -> state), bit 1 = store state_tmp's
 // interior (the last direction of the call only).
-template <int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_ens_x(const MemberDev* __restrict__ m, int n, int pass,
-                                              int total, int per_xcd) {
-  constexpr int C = NT - 12;
-  __shared__ XTileLds<NT> sm;
+template <int NS>
+__global__ __launch_bounds__(64 * kXwWaves)
+    __attribute__((amdgpu_waves_per_eu(xw_waves_per_simd(NS / 256)))) void k_ens_x(
+        const MemberDev* __restrict__ m, int n, int pass, int total, int per_xcd) {
+  constexpr int K = NS / 256;
+  __shared__ XWaveLds<K> sm;
   const int item = xcd_logical(blockIdx.x, per_xcd);
-  if (item >= total) return;  // whole block, before any barrier
+  if (item >= total) return;
   const MemberDev& md = m[member_of<0>(m, n, item)];
   const DirArgs a = member_args(md, 0, pass & 1, pass >> 1);
   const int local = item - md.x_start;
-  const int row = local / md.x_ntiles;
-  if (row >= md.nz) return;  // a plan that is not the prepared one: stay in bounds
-  dir_x_tile<NT>(a, Grid(md.nx, md.nz), row, (local % md.x_ntiles) * C, sm);
-}
-
-template <int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_ens_xd(const MemberDev* __restrict__ m, int n, int pass,
-                                               int total, int per_xcd) {
-  __shared__ XTileLds<NT> sm;
-  const int item = xcd_logical(blockIdx.x, per_xcd);
-  if (item >= total) return;  // whole block, before any barrier
-  const MemberDev& md = m[member_of<0>(m, n, item)];
-  const DirArgs a = member_args(md, 0, pass & 1, pass >> 1);
-  const int local = item - md.x_start;
-  if (local >= md.x_ntiles) return;  // as in k_ens_x
-  dir_xd_tile<NT>(a, Grid(md.nx, md.nz), local, sm);
+  if (local >= md.x_blocks) return;  // a plan that is not the prepared one: stay in bounds
+  dir_x_wave<K>(a, Grid(md.nx, md.nz), xw_wave(local), xw_row_slots(md.nx, K), 0, md.nz,
+                sm.s[threadIdx.x >> 6]);
 }
 
 template <int L>
@@ -1632,22 +1572,17 @@ int launch_zt2d(const DirArgs& a, Grid g, hipStream_t st, int members) {
   return PMW_OK;
 }
 
-template <int NT>
+template <int K>
 int launch_x(const DirArgs& a, Grid g, hipStream_t st, int members) {
-  constexpr int C = NT - 12;
-  const int ntiles = (g.nx + C - 1) / C;
-  const long long nreal = (long long)ntiles * g.nz;
-  const int per = (int)((nreal + kNumXcd - 1) / kNumXcd);
-  k_dir_x<NT><<<dim3(per * kNumXcd, members), NT, 0, st>>>(a, g, ntiles, (int)nreal, per);
-  PMW_CHECK_LAUNCH();
-  return PMW_OK;
-}
-
-template <int NT>
-int launch_xd(const DirArgs& a, Grid g, hipStream_t st, int members) {
-  const int nreal = dense_x_blocks(g.nx, g.nz, NT);
+  const unsigned E = xw_row_slots(g.nx, K);
+  // slots are 32-bit: rows beyond 2^31 of them go to further blockIdx.z
+  const int rows = (int)std::min<long long>(g.nz, std::max(1LL, (1LL << 31) / E));
+  const int chunks = (g.nz + rows - 1) / rows;
+  if (chunks > 65535) return PMW_EINVAL;
+  const int nreal = xw_blocks(g.nx, rows, K);
   const int per = (nreal + kNumXcd - 1) / kNumXcd;
-  k_dir_xd<NT><<<dim3(per * kNumXcd, members), NT, 0, st>>>(a, g, nreal, per);
+  k_dir_x<256 * K><<<dim3(per * kNumXcd, members, chunks), 64 * kXwWaves, 0, st>>>(
+      a, g, E, rows, nreal, per);
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
@@ -1679,10 +1614,24 @@ int launch_z(const DirArgs& a, Grid g, hipStream_t st, int members) {
 
 namespace pmw {
 
-// x: 256, 448, 512 = threads per row tile; 1000 + 256 or 512 = dense tiles
 bool fused_x_tile_ok(int nt) {
   return nt == 256 || nt == 448 || nt == 512 || nt == 1256 || nt == 1512;
 }
+
+// Cells per lane of the x waves for a launch over `cells` cells: code 256
+// forces one, 1512 two; the other codes go by size. Two cells waste 10 % of
+// the slots on wave overlap instead of 23 % and halve the neighbour exchange
+// per cell, but each wave takes twice as long: one cell per lane is faster
+// while all its waves (one per 52 slots) fit the 6 x 1024 the GPU holds at
+// once. Step time in us, one / two cells per lane (x kernel: see above):
+// 400x200 17.9 / 18.7, 800x400 (just over one round of waves) 28.9 / 27.3,
+// 1003x517 39.1 / 40.4, 1200x600 47.7 / 47.9, 1500x750 66.6 / 63.6,
+// 2000x1000 104.8 / 99.2.
+int fused_x_cells(int nt, long long cells) {
+  if (nt == 256 || nt == 1512) return nt == 256 ? 1 : 2;
+  return cells <= 300000 ? 1 : 2;
+}
+
 // z: 8..64 = rows per marching segment; columns*1000 + rows = LDS tiles:
 // 8064, 4128 (one cell per thread, RK init in LDS), 8096 (one cell per
 // thread, RK init in registers, stage state updated in place), 8128 (two
@@ -1694,15 +1643,11 @@ bool fused_z_seg_ok(int seg) {
 
 int launch_dir_x(const DirArgs& a, Grid g, int nt, hipStream_t st, int members) {
   if (members < 1 || members > 65535 || (members > 1 && a.mstride <= 0)) return PMW_EINVAL;
-  if (nt > 1000 && dense_x_slots(g.nx, g.nz) > (1LL << 30)) return PMW_EINVAL;
-  switch (nt) {
-    case 256: return launch_x<256>(a, g, st, members);
-    case 448: return launch_x<448>(a, g, st, members);
-    case 512: return launch_x<512>(a, g, st, members);
-    case 1256: return launch_xd<256>(a, g, st, members);
-    case 1512: return launch_xd<512>(a, g, st, members);
-    default: return PMW_EINVAL;
-  }
+  if (!fused_x_tile_ok(nt)) return PMW_EINVAL;
+  if (nt > 1000 && (long long)g.nz * (g.nx + 12) > (1LL << 30)) return PMW_EINVAL;
+  return fused_x_cells(nt, (long long)g.nx * g.nz * members) == 1
+             ? launch_x<1>(a, g, st, members)
+             : launch_x<2>(a, g, st, members);
 }
 
 int launch_dir_z(const DirArgs& a, Grid g, int seg, hipStream_t st, int members) {
@@ -1733,15 +1678,16 @@ int launch_dir_z(const DirArgs& a, Grid g, int seg, hipStream_t st, int members)
 // ============================================================ ensemble ABI ==
 namespace {
 
-int ens_x_cells(int nt) { return nt - 12; }
-
 struct EnsPlan {
   int x_total, z_total;
+  int x_k;  // cells per lane of the x waves
 };
 
 int plan_members(const pmw_member* mem, int n, int x_nt, int z_seg, MemberDev* dev,
                  EnsPlan& plan) {
-  long long xs = 0, zs = 0;
+  long long xs = 0, zs = 0, cells = 0;
+  for (int q = 0; q < n; ++q) cells += (long long)mem[q].nx * mem[q].nz;
+  plan.x_k = pmw::fused_x_cells(x_nt, cells);
   for (int q = 0; q < n; ++q) {
     const pmw_member& m = mem[q];
     if (m.nx < 2 || m.nz < 2 || !m.state || !m.state_tmp || !m.state_work ||
@@ -1750,10 +1696,10 @@ int plan_members(const pmw_member* mem, int n, int x_nt, int z_seg, MemberDev* d
       return PMW_EINVAL;
     if (m.state == m.state_tmp || m.state == m.state_work || m.state_tmp == m.state_work)
       return PMW_EALIAS;
-    const bool dense = x_nt > 1000;
-    if (dense && dense_x_slots(m.nx, m.nz) > (1LL << 30)) return PMW_EINVAL;
-    const int xt = dense ? dense_x_blocks(m.nx, m.nz, x_nt - 1000)
-                         : (m.nx + ens_x_cells(x_nt) - 1) / ens_x_cells(x_nt);
+    if ((x_nt > 1000 && (long long)m.nz * (m.nx + 12) > (1LL << 30)) ||
+        xw_slots(m.nx, m.nz, plan.x_k) > (1LL << 32) - 1024)
+      return PMW_EINVAL;
+    const int xt = xw_blocks(m.nx, m.nz, plan.x_k);
     int zc, zsg;
     if (z_seg == 18128 || z_seg == 18096) {  // dense tiles: zc = the member's blocks, one "segment"
       if (dense_z_rows(m.nx, m.nz, 8) > (1LL << 30)) return PMW_EINVAL;
@@ -1791,10 +1737,10 @@ int plan_members(const pmw_member* mem, int n, int x_nt, int z_seg, MemberDev* d
       d.hvz = -kHvBeta * m.dz / (16 * m.dt_full);
       d.x_start = (int)xs;
       d.z_start = (int)zs;
-      d.x_ntiles = xt;
+      d.x_blocks = xt;
       d.z_ncol = zc;
     }
-    xs += dense ? (long long)xt : (long long)xt * m.nz;  // dense: blocks, else tiles x rows
+    xs += xt;
     zs += (long long)zc * zsg;
     if (xs > (1LL << 30) || zs > (1LL << 30)) return PMW_EINVAL;
   }
@@ -1849,18 +1795,10 @@ EnsPrepared prepared_for(const pmw_member* m, int n, int x_nt, int z_seg,
 
 inline int ens_per_xcd(int total) { return (total + kNumXcd - 1) / kNumXcd; }
 
-template <int NT>
+template <int K>
 int launch_ens_x(const MemberDev* d, int n, int pass, int total, hipStream_t st) {
   const int per = ens_per_xcd(total);
-  k_ens_x<NT><<<per * kNumXcd, NT, 0, st>>>(d, n, pass, total, per);
-  PMW_CHECK_LAUNCH();
-  return PMW_OK;
-}
-
-template <int NT>
-int launch_ens_xd(const MemberDev* d, int n, int pass, int total, hipStream_t st) {
-  const int per = ens_per_xcd(total);
-  k_ens_xd<NT><<<per * kNumXcd, NT, 0, st>>>(d, n, pass, total, per);
+  k_ens_x<256 * K><<<per * kNumXcd, 64 * kXwWaves, 0, st>>>(d, n, pass, total, per);
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
@@ -1913,14 +1851,11 @@ int launch_ens_zt(const MemberDev* d, int n, int pass, int total, hipStream_t st
   return PMW_OK;
 }
 
-int launch_ens(int dir, int x_nt, int z_seg, const MemberDev* d, int n, int pass,
+int launch_ens(int dir, int z_seg, const MemberDev* d, int n, int pass,
                const EnsPlan& plan, hipStream_t st) {
   if (dir == 0) {
-    if (x_nt == 256) return launch_ens_x<256>(d, n, pass, plan.x_total, st);
-    if (x_nt == 448) return launch_ens_x<448>(d, n, pass, plan.x_total, st);
-    if (x_nt == 1256) return launch_ens_xd<256>(d, n, pass, plan.x_total, st);
-    if (x_nt == 1512) return launch_ens_xd<512>(d, n, pass, plan.x_total, st);
-    return launch_ens_x<512>(d, n, pass, plan.x_total, st);
+    return plan.x_k == 1 ? launch_ens_x<1>(d, n, pass, plan.x_total, st)
+                         : launch_ens_x<2>(d, n, pass, plan.x_total, st);
   }
   switch (z_seg) {
     case 8: return launch_ens_z<8>(d, n, pass, plan.z_total, st);
@@ -2024,7 +1959,7 @@ int pmw_ensemble_evolve(const pmw_member* members, int nmembers, const int* tuni
       }
       // state_tmp's interior: only the call's last direction keeps its stores
       const int keep_tmp = pass == 1 && step == nsteps - 1;
-      rc = launch_ens(dir, x_nt, z_seg, d, nmembers, pass | keep_tmp << 1, plan, st);
+      rc = launch_ens(dir, z_seg, d, nmembers, pass | keep_tmp << 1, plan, st);
       if (kernel_ms && rc == PMW_OK) {
         hipError_t e = hipEventRecord(ev[1], st);
         float ms = 0.f;
