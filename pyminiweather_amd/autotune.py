@@ -2,8 +2,8 @@
 
 For one grid (or one ensemble) it times every candidate shape with HIP
 events around each launch (``pmw_evolve_ex`` / ``pmw_ensemble_evolve``
-``kernel_ms``) and keeps, independently, the fastest x block size and the
-fastest z segment length (the two directions are separate launches), then
+``kernel_ms``) and keeps, independently, the fastest x code and the fastest
+z code (the two directions are separate launches), then
 checks the fused choice against one launch per RK stage. Single grids are
 timed on scratch copies of the state, so tuning does not advance the
 solution; ensembles are timed in place (tuning advances them, like warm-up
@@ -21,10 +21,8 @@ from ._lib import ptr, stream_of
 # x: waves with one (256) or two (1512) cells per lane; the other codes choose
 # between them by size
 X_BLOCKS = (256, 448, 512, 1256, 1512)
-# z: rows per marching segment, or an LDS tile code columns*1000 + rows
-# (8064, 4128: one cell per thread; 8096: one cell per thread with the RK
-# init in registers; 8128: two cells per thread; 18128 / 18096: 8128 /
-# 8096 as dense tiles, column groups end to end)
+# z: 8..64 one-cell tiles of 32 rows, 18096 / 18128 dense one-cell tiles of 96
+# rows; the other codes choose by size
 Z_SEGMENTS = (8, 16, 24, 32, 48, 64, 8064, 4128, 8096, 8128, 18128, 18096)
 
 

@@ -20,17 +20,11 @@
 //  * x (k_dir_x<NS>): independent waves over the rows laid end to end, K cells
 //    per lane in registers, neighbours by one-lane shifts; the periodic cells
 //    are part of the extended rows.
-//  * z, LDS tiles (k_dir_zt<CW,NT>; k_dir_zt2<CW,NR> with two cells per
-//    thread): CW columns per block, S, the running stage state and the face
-//    fluxes in LDS, the wall halo rows of every stage state rebuilt from its
-//    edge row.
-//    k_dir_zt2d: the same over the column groups laid end to end.
-//  * z, marching (k_dir_z<L>): a block is three waves over 64 columns and a
-//    segment of L rows; wave s runs RK stage s+1 one row step behind the
-//    previous stage, rows handed over through a 2-slot LDS ring with one
-//    barrier per step. Wall halo rows are synthesised in registers. Extra
-//    lanes past nx write the corner columns of the halo rows.
-//  * k_ens_*: the same tiles over the flattened tile list of an ensemble.
+//  * z, LDS tiles: k_dir_zt1<NW,NR> with three rows per thread in registers,
+//    k_dir_z1<NR> with one cell per thread (small grids, low columns) and
+//    k_dir_z1d<NR>, the same over the column groups laid end to end. The wall
+//    halo rows of every stage state are rebuilt from its edge row.
+//  * k_ens_*: the same over the flattened tile list of an ensemble.
 // Block ids are remapped so that each XCD runs a contiguous range of tiles.
 #include <algorithm>
 #include <mutex>
@@ -324,358 +318,85 @@ __global__ __launch_bounds__(64 * kXwWaves)
 }
 
 // ------------------------------------------------------------------ z ------
-// Face k of a z stage from the window rows k-2..k+1 (w[0..3]).
-__device__ __forceinline__ void z_face(const double w[4][4], const DirArgs& a, int k,
-                                       int nz, double G[4]) {
-  double v4[4], d3[4];
-#pragma unroll
-  for (int v = 0; v < kNv; ++v) recon4(w[0][v], w[1][v], w[2][v], w[3][v], v4[v], d3[v]);
-  flux_z_face(v4, d3, a.hyr_int[k], a.hyt_int[k], a.hyp_int[k], a.hv, k == 0 || k == nz, G);
-}
+// z tiles, three rows per thread (k_dir_zt1): a block of NW waves holds 16
+// columns x NR rows (slot row r of column c in thread (r/3)*16 + c), the
+// running stage state and S in registers; LDS only carries what threads of
+// neighbouring rows need of each other: the first and the last two rows of
+// each thread's three and the flux at its first face (14 doubles of LDS
+// traffic per cell and stage instead of the 33 of one cell per thread), and
+// the rows' face hydrostatics. A wave holds 12 whole rows, and every phase
+// reads and writes only the wave's rows and those of its neighbours, so the
+// phases are ordered by the waves' flags (wave_phase_done).
+//
+// Rows of the tiles: the first holds rows -2 .. NR-3 of the column, the last
+// rows nz+2-NR .. nz+1, so that a wall's halo rows share a thread with their
+// edge row and set_bc_z between the stages stays in one thread's registers;
+// the tiles between start 6 rows before the first row they own. Next to a wall nothing is lost to the
+// stencil, so the first and last own NR - 8 rows, the others NR - 12. Tiles
+// overlap where nz does not divide; each row has one owner. Tiles of one row
+// of blocks are neighbours along x (their 128-byte rows straddle cache lines,
+// which then meet in one XCD's L2).
+//
+// Measured (between events, one cell per thread with the RK init in registers
+// / this): 2000 x 1000 63.2 / 55 us, 8192 x 4096 980 / 867 us. Three rows per thread fit
+// 128 VGPRs (4 waves per SIMD, two 66 KB blocks per CU). Same boxes, not kept:
+// 8 columns x 96 rows in 256 threads 58 and 1200 us (64-byte rows), 4 rows per
+// thread (x 24 row groups) 73 and 1190 us, 6 rows (2 waves per SIMD) 53 and 874
+// us, 2 columns per wave without LDS 127 and 2740 us; block barriers instead of
+// the flags 50.4 and 801 us against 50.0 and 786.
+template <int NW, int NR>
+struct ZTileLds {
+  static constexpr int NT = 64 * NW;
+  double lo[kNv][NT];  // each thread's first row,
+  double h1[kNv][NT];  // its last row
+  double h2[kNv][NT];  // and the one before
+  double f0[kNv][NT];  // flux at its first face
+  double hz[3][NR];    // rho, rho*theta, p at the rows' lower faces
+  int wf[NW + 2];      // wave phase flags
+};
 
-__device__ __forceinline__ void shift4(double w[4][4]) {
-#pragma unroll
-  for (int p = 0; p < 3; ++p)
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) w[p][v] = w[p + 1][v];
-}
+constexpr int kZtCols = 16, kZtK = 3, kZtWaves = 8, kZtRows = 96;
 
-// Halo row values of set_bc_z from an edge row e (padded row pe) into halo
-// padded row ph.
-__device__ __forceinline__ void wall_row(const double e[4], const double* hy, int pe,
-                                         int ph, double out[4]) {
-#pragma unroll
-  for (int v = 0; v < kNv; ++v) out[v] = wall_halo(v, e[v], hy[pe], hy[ph]);
-}
+template <int NR>
+struct ZTileRows {
+  static constexpr int C = NR - 12, CE = NR - 8;  // rows owned: inside, at a wall
+  static __host__ __device__ int tiles(int nz) {
+    return nz <= 2 * CE ? 2 : 2 + (nz - 2 * CE + C - 1) / C;
+  }
+};
 
-// One step of one z stage for one lane. The window slot of input row
-// base + p (p = 0..3) is (PH + 1 + p) & 3 where PH = step & 3, so advancing a
-// row changes the phase instead of copying registers. Input row r arrives,
-// face r-1 and cell r-2 are finished. Returns true and the cell's new value
-// in `res` when a cell was finished.
-template <int PH, int stage>
-__device__ __forceinline__ bool z_stage_step(double w[4][4], double F[4], const DirArgs& a,
-                                             const Grid& g, int r, int lo,
-                                             int hi, int pc, int i, const double* lds_row,
-                                             const double cur[4], double dts, double res[4]) {
-  constexpr int S0 = (PH + 1) & 3, S1 = (PH + 2) & 3, S2 = (PH + 3) & 3, S3 = PH & 3;
-  const int nz = g.nz;
+template <int NW, int NR>
+__device__ __forceinline__ void dir_zt1_tile(const DirArgs& a, const Grid& g, int tile, int ntile,
+                                             int c0, ZTileLds<NW, NR>& sm, bool corners) {
+  constexpr int NT = 64 * NW, CW = kZtCols, K = kZtK, NG = NT / CW;
+  constexpr int C = ZTileRows<NR>::C, CE = ZTileRows<NR>::CE;
+  static_assert(NG * K == NR && NT >= NR, "three rows per thread");
+  const int nx = g.nx, nz = g.nz, t = threadIdx.x;
+  const int col = t % CW, rg = t / CW;
   const gdouble* hy = a.hy_cell;
-  // the new row is formed in nv and stored once, so that every window slot
-  // is written through a static index (no merged private-array stores)
-  if (r >= lo - 2 && r <= hi + 1 && r < nz + 2) {
-    double nv[4];
-    if (r >= 0 && r < nz) {
-      if (stage == 0) {
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) nv[v] = cur[v];  // row r, loaded a step ahead
-      } else {
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) nv[v] = lds_row[v * 64];
-      }
-    } else if (r == nz) {
-      wall_row(w[S2], hy, nz + 1, nz + 2, nv);
-    } else {  // r == nz + 1, or r < 0 (rows -2, -1: refreshed when row 0 arrives)
-      wall_row(w[S1], hy, nz + 1, nz + 3, nv);
-    }
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) w[S3][v] = nv[v];
-    if (r == 0) {
-      double h1[4], h2[4];
-      wall_row(nv, hy, kHs, 0, h1);
-      wall_row(nv, hy, kHs, 1, h2);
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) {
-        w[S1][v] = h1[v];
-        w[S2][v] = h2[v];
-      }
-    }
+  const int plo = kHs, phi = nz + kHs - 1;
+  const bool first = tile == 0, last = tile == ntile - 1;
+  const int base = first ? -2 : last ? nz + 2 - NR : CE + (tile - 1) * C - 6;
+  const int own0 = first ? 0 : last ? nz - CE : base + 6;
+  const int own1 = last ? nz : min(first ? CE : base + 6 + C, nz - CE);
+  wave_flags_init(sm.wf, NW, t);
+  if (t < NR) {
+    const int k = min(max(base + t, 0), nz);
+    sm.hz[0][t] = a.hyr_int[k];
+    sm.hz[1][t] = a.hyt_int[k];
+    sm.hz[2][t] = a.hyp_int[k];
   }
-  const int f = r - 1;
-  bool done = false;
-  // RK init of the cell this step may finish (row r-2; clamped so the load
-  // is always in bounds), issued before the face so its latency overlaps it
-  double iv[4];
-  if (stage > 0) {
-    const int cc = min(max(r - 2, 0), nz - 1);
+  const int k0 = base + rg * K;  // the thread's first row
+  const bool colok = c0 + col < nx;
+  const int lcol = colok ? col : nx - 1 - c0;
+  const long long ubase = (long long)(base + kHs) * g.ld + c0 + kHs;  // block-uniform
+  const unsigned lo = ((unsigned)(rg * K) * (unsigned)g.ld + (unsigned)lcol) * 8u;
+  double S[K][4], s[K][4];
 #pragma unroll
-    for (int v = 0; v < kNv; ++v) iv[v] = a.in[g.at(v, cc + kHs, pc)];
-  }
-  if (f >= lo && f <= hi) {
-    double v4[4], d3[4], G[4];
+  for (int j = 0; j < K; ++j)
 #pragma unroll
     for (int v = 0; v < kNv; ++v)
-      recon4(w[S0][v], w[S1][v], w[S2][v], w[S3][v], v4[v], d3[v]);
-    flux_z_face(v4, d3, a.hyr_int[f], a.hyt_int[f], a.hyp_int[f], a.hv, f == 0 || f == nz, G);
-    const int c = f - 1;  // window row 1
-    if (c >= lo) {
-      const double id = a.id;
-      double td[4];
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) td[v] = tend_of(F[v], G[v], a.d, id);
-      td[2] = td[2] - w[S1][0] * kGrav;
-      if (a.src_w) td[2] = td[2] + a.src_w[(long long)c * g.nx + i];
-      if (stage == 0) {
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) res[v] = w[S1][v] + dts * td[v];
-      } else {
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) res[v] = iv[v] + dts * td[v];
-      }
-      done = true;
-    }
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) F[v] = G[v];
-  }
-  return done;
-}
-
-__device__ __forceinline__ void store_row(gdouble* buf, const Grid& g, int prow, int pc,
-                                          const double q[4]) {
-#pragma unroll
-  for (int v = 0; v < kNv; ++v) buf[g.at(v, prow, pc)] = q[v];
-}
-
-// Body of one step j for the wave of `stage` (0, 1, 2 = RK stage 1, 2, 3).
-template <int PH, int stage>
-__device__ __forceinline__ void z_block_step(double w[4][4], double F[4], const DirArgs& a,
-                                             const Grid& g, double (*ring)[2][kNv][64],
-                                             int j, int lo, int hi, int k0,
-                                             int k1, int pc, int i, int lane, bool active,
-                                             const double cur[4], double dts) {
-  const int nz = g.nz;
-  const gdouble* hy = a.hy_cell;
-  const int r = j - 3 * stage;  // input row of this stage at step j
-  if (active) {
-    // rows of S1 / S2 come from the previous stage's ring (written one step ago)
-    const double* lds_row = stage > 0 ? &ring[stage - 1][r & 1][0][lane] : nullptr;
-    double res[4];
-    const bool done =
-        z_stage_step<PH, stage>(w, F, a, g, r, lo, hi, pc, i, lds_row, cur, dts, res);
-    if (stage == 0 && r == 0 && k0 == 0) {  // set_bc_z of stage 1 into st
-      double h[4];
-      wall_row(w[PH & 3], hy, kHs, 0, h);
-      store_row(a.st, g, 0, pc, h);
-      wall_row(w[PH & 3], hy, kHs, 1, h);
-      store_row(a.st, g, 1, pc, h);
-    }
-    if (stage == 0 && r == nz - 1 && k1 == nz && r >= lo - 2) {
-      double h[4];
-      wall_row(w[PH & 3], hy, nz + 1, nz + 2, h);
-      store_row(a.st, g, nz + 2, pc, h);
-      wall_row(w[PH & 3], hy, nz + 1, nz + 3, h);
-      store_row(a.st, g, nz + 3, pc, h);
-    }
-    if (done) {
-      const int c = r - 2;
-      if (stage < 2) {
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) ring[stage][c & 1][v][lane] = res[v];
-      }
-      if (stage == 0 && a.s1 && c >= k0 && c < k1) store_row(a.s1, g, c + kHs, pc, res);
-      if (stage == 1) {
-        if (a.tmp_interior && c >= k0 && c < k1) store_row(a.tmp, g, c + kHs, pc, res);
-        if (c == 0 && k0 == 0) {  // set_bc_z of stage 3 into tmp
-          double h[4];
-          wall_row(res, hy, kHs, 0, h);
-          store_row(a.tmp, g, 0, pc, h);
-          wall_row(res, hy, kHs, 1, h);
-          store_row(a.tmp, g, 1, pc, h);
-        }
-        if (c == nz - 1 && k1 == nz) {
-          double h[4];
-          wall_row(res, hy, nz + 1, nz + 2, h);
-          store_row(a.tmp, g, nz + 2, pc, h);
-          wall_row(res, hy, nz + 1, nz + 3, h);
-          store_row(a.tmp, g, nz + 3, pc, h);
-        }
-      }
-      if (stage == 2) store_row(a.out, g, c + kHs, pc, res);
-    }
-  }
-  __syncthreads();
-}
-
-// March of one stage's wave over steps j0..j1 (one barrier per step; all
-// three waves of the block run the same number of steps).
-template <int stage>
-__device__ __forceinline__ void z_march(const DirArgs& a, const Grid& g,
-                                        double (*ring)[2][kNv][64], int j0, int j1, int lo,
-                                        int hi, int k0, int k1, int pc, int i, int lane,
-                                        bool active, double dts) {
-  double w[4][4], F[4];
-#pragma unroll
-  for (int p = 0; p < 4; ++p)
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) w[p][v] = 0.0;
-#pragma unroll
-  for (int v = 0; v < kNv; ++v) F[v] = 0.0;
-  // stage 0 reads S row j at step j: keep the next row's load in flight
-  const int nz = g.nz;
-  double pre[4] = {0.0, 0.0, 0.0, 0.0};
-  if (stage == 0 && active) {
-    const int rr = min(max(j0, 0), nz - 1);
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) pre[v] = a.in[g.at(v, rr + kHs, pc)];
-  }
-#pragma unroll 1
-  for (int j = j0; j <= j1; ++j) {
-    // slot p holds row r-3+p once the step's row has arrived in slot 3
-#pragma unroll
-    for (int p = 0; p < 3; ++p)
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) w[p][v] = w[p + 1][v];
-    double cur[4];
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) cur[v] = pre[v];
-    if (stage == 0 && active) {
-      const int rr = min(max(j + 1, 0), nz - 1);
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) pre[v] = a.in[g.at(v, rr + kHs, pc)];
-    }
-    z_block_step<3, stage>(w, F, a, g, ring, j, lo, hi, k0, k1, pc, i, lane, active, cur, dts);
-  }
-}
-
-// z direction: a block is 3 waves over the same 64 columns and segment of L
-// output rows; wave s runs RK stage s+1. Stage s+1 consumes the rows stage s
-// produced one step earlier through a 2-slot LDS ring, so it lags by 3 rows
-// (2 for the stencil, 1 for the hand-over); one barrier per step.
-// One z block: 64 columns starting at column 64*colgrp, output rows of
-// segment `seg` (L rows). Called by all 192 threads (contains barriers).
-template <int L>
-__device__ __forceinline__ void dir_z_block(const DirArgs& a, const Grid& g, int colgrp,
-                                            int seg, double (*ring)[2][kNv][64]) {
-  const int nx = g.nx, nz = g.nz;
-  const int lane = threadIdx.x & 63;
-  // wave-uniform; readfirstlane makes that visible to the compiler so the
-  // stage's bounds and branches are scalar
-  const int stage = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int i = colgrp * 64 + lane;  // interior column
-  const int k0 = seg * L, k1 = min(k0 + L, nz);
-  const gdouble* hy = a.hy_cell;
-  if (stage == 0 && i >= nx && i < nx + 4) {
-    // corner columns of the halo rows (padded 0, 1, nx+2, nx+3) of st and tmp
-    const int q = i - nx;
-    const int cc = q < 2 ? q : nx + q;
-    const int lo = kHs, hi = nz + kHs - 1;
-    for (int pass = 0; pass < 2; ++pass) {
-      gdouble* buf = pass == 0 ? a.st : a.tmp;
-      if (k0 == 0) {
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) {
-          const double e = buf[g.at(v, lo, cc)];
-          buf[g.at(v, 0, cc)] = wall_halo(v, e, hy[lo], hy[0]);
-          buf[g.at(v, 1, cc)] = wall_halo(v, e, hy[lo], hy[1]);
-        }
-      }
-      if (k1 == nz) {
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) {
-          const double e = buf[g.at(v, hi, cc)];
-          buf[g.at(v, nz + 2, cc)] = wall_halo(v, e, hy[hi], hy[nz + 2]);
-          buf[g.at(v, nz + 3, cc)] = wall_halo(v, e, hy[hi], hy[nz + 3]);
-        }
-      }
-    }
-  }
-  const bool active = i < nx;
-  const int pc = i + kHs;
-  // output rows of each stage: [a1,b1) S1, [a2,b2) S2, [k0,k1) result
-  const int a1 = max(k0 - 4, 0), b1 = min(k1 + 4, nz);
-  const int a2 = max(k0 - 2, 0), b2 = min(k1 + 2, nz);
-  const int lo = stage == 0 ? a1 : stage == 1 ? a2 : k0;
-  const int hi = stage == 0 ? b1 : stage == 1 ? b2 : k1;
-  if (stage == 0)
-    z_march<0>(a, g, ring, a1 - 2, k1 + 7, lo, hi, k0, k1, pc, i, lane, active, a.dt1);
-  else if (stage == 1)
-    z_march<1>(a, g, ring, a1 - 2, k1 + 7, lo, hi, k0, k1, pc, i, lane, active, a.dt2);
-  else
-    z_march<2>(a, g, ring, a1 - 2, k1 + 7, lo, hi, k0, k1, pc, i, lane, active, a.dt3);
-}
-
-template <int L>
-__global__ __launch_bounds__(192) void k_dir_z(DirArgs a, Grid g, int ncolblk, int nreal,
-                                               int per_xcd) {
-  __shared__ double ring[2][2][kNv][64];
-  const int logical = xcd_logical(blockIdx.x, per_xcd);
-  if (logical >= nreal) return;  // whole block, before any barrier
-  member_offset(a);
-  dir_z_block<L>(a, g, logical % ncolblk, logical / ncolblk, ring);
-}
-
-// ------------------------------------------------------------- z tiles --
-// LDS arrays of the one-cell z tiles: S, the running stage state and the face
-// fluxes, one entry per slot.
-template <int NT>
-struct XTileLds {
-  double s0[kNv][NT];
-  double s1[kNv][NT];
-  double fl[kNv][NT];
-};
-
-// LDS of a one-cell-per-thread z tile: those arrays and the tile
-// rows' face hydrostatics (rho, rho*theta, p at the lower face of each tile
-// row), read from HBM once per tile; all CW columns of a row read one word.
-template <int NT, int NR>
-struct ZTileLds : XTileLds<NT> {
-  double hz[3][NR];
-};
-
-// z direction as LDS tiles, the x kernel's scheme turned on its side: a block
-// of NT threads holds CW columns x NR = NT/CW rows (slot t = row*CW + col,
-// tile row j = logical row r0-6+j), runs the three stages in LDS (stage 1 on
-// tile rows 2..NR-3, stage 2 on 4..NR-5, stage 3 on the NR-12 output rows)
-// and rebuilds the wall halo rows of every stage state from its edge row, as
-// set_bc_z does between the stages (ics/bcs.py:64-148). Same operations in
-// the same order as the marching kernel, so results are bitwise equal.
-template <int CW, int NT, bool CONT = true>
-__device__ __forceinline__ void dir_zt_tile(const DirArgs& a, const Grid& g, int c0, int r0,
-                                            ZTileLds<NT, NT / CW>& sm, bool corners) {
-  constexpr int NR = NT / CW, H = 6, C = NR - 2 * H;
-  auto& s0 = sm.s0;
-  auto& s1 = sm.s1;
-  auto& fl = sm.fl;
-  auto& hz = sm.hz;
-  const int nx = g.nx, nz = g.nz, t = threadIdx.x;
-  const int j = t / CW, col = t % CW;
-  const int i = c0 + col;     // interior column
-  const int k = r0 - H + j;   // logical row of this slot
-  const bool colok = i < nx;
-  const int pc = i + kHs;
-  const gdouble* hy = a.hy_cell;
-  const int plo = kHs, phi = nz + kHs - 1;  // padded edge rows
-  const bool wlo = k == -2 || k == -1, whi = k == nz || k == nz + 1;
-  const bool own = colok && k >= r0 && k < r0 + C && k < nz;
-  const bool own_lo = r0 == 0, own_hi = r0 <= nz - 1 && nz - 1 < r0 + C;
-  gdouble* const tmp_own = a.tmp_interior ? a.tmp : nullptr;
-  static_assert(NT >= NR, "one thread per tile row fills the face hydrostatics");
-  if (t < NR) {
-    const int kr = r0 - H + t;
-    const bool f = kr >= 0 && kr <= nz;
-    hz[0][t] = f ? a.hyr_int[kr] : 0.0;
-    hz[1][t] = f ? a.hyt_int[kr] : 0.0;
-    hz[2][t] = f ? a.hyp_int[kr] : 0.0;
-  }
-  {
-    double q[4] = {0.0, 0.0, 0.0, 0.0};
-    if (colok) {
-      if (k >= 0 && k < nz) {
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) q[v] = a.in[g.at(v, k + kHs, pc)];
-      } else if (wlo || whi) {
-        const int pe = wlo ? plo : phi;
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) q[v] = wall_halo(v, a.in[g.at(v, pe, pc)], hy[pe], hy[k + kHs]);
-        if ((wlo && own_lo) || (whi && own_hi)) {  // set_bc_z of stage 1 into st
-#pragma unroll
-          for (int v = 0; v < kNv; ++v) a.st[g.at(v, k + kHs, pc)] = q[v];
-        }
-      }
-    }
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) s0[v][t] = q[v];
-  }
+      S[j][v] = ld_off(a.in + v * g.plane + ubase + (long long)j * g.ld, lo);
   if (corners && t < 8) {
     // corner columns (padded 0, 1, nx+2, nx+3) of the halo rows of st, tmp
     gdouble* buf = t < 4 ? a.st : a.tmp;
@@ -691,54 +412,236 @@ __device__ __forceinline__ void dir_zt_tile(const DirArgs& a, const Grid& g, int
       buf[g.at(v, nz + 3, cc)] = wall_halo(v, f, hy[phi], hy[nz + 3]);
     }
   }
+#pragma unroll
+  for (int j = 0; j < K; ++j)
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) s[j][v] = S[j][v];
+  // the wall halo rows of the running state, also stored to dst (set_bc_z)
+  auto walls = [&](gdouble* dst) {
+    if (first && rg == 0) {  // rows -2, -1 of the thread holding row 0
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int v = 0; v < kNv; ++v) {
+          s[j][v] = wall_halo(v, s[2][v], hy[plo], hy[j]);
+          if (dst && colok) st_off(dst + v * g.plane + ubase + (long long)j * g.ld, lo, s[j][v]);
+        }
+    }
+    if (last && rg == NG - 1) {  // rows nz, nz+1 of the thread holding row nz-1
+#pragma unroll
+      for (int j = 1; j < 3; ++j)
+#pragma unroll
+        for (int v = 0; v < kNv; ++v) {
+          s[j][v] = wall_halo(v, s[0][v], hy[phi], hy[nz + 1 + j]);
+          if (dst && colok) st_off(dst + v * g.plane + ubase + (long long)j * g.ld, lo, s[j][v]);
+        }
+    }
+  };
+  auto publish = [&]() {
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) {
+      sm.lo[v][t] = s[0][v];
+      sm.h2[v][t] = s[1][v];
+      sm.h1[v][t] = s[2][v];
+    }
+  };
+  walls(a.st);
+  publish();
+  const int tp = t >= CW ? t - CW : t, tn = t + CW < NT ? t + CW : t;  // rows before, after
   const double id = a.id;
-  const double src = (a.src_w && colok && k >= 0 && k < nz) ? a.src_w[(long long)k * nx + i] : 0.0;
-  PowRef pref;  // CONT: this face's stage-1 power, continued in stages 2 and 3
-  __syncthreads();
+  __syncthreads();  // also publishes the flags
 #pragma unroll
   for (int stage = 0; stage < 3; ++stage) {
-    double (*sin)[NT] = stage == 0 ? s0 : s1;
+    const double dts = stage == 0 ? a.dt1 : stage == 1 ? a.dt2 : a.dt3;
+    gdouble* const dst = stage == 0 ? a.s1 : stage == 1 ? (a.tmp_interior ? a.tmp : nullptr) : a.out;
+    auto update = [&](int j, const double cell[4], const double flo[4], const double fhi[4]) {
+      double td[4];
+#pragma unroll
+      for (int v = 0; v < kNv; ++v) td[v] = tend_of(flo[v], fhi[v], a.d, id);
+      td[2] = td[2] - cell[0] * kGrav;
+      if (a.src_w)
+        td[2] = td[2] + a.src_w[(long long)min(max(k0 + j, 0), nz - 1) * nx + c0 + lcol];
+#pragma unroll
+      for (int v = 0; v < kNv; ++v) s[j][v] = S[j][v] + dts * td[v];
+      if (dst && colok && k0 + j >= own0 && k0 + j < own1) {
+#pragma unroll
+        for (int v = 0; v < kNv; ++v)
+          st_off(dst + v * g.plane + ubase + (long long)j * g.ld, lo, s[j][v]);
+      }
+    };
+    double b2[4], b1[4], Fp[4];  // the two rows before, the flux behind
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) {
+      b2[v] = sm.h2[v][tp];
+      b1[v] = sm.h1[v][tp];
+    }
+#pragma unroll
+    for (int j = 0; j < K; ++j) {  // face k0+j, then row k0+j-1
+      double v4[4], d3[4], F[4], cur[4];
+#pragma unroll
+      for (int v = 0; v < kNv; ++v) {
+        cur[v] = s[j][v];
+        recon4(b2[v], b1[v], cur[v], j + 1 < K ? s[j + 1 < K ? j + 1 : j][v] : sm.lo[v][tn],
+               v4[v], d3[v]);
+      }
+      const int q = rg * K + j;
+      flux_z_face(v4, d3, sm.hz[0][q], sm.hz[1][q], sm.hz[2][q], a.hv,
+                  k0 + j == 0 || k0 + j == nz, F);
+      if (j == 0) {
+#pragma unroll
+        for (int v = 0; v < kNv; ++v) sm.f0[v][t] = F[v];
+      } else {
+        update(j - 1, b1, Fp, F);
+      }
+#pragma unroll
+      for (int v = 0; v < kNv; ++v) {
+        b2[v] = b1[v];
+        b1[v] = cur[v];
+        Fp[v] = F[v];
+      }
+      __builtin_amdgcn_sched_barrier(0);  // one face's values live at a time
+    }
+    wave_phase_done(sm.wf, 2 * stage + 1, t);
+    {
+      double Fn[4];
+#pragma unroll
+      for (int v = 0; v < kNv; ++v) Fn[v] = sm.f0[v][tn];
+      update(K - 1, b1, Fp, Fn);
+    }
+    if (stage < 2) {
+      walls(stage == 1 ? a.tmp : nullptr);
+      publish();
+      wave_phase_done(sm.wf, 2 * stage + 2, t);
+    }
+  }
+}
+
+template <int NW, int NR>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void k_dir_zt1(
+    DirArgs a, Grid g, int ncol, int ntile, int per_xcd) {
+  __shared__ ZTileLds<NW, NR> sm;
+  const int logical = xcd_logical(blockIdx.x, per_xcd);
+  if (logical >= ncol * ntile) return;  // whole block, before any barrier
+  member_offset(a);
+  dir_zt1_tile<NW, NR>(a, g, logical / ncol, ntile, (logical % ncol) * kZtCols, sm, logical == 0);
+}
+
+// ---- z, one cell per thread, for small grids and low columns.
+// A block holds 8 columns x NR rows (slot t = row*8 + col, tile row j =
+// logical row r0-6+j; NR-12 rows are written), the RK init in registers and
+// the stage state updated in place; the wall halo rows of each stage state are
+// written by the edge row's thread in the update phase (no thread reads them
+// then). A wave holds 8 whole rows: phases by wave flags. NR = 32 for small
+// grids: a launch that leaves most of the GPU idle takes as long as one block,
+// and at 200 x 100 4-wave blocks (one wave per SIMD) take 10.6 us between
+// events where 12-wave blocks (NR = 96) take 12.7; NR = 24 (three waves) is
+// 0.6 us faster there and 0.7 us slower at 400 x 200.
+constexpr int kZ1Cols = 8;
+
+template <int NR>
+struct Z1Lds {
+  double s[kNv][kZ1Cols * NR];
+  double fl[kNv][kZ1Cols * NR];
+  double hz[3][NR];
+  int wf[kZ1Cols * NR / 64 + 2];
+};
+
+template <int NR>
+__device__ __forceinline__ void dir_z1_tile(const DirArgs& a, const Grid& g, int c0, int r0,
+                                            Z1Lds<NR>& sm, bool corners) {
+  constexpr int CW = kZ1Cols, NT = CW * NR, C = NR - 12;
+  auto& s = sm.s;
+  auto& fl = sm.fl;
+  auto& hz = sm.hz;
+  const int nx = g.nx, nz = g.nz, t = threadIdx.x;
+  wave_flags_init(sm.wf, NT / 64, t);
+  if (t < NR) {
+    const int k = r0 - 6 + t;
+    const bool f = k >= 0 && k <= nz;
+    hz[0][t] = f ? a.hyr_int[k] : 0.0;
+    hz[1][t] = f ? a.hyt_int[k] : 0.0;
+    hz[2][t] = f ? a.hyp_int[k] : 0.0;
+  }
+  const int col = t % CW, u = t, j = t / CW;
+  const gdouble* hy = a.hy_cell;
+  const int plo = kHs, phi = nz + kHs - 1;
+  const int k = r0 - 6 + j;
+  const int i = c0 + col;
+  const bool colok = i < nx;
+  const int pc = (colok ? i : 0) + kHs;
+  const bool wl = k == -2 || k == -1, wh = k == nz || k == nz + 1;
+  const bool own = colok && j >= 6 && j < 6 + C && k >= 0 && k < nz;
+  double S[4];
+  {
+    double q[4] = {0.0, 0.0, 0.0, 0.0};
+    if (colok) {
+      if (k >= 0 && k < nz) {
+#pragma unroll
+        for (int v = 0; v < kNv; ++v) q[v] = a.in[g.at(v, k + kHs, pc)];
+      } else if (wl || wh) {
+        const int pe = wl ? plo : phi;
+#pragma unroll
+        for (int v = 0; v < kNv; ++v) q[v] = wall_halo(v, a.in[g.at(v, pe, pc)], hy[pe], hy[k + kHs]);
+        const int je = wl ? j - k : j - (k - (nz - 1));  // the edge row's tile row
+        if (je >= 6 && je < NR - 6) {  // set_bc_z of stage 1 into st
+#pragma unroll
+          for (int v = 0; v < kNv; ++v) a.st[g.at(v, k + kHs, pc)] = q[v];
+        }
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) {
+      s[v][u] = q[v];
+      S[v] = q[v];
+    }
+  }
+  const double src = (a.src_w && colok && k >= 0 && k < nz) ? a.src_w[(long long)k * nx + i] : 0.0;
+  if (corners && t < 8) {
+    // corner columns (padded 0, 1, nx+2, nx+3) of the halo rows of st, tmp
+    gdouble* buf = t < 4 ? a.st : a.tmp;
+    const int qq = t & 3;
+    const int cc = qq < 2 ? qq : nx + qq;
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) {
+      const double e = buf[g.at(v, plo, cc)];
+      buf[g.at(v, 0, cc)] = wall_halo(v, e, hy[plo], hy[0]);
+      buf[g.at(v, 1, cc)] = wall_halo(v, e, hy[plo], hy[1]);
+      const double f = buf[g.at(v, phi, cc)];
+      buf[g.at(v, nz + 2, cc)] = wall_halo(v, f, hy[phi], hy[nz + 2]);
+      buf[g.at(v, nz + 3, cc)] = wall_halo(v, f, hy[phi], hy[nz + 3]);
+    }
+  }
+  gdouble* const tmp_own = a.tmp_interior ? a.tmp : nullptr;
+  const double id = a.id;
+  __syncthreads();  // also publishes the flags
+#pragma unroll
+  for (int stage = 0; stage < 3; ++stage) {
     const int e = 2 + 2 * stage;
-    // faces: tile rows e .. NR-e (face k between logical rows k-1 and k)
-    bool ok = true;
     if (colok && j >= e && j <= NR - e && k >= 0 && k <= nz) {
       double v4[4], d3[4], G[4];
 #pragma unroll
       for (int v = 0; v < kNv; ++v)
-        recon4(sin[v][t - 2 * CW], sin[v][t - CW], sin[v][t], sin[v][t + CW], v4[v], d3[v]);
-      flux_z_face(v4, d3, hz[0][j], hz[1][j], hz[2][j], a.hv, k == 0 || k == nz, G,
-                  !CONT ? POW_PLAIN : stage == 0 ? POW_FIRST : POW_TRY, &pref, &ok);
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) fl[v][t] = G[v];
-    }
-    if (CONT && !ok) {  // the face again with pow_pos (rare)
-      double v4[4], d3[4], G[4];
-#pragma unroll
-      for (int v = 0; v < kNv; ++v)
-        recon4(sin[v][t - 2 * CW], sin[v][t - CW], sin[v][t], sin[v][t + CW], v4[v], d3[v]);
+        recon4(s[v][u - 2 * CW], s[v][u - CW], s[v][u], s[v][u + CW], v4[v], d3[v]);
       flux_z_face(v4, d3, hz[0][j], hz[1][j], hz[2][j], a.hv, k == 0 || k == nz, G);
 #pragma unroll
-      for (int v = 0; v < kNv; ++v) fl[v][t] = G[v];
+      for (int v = 0; v < kNv; ++v) fl[v][u] = G[v];
     }
-    __syncthreads();
-    // cells: tile rows e .. NR-e-1
+    wave_phase_done(sm.wf, 2 * stage + 1, t);
+    const double dts = stage == 0 ? a.dt1 : stage == 1 ? a.dt2 : a.dt3;
     if (colok && j >= e && j <= NR - e - 1 && k >= 0 && k < nz) {
-      const double dts = stage == 0 ? a.dt1 : stage == 1 ? a.dt2 : a.dt3;
       double td[4];
 #pragma unroll
-      for (int v = 0; v < kNv; ++v) td[v] = tend_of(fl[v][t], fl[v][t + CW], a.d, id);
-      td[2] = td[2] - sin[0][t] * kGrav;
+      for (int v = 0; v < kNv; ++v) td[v] = tend_of(fl[v][u], fl[v][u + CW], a.d, id);
+      td[2] = td[2] - s[0][u] * kGrav;
       if (a.src_w) td[2] = td[2] + src;
       double q[4];
 #pragma unroll
-      for (int v = 0; v < kNv; ++v) q[v] = s0[v][t] + dts * td[v];
+      for (int v = 0; v < kNv; ++v) q[v] = S[v] + dts * td[v];
       if (stage < 2) {
 #pragma unroll
-        for (int v = 0; v < kNv; ++v) s1[v][t] = q[v];
-        // The wall halo rows of the new stage state, written by the edge
-        // row's thread: no thread reads them in this phase (an update reads
-        // its own cell only), and a tile holding a wall has its edge row in
-        // the window, updated at every stage.
+        for (int v = 0; v < kNv; ++v) s[v][u] = q[v];  // in place: faces are done
+        // the wall halo rows of the new stage state (slots u -+ CW, 2 CW of
+        // this column group; no thread reads them in this phase)
 #pragma unroll
         for (int side = 0; side < 2; ++side) {
           if (k == (side == 0 ? 0 : nz - 1)) {
@@ -751,8 +654,8 @@ __device__ __forceinline__ void dir_zt_tile(const DirArgs& a, const Grid& g, int
 #pragma unroll
               for (int v = 0; v < kNv; ++v) w[v] = wall_halo(v, q[v], hy[pe], hy[kh + kHs]);
 #pragma unroll
-              for (int v = 0; v < kNv; ++v) s1[v][t + h * step] = w[v];
-              if (stage == 1 && (side == 0 ? own_lo : own_hi)) {  // set_bc_z of stage 3
+              for (int v = 0; v < kNv; ++v) s[v][u + h * step] = w[v];
+              if (stage == 1 && own) {  // set_bc_z of stage 3
 #pragma unroll
                 for (int v = 0; v < kNv; ++v) a.tmp[g.at(v, kh + kHs, pc)] = w[v];
               }
@@ -769,229 +672,15 @@ __device__ __forceinline__ void dir_zt_tile(const DirArgs& a, const Grid& g, int
       }
     }
     if (stage == 2) break;
-    __syncthreads();
+    wave_phase_done(sm.wf, 2 * stage + 2, t);
   }
 }
 
-// 6 waves per SIMD (the LDS limit of a 512-thread tile): left alone the
-// compiler allocates ~106 VGPRs (4 waves); asked, it fits 72 without spills.
-template <int CW, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_dir_zt(
-    DirArgs a, Grid g, int ncolgrp, int nreal, int per_xcd) {
-  constexpr int C = NT / CW - 12;
-  __shared__ ZTileLds<NT, NT / CW> sm;
-  const int logical = xcd_logical(blockIdx.x, per_xcd);
-  if (logical >= nreal) return;  // whole block, before any barrier
-  member_offset(a);
-  dir_zt_tile<CW, NT>(a, g, (logical % ncolgrp) * CW, (logical / ncolgrp) * C, sm,
-                      logical == 0);
-}
-
-// z tiles of CW columns x NR rows with two cells per thread (tile rows j
-// and j + NR/2 of one column) and the stage state updated in place: LDS holds
-// the running stage state and the face fluxes only (the RK init S of a
-// thread's two cells stays in registers), 64 B per cell, so an 8 x 128 tile
-// fits in 64 KB. Same operations in the same order as dir_zt_tile.
-template <int NC>
-struct ZTile2Lds {
-  double s[kNv][NC];
-  double fl[kNv][NC];
-};
-
-// The same with the tile rows' face hydrostatics (rho, rho*theta, p at the
-// lower face of each tile row), read from HBM once per tile instead of once
-// per stage and cell; all CW columns of a row read one LDS word (broadcast).
-template <int CW, int NR>
-struct ZTile2HLds : ZTile2Lds<CW * NR> {
-  double hz[3][NR];
-  int wf[CW * NR / 64 + 2];  // wave phase flags (one-cell tiles)
-};
-
-// CPT cells per thread: 2 (tile rows j and j + NR/2) or 1. WSYNC (one cell
-// per thread, 8 columns, so that a wave holds 8 whole tile rows): the phases
-// are ordered by wave flags instead of block barriers; every phase touches
-// only the wave's rows and 2 rows on either side.
-template <int CW, int NR, int CPT = 2, bool WSYNC = false>
-__device__ __forceinline__ void dir_zt2_tile(const DirArgs& a, const Grid& g, int c0, int r0,
-                                             ZTile2HLds<CW, NR>& sm, bool corners) {
-  constexpr int NC = CW * NR, NT = NC / CPT, H = 6, C = NR - 2 * H;
-  auto& s = sm.s;
-  auto& fl = sm.fl;
-  auto& hz = sm.hz;
-  const int nx = g.nx, nz = g.nz, t = threadIdx.x;
-  const int col = t % CW;
-  const int i = c0 + col;
-  const bool colok = i < nx;
-  const int pc = i + kHs;
-  const gdouble* hy = a.hy_cell;
-  const int plo = kHs, phi = nz + kHs - 1;
-  const bool own_lo = r0 == 0, own_hi = r0 <= nz - 1 && nz - 1 < r0 + C;
-  gdouble* const tmp_own = a.tmp_interior ? a.tmp : nullptr;
-  static_assert(NT >= NR, "one thread per tile row fills the face hydrostatics");
-  static_assert(!WSYNC || (CPT == 1 && CW == 8 && NT % 64 == 0), "waves of 8 whole rows");
-  if (WSYNC) wave_flags_init(sm.wf, NT / 64, t);
-  // between phases: block barrier, or the neighbouring waves' flags
-  auto phase_done = [&](int P) {
-    if constexpr (WSYNC)
-      wave_phase_done(sm.wf, P, t);
-    else
-      __syncthreads();
-  };
-  if (t < NR) {
-    const int k = r0 - H + t;
-    const bool f = k >= 0 && k <= nz;
-    hz[0][t] = f ? a.hyr_int[k] : 0.0;
-    hz[1][t] = f ? a.hyt_int[k] : 0.0;
-    hz[2][t] = f ? a.hyp_int[k] : 0.0;
-  }
-  int jj[CPT], kk[CPT], sl[CPT];
-  bool wl[CPT], wh[CPT], own[CPT];
-  double S[CPT][4], src[CPT];
-#pragma unroll
-  for (int c = 0; c < CPT; ++c) {
-    sl[c] = t + c * NT;
-    jj[c] = sl[c] / CW;
-    kk[c] = r0 - H + jj[c];
-    wl[c] = kk[c] == -2 || kk[c] == -1;
-    wh[c] = kk[c] == nz || kk[c] == nz + 1;
-    own[c] = colok && kk[c] >= r0 && kk[c] < r0 + C && kk[c] < nz;
-    double q[4] = {0.0, 0.0, 0.0, 0.0};
-    if (colok) {
-      if (kk[c] >= 0 && kk[c] < nz) {
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) q[v] = a.in[g.at(v, kk[c] + kHs, pc)];
-      } else if (wl[c] || wh[c]) {
-        const int pe = wl[c] ? plo : phi;
-#pragma unroll
-        for (int v = 0; v < kNv; ++v)
-          q[v] = wall_halo(v, a.in[g.at(v, pe, pc)], hy[pe], hy[kk[c] + kHs]);
-        if ((wl[c] && own_lo) || (wh[c] && own_hi)) {  // set_bc_z of stage 1 into st
-#pragma unroll
-          for (int v = 0; v < kNv; ++v) a.st[g.at(v, kk[c] + kHs, pc)] = q[v];
-        }
-      }
-    }
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) {
-      s[v][sl[c]] = q[v];
-      S[c][v] = q[v];
-    }
-    src[c] = (a.src_w && colok && kk[c] >= 0 && kk[c] < nz)
-                 ? a.src_w[(long long)kk[c] * nx + i] : 0.0;
-  }
-  if (corners && t < 8) {
-    // corner columns (padded 0, 1, nx+2, nx+3) of the halo rows of st, tmp
-    gdouble* buf = t < 4 ? a.st : a.tmp;
-    const int qq = t & 3;
-    const int cc = qq < 2 ? qq : nx + qq;
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) {
-      const double e = buf[g.at(v, plo, cc)];
-      buf[g.at(v, 0, cc)] = wall_halo(v, e, hy[plo], hy[0]);
-      buf[g.at(v, 1, cc)] = wall_halo(v, e, hy[plo], hy[1]);
-      const double f = buf[g.at(v, phi, cc)];
-      buf[g.at(v, nz + 2, cc)] = wall_halo(v, f, hy[phi], hy[nz + 2]);
-      buf[g.at(v, nz + 3, cc)] = wall_halo(v, f, hy[phi], hy[nz + 3]);
-    }
-  }
-  const double id = a.id;
-  PowRef pref[CPT];  // each thread computes the faces at its slots in every stage
-  __syncthreads();
-#pragma unroll
-  for (int stage = 0; stage < 3; ++stage) {
-    const int e = 2 + 2 * stage;
-    bool ok[CPT];
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) ok[c] = true;
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) {
-      const int j = jj[c], k = kk[c], u = sl[c];
-      if (colok && j >= e && j <= NR - e && k >= 0 && k <= nz) {
-        double v4[4], d3[4], G[4];
-#pragma unroll
-        for (int v = 0; v < kNv; ++v)
-          recon4(s[v][u - 2 * CW], s[v][u - CW], s[v][u], s[v][u + CW], v4[v], d3[v]);
-        flux_z_face(v4, d3, hz[0][j], hz[1][j], hz[2][j], a.hv, k == 0 || k == nz,
-                    G, stage == 0 ? POW_FIRST : POW_TRY, &pref[c], &ok[c]);
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) fl[v][u] = G[v];
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) {
-      if (!ok[c]) {  // the face again with pow_pos (rare)
-        const int j = jj[c], k = kk[c], u = sl[c];
-        double v4[4], d3[4], G[4];
-#pragma unroll
-        for (int v = 0; v < kNv; ++v)
-          recon4(s[v][u - 2 * CW], s[v][u - CW], s[v][u], s[v][u + CW], v4[v], d3[v]);
-        flux_z_face(v4, d3, hz[0][j], hz[1][j], hz[2][j], a.hv, k == 0 || k == nz, G);
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) fl[v][u] = G[v];
-      }
-    }
-    phase_done(2 * stage + 1);
-    const double dts = stage == 0 ? a.dt1 : stage == 1 ? a.dt2 : a.dt3;
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) {
-      const int j = jj[c], k = kk[c], u = sl[c];
-      if (colok && j >= e && j <= NR - e - 1 && k >= 0 && k < nz) {
-        double td[4];
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) td[v] = tend_of(fl[v][u], fl[v][u + CW], a.d, id);
-        td[2] = td[2] - s[0][u] * kGrav;
-        if (a.src_w) td[2] = td[2] + src[c];
-        double q[4];
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) q[v] = S[c][v] + dts * td[v];
-        if (stage < 2) {
-#pragma unroll
-          for (int v = 0; v < kNv; ++v) s[v][u] = q[v];  // in place: faces are done
-          // The wall halo rows of the new stage state, written by the edge
-          // row's thread: no thread reads them in this phase (every update
-          // reads its own cell and faces only), and a tile holding a wall
-          // has its edge row in the window, updated at every stage.
-#pragma unroll
-          for (int side = 0; side < 2; ++side) {
-            if (k == (side == 0 ? 0 : nz - 1)) {
-              const int pe = side == 0 ? plo : phi;
-              const int step = side == 0 ? -CW : CW;
-#pragma unroll
-              for (int h = 1; h <= 2; ++h) {
-                const int kh = side == 0 ? -h : nz - 1 + h;  // the halo row's k
-                double w[4];
-#pragma unroll
-                for (int v = 0; v < kNv; ++v) w[v] = wall_halo(v, q[v], hy[pe], hy[kh + kHs]);
-#pragma unroll
-                for (int v = 0; v < kNv; ++v) s[v][u + h * step] = w[v];
-                if (stage == 1 && (side == 0 ? own_lo : own_hi)) {  // set_bc_z of stage 3
-#pragma unroll
-                  for (int v = 0; v < kNv; ++v) a.tmp[g.at(v, kh + kHs, pc)] = w[v];
-                }
-              }
-            }
-          }
-        }
-        if (own[c]) {
-          gdouble* dst = stage == 0 ? a.s1 : stage == 1 ? tmp_own : a.out;
-          if (dst) {
-#pragma unroll
-            for (int v = 0; v < kNv; ++v) dst[g.at(v, k + kHs, pc)] = q[v];
-          }
-        }
-      }
-    }
-    if (stage == 2) break;
-    phase_done(2 * stage + 2);
-  }
-}
-
-// ---- z, dense tiles: the extended columns of the CW-column groups (rows
+// The same,  dense: the extended columns of the CW-column groups (rows
 // -2 .. nz+1: the wall halo rows are rebuilt from the edge row at every
 // stage, so a column needs no more) laid end to end, slot row g of block b
 // being b*(NR-12) + j - 4, cut into tiles of NR rows; the offset puts row 0
-// of the first group at the first window row. A slot row is (group, row);
-// the two cells of a thread may lie in different groups. Windows [6, NR-6)
+// of the first group at the first window row. Windows [6, NR-6)
 // partition the interior rows; the wall halo rows written to st and tmp
 // belong to the block whose window holds their edge row. A halo row whose
 // edge row lies outside the block is left unrebuilt: no correct cell of the
@@ -1003,169 +692,6 @@ inline int dense_z_blocks(int nx, int nz, int cw, int nr) {
   return (int)((dense_z_rows(nx, nz, cw) - 5) / (nr - 12)) + 1;
 }
 
-template <int CW, int NR>
-__device__ __forceinline__ void dir_zt2d_tile(const DirArgs& a, const Grid& g, int b,
-                                              ZTile2HLds<CW, NR>& sm, bool corners) {
-  constexpr int NC = CW * NR, NT = NC / 2, C = NR - 12;
-  auto& s = sm.s;
-  auto& fl = sm.fl;
-  auto& hz = sm.hz;
-  const int nx = g.nx, nz = g.nz, t = threadIdx.x;
-  const int Ez = nz + 4;
-  static_assert(NT >= NR, "one thread per tile row fills the face hydrostatics");
-  if (t < NR) {  // a tile row is one row k of one column group
-    const int gr = b * C + t - 4;
-    const int k = gr >= 0 ? gr % Ez - 2 : -3;
-    const bool f = k >= 0 && k <= nz;
-    hz[0][t] = f ? a.hyr_int[k] : 0.0;
-    hz[1][t] = f ? a.hyt_int[k] : 0.0;
-    hz[2][t] = f ? a.hyp_int[k] : 0.0;
-  }
-  const int col = t % CW;
-  const gdouble* hy = a.hy_cell;
-  const int plo = kHs, phi = nz + kHs - 1;
-  int jj[2], kk[2], sl[2], es[2], pc[2], ii[2];
-  bool colok[2], wl[2], wh[2], own[2], ownh[2], esok[2];
-  double S[2][4], src[2];
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    sl[c] = t + c * NT;
-    jj[c] = sl[c] / CW;
-    const int gr = b * C + jj[c] - 4;
-    const int grp = gr >= 0 ? gr / Ez : -1;
-    kk[c] = gr >= 0 ? gr - grp * Ez - 2 : -3;  // -3: padding before the first group
-    ii[c] = grp * CW + col;
-    colok[c] = gr >= 0 && ii[c] < nx;
-    pc[c] = (colok[c] ? ii[c] : 0) + kHs;
-    wl[c] = kk[c] == -2 || kk[c] == -1;
-    wh[c] = kk[c] == nz || kk[c] == nz + 1;
-    own[c] = colok[c] && jj[c] >= 6 && jj[c] < NR - 6 && kk[c] >= 0 && kk[c] < nz;
-    const int je = wl[c] ? jj[c] - kk[c] : jj[c] - (kk[c] - (nz - 1));  // edge row's tile row
-    esok[c] = (wl[c] || wh[c]) && je >= 0 && je < NR;
-    es[c] = esok[c] ? je * CW + col : 0;
-    ownh[c] = colok[c] && (wl[c] || wh[c]) && je >= 6 && je < NR - 6;
-    double q[4] = {0.0, 0.0, 0.0, 0.0};
-    if (colok[c]) {
-      if (kk[c] >= 0 && kk[c] < nz) {
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) q[v] = a.in[g.at(v, kk[c] + kHs, pc[c])];
-      } else if (wl[c] || wh[c]) {
-        const int pe = wl[c] ? plo : phi;
-#pragma unroll
-        for (int v = 0; v < kNv; ++v)
-          q[v] = wall_halo(v, a.in[g.at(v, pe, pc[c])], hy[pe], hy[kk[c] + kHs]);
-        if (ownh[c]) {  // set_bc_z of stage 1 into st
-#pragma unroll
-          for (int v = 0; v < kNv; ++v) a.st[g.at(v, kk[c] + kHs, pc[c])] = q[v];
-        }
-      }
-    }
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) {
-      s[v][sl[c]] = q[v];
-      S[c][v] = q[v];
-    }
-    src[c] = (a.src_w && colok[c] && kk[c] >= 0 && kk[c] < nz)
-                 ? a.src_w[(long long)kk[c] * nx + ii[c]] : 0.0;
-  }
-  if (corners && t < 8) {
-    // corner columns (padded 0, 1, nx+2, nx+3) of the halo rows of st, tmp
-    gdouble* buf = t < 4 ? a.st : a.tmp;
-    const int qq = t & 3;
-    const int cc = qq < 2 ? qq : nx + qq;
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) {
-      const double e = buf[g.at(v, plo, cc)];
-      buf[g.at(v, 0, cc)] = wall_halo(v, e, hy[plo], hy[0]);
-      buf[g.at(v, 1, cc)] = wall_halo(v, e, hy[plo], hy[1]);
-      const double f = buf[g.at(v, phi, cc)];
-      buf[g.at(v, nz + 2, cc)] = wall_halo(v, f, hy[phi], hy[nz + 2]);
-      buf[g.at(v, nz + 3, cc)] = wall_halo(v, f, hy[phi], hy[nz + 3]);
-    }
-  }
-  gdouble* const tmp_own = a.tmp_interior ? a.tmp : nullptr;
-  const double id = a.id;
-  PowRef pref[2];  // each thread computes the faces at its two slots in every stage
-  __syncthreads();
-#pragma unroll
-  for (int stage = 0; stage < 3; ++stage) {
-    const int e = 2 + 2 * stage;
-    bool ok[2] = {true, true};
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int j = jj[c], k = kk[c], u = sl[c];
-      if (colok[c] && j >= e && j <= NR - e && k >= 0 && k <= nz) {
-        double v4[4], d3[4], G[4];
-#pragma unroll
-        for (int v = 0; v < kNv; ++v)
-          recon4(s[v][u - 2 * CW], s[v][u - CW], s[v][u], s[v][u + CW], v4[v], d3[v]);
-        flux_z_face(v4, d3, hz[0][j], hz[1][j], hz[2][j], a.hv, k == 0 || k == nz,
-                    G, stage == 0 ? POW_FIRST : POW_TRY, &pref[c], &ok[c]);
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) fl[v][u] = G[v];
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      if (!ok[c]) {  // the face again with pow_pos (rare)
-        const int j = jj[c], k = kk[c], u = sl[c];
-        double v4[4], d3[4], G[4];
-#pragma unroll
-        for (int v = 0; v < kNv; ++v)
-          recon4(s[v][u - 2 * CW], s[v][u - CW], s[v][u], s[v][u + CW], v4[v], d3[v]);
-        flux_z_face(v4, d3, hz[0][j], hz[1][j], hz[2][j], a.hv, k == 0 || k == nz, G);
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) fl[v][u] = G[v];
-      }
-    }
-    __syncthreads();
-    const double dts = stage == 0 ? a.dt1 : stage == 1 ? a.dt2 : a.dt3;
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int j = jj[c], k = kk[c], u = sl[c];
-      if (colok[c] && j >= e && j <= NR - e - 1 && k >= 0 && k < nz) {
-        double td[4];
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) td[v] = tend_of(fl[v][u], fl[v][u + CW], a.d, id);
-        td[2] = td[2] - s[0][u] * kGrav;
-        if (a.src_w) td[2] = td[2] + src[c];
-        double q[4];
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) q[v] = S[c][v] + dts * td[v];
-        if (stage < 2) {
-#pragma unroll
-          for (int v = 0; v < kNv; ++v) s[v][u] = q[v];  // in place: faces are done
-        }
-        if (own[c]) {
-          gdouble* dst = stage == 0 ? a.s1 : stage == 1 ? tmp_own : a.out;
-          if (dst) {
-#pragma unroll
-            for (int v = 0; v < kNv; ++v) dst[g.at(v, k + kHs, pc[c])] = q[v];
-          }
-        }
-      }
-    }
-    if (stage == 2) break;
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      if (colok[c] && esok[c]) {
-        const int pe = wl[c] ? plo : phi;
-        double q[4];
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) q[v] = wall_halo(v, s[v][es[c]], hy[pe], hy[kk[c] + kHs]);
-#pragma unroll
-        for (int v = 0; v < kNv; ++v) s[v][sl[c]] = q[v];
-        if (stage == 1 && ownh[c]) {  // set_bc_z of stage 3
-#pragma unroll
-          for (int v = 0; v < kNv; ++v) a.tmp[g.at(v, kk[c] + kHs, pc[c])] = q[v];
-        }
-      }
-    }
-    __syncthreads();
-  }
-}
-
 // The dense tiles with one cell per thread (CW x NR threads, a wave holding 8
 // whole slot rows): the RK init in registers, the stage state updated in
 // place, the wall halo rows of each stage state written by the edge row's
@@ -1174,11 +700,10 @@ __device__ __forceinline__ void dir_zt2d_tile(const DirArgs& a, const Grid& g, i
 // window, so its edge row was updated, and its halo rows written, in this
 // block at the stage before; halo rows of edge rows outside that window are
 // left unwritten, as no face of the block that is kept reads them.
-template <int CW, int NR>
-__device__ __forceinline__ void dir_zt1d_tile(const DirArgs& a, const Grid& g, int b,
-                                              ZTile2HLds<CW, NR>& sm, bool corners) {
-  constexpr int NT = CW * NR, C = NR - 12;
-  static_assert(CW == 8 && NT % 64 == 0, "waves of 8 whole slot rows");
+template <int NR>
+__device__ __forceinline__ void dir_z1d_tile(const DirArgs& a, const Grid& g, int b,
+                                              Z1Lds<NR>& sm, bool corners) {
+  constexpr int CW = kZ1Cols, NT = CW * NR, C = NR - 12;
   auto& s = sm.s;
   auto& fl = sm.fl;
   auto& hz = sm.hz;
@@ -1246,23 +771,11 @@ __device__ __forceinline__ void dir_zt1d_tile(const DirArgs& a, const Grid& g, i
   }
   gdouble* const tmp_own = a.tmp_interior ? a.tmp : nullptr;
   const double id = a.id;
-  PowRef pref;  // the face at this slot, every stage
   __syncthreads();  // also publishes the flags
 #pragma unroll
   for (int stage = 0; stage < 3; ++stage) {
     const int e = 2 + 2 * stage;
-    bool ok = true;
     if (colok && j >= e && j <= NR - e && k >= 0 && k <= nz) {
-      double v4[4], d3[4], G[4];
-#pragma unroll
-      for (int v = 0; v < kNv; ++v)
-        recon4(s[v][u - 2 * CW], s[v][u - CW], s[v][u], s[v][u + CW], v4[v], d3[v]);
-      flux_z_face(v4, d3, hz[0][j], hz[1][j], hz[2][j], a.hv, k == 0 || k == nz, G,
-                  stage == 0 ? POW_FIRST : POW_TRY, &pref, &ok);
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) fl[v][u] = G[v];
-    }
-    if (!ok) {  // the face again with pow_pos (rare)
       double v4[4], d3[4], G[4];
 #pragma unroll
       for (int v = 0; v < kNv; ++v)
@@ -1321,49 +834,25 @@ __device__ __forceinline__ void dir_zt1d_tile(const DirArgs& a, const Grid& g, i
   }
 }
 
-template <int CW, int NR>
-__global__ __launch_bounds__(CW * NR / 2) __attribute__((amdgpu_waves_per_eu(4))) void k_dir_zt2d(DirArgs a, Grid g, int nreal,
-                                                          int per_xcd) {
-  __shared__ ZTile2HLds<CW, NR> sm;
-  const int logical = xcd_logical(blockIdx.x, per_xcd);
-  if (logical >= nreal) return;  // whole block, before any barrier
-  member_offset(a);
-  dir_zt2d_tile<CW, NR>(a, g, logical, sm, logical == 0);
-}
-
-template <int CW, int NR>
-__global__ __launch_bounds__(CW * NR / 2) __attribute__((amdgpu_waves_per_eu(4))) void k_dir_zt2(
+template <int NR>
+__global__ __launch_bounds__(kZ1Cols * NR) __attribute__((amdgpu_waves_per_eu(6))) void k_dir_z1(
     DirArgs a, Grid g, int ncolgrp, int nreal, int per_xcd) {
-  __shared__ ZTile2HLds<CW, NR> sm;
+  __shared__ Z1Lds<NR> sm;
   const int logical = xcd_logical(blockIdx.x, per_xcd);
   if (logical >= nreal) return;  // whole block, before any barrier
   member_offset(a);
-  dir_zt2_tile<CW, NR>(a, g, (logical % ncolgrp) * CW, (logical / ncolgrp) * (NR - 12), sm,
-                       logical == 0);
+  dir_z1_tile<NR>(a, g, (logical % ncolgrp) * kZ1Cols, (logical / ncolgrp) * (NR - 12), sm,
+                  logical == 0);
 }
 
-template <int CW, int NR>
-__global__ __launch_bounds__(CW * NR) __attribute__((amdgpu_waves_per_eu(6))) void k_dir_zt1d(
+template <int NR>
+__global__ __launch_bounds__(kZ1Cols * NR) __attribute__((amdgpu_waves_per_eu(6))) void k_dir_z1d(
     DirArgs a, Grid g, int nreal, int per_xcd) {
-  __shared__ ZTile2HLds<CW, NR> sm;
+  __shared__ Z1Lds<NR> sm;
   const int logical = xcd_logical(blockIdx.x, per_xcd);
   if (logical >= nreal) return;  // whole block, before any barrier
   member_offset(a);
-  dir_zt1d_tile<CW, NR>(a, g, logical, sm, logical == 0);
-}
-
-// The same tiles with one cell per thread (CW x NR threads): at 8 x 96, two
-// 12-wave blocks per CU (50 KB of LDS each) at 6 waves per SIMD, the waves
-// ordered by neighbour flags.
-template <int CW, int NR>
-__global__ __launch_bounds__(CW * NR) __attribute__((amdgpu_waves_per_eu(6))) void k_dir_zt1(
-    DirArgs a, Grid g, int ncolgrp, int nreal, int per_xcd) {
-  __shared__ ZTile2HLds<CW, NR> sm;
-  const int logical = xcd_logical(blockIdx.x, per_xcd);
-  if (logical >= nreal) return;  // whole block, before any barrier
-  member_offset(a);
-  dir_zt2_tile<CW, NR, 1, true>(a, g, (logical % ncolgrp) * CW,
-                                (logical / ncolgrp) * (NR - 12), sm, logical == 0);
+  dir_z1d_tile<NR>(a, g, logical, sm, logical == 0);
 }
 
 // ------------------------------------------------------------- ensemble --
@@ -1448,126 +937,74 @@ __global__ __launch_bounds__(64 * kXwWaves)
                 sm.s[threadIdx.x >> 6]);
 }
 
-template <int L>
-__global__ __launch_bounds__(192) void k_ens_z(const MemberDev* __restrict__ m, int n, int pass,
-                                               int total, int per_xcd) {
-  __shared__ double ring[2][2][kNv][64];
-  const int item = xcd_logical(blockIdx.x, per_xcd);
-  if (item >= total) return;  // whole block, before any barrier
-  const MemberDev& md = m[member_of<1>(m, n, item)];
-  const DirArgs a = member_args(md, 1, pass & 1, pass >> 1);
-  const int local = item - md.z_start;
-  if ((long long)(local / md.z_ncol) * L >= md.nz) return;  // as in k_ens_x
-  dir_z_block<L>(a, Grid(md.nx, md.nz), local % md.z_ncol, local / md.z_ncol, ring);
-}
-
-template <int CW, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_ens_zt(
+template <int NW, int NR>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void k_ens_zt1(
     const MemberDev* __restrict__ m, int n, int pass, int total, int per_xcd) {
-  constexpr int C = NT / CW - 12;
-  __shared__ ZTileLds<NT, NT / CW> sm;
+  __shared__ ZTileLds<NW, NR> sm;
   const int item = xcd_logical(blockIdx.x, per_xcd);
   if (item >= total) return;  // whole block, before any barrier
   const MemberDev& md = m[member_of<1>(m, n, item)];
   const DirArgs a = member_args(md, 1, pass & 1, pass >> 1);
-  const int local = item - md.z_start;
-  if ((long long)(local / md.z_ncol) * C >= md.nz) return;  // as in k_ens_x
-  dir_zt_tile<CW, NT>(a, Grid(md.nx, md.nz), (local % md.z_ncol) * CW,
-                      (local / md.z_ncol) * C, sm, local == 0);
+  const int local = item - md.z_start, ntile = ZTileRows<NR>::tiles(md.nz);
+  if (local >= md.z_ncol * ntile) return;  // as in k_ens_x
+  dir_zt1_tile<NW, NR>(a, Grid(md.nx, md.nz), local / md.z_ncol, ntile,
+                       (local % md.z_ncol) * kZtCols, sm, local == 0);
 }
 
-template <int CW, int NR>
-__global__ __launch_bounds__(CW * NR / 2) __attribute__((amdgpu_waves_per_eu(4))) void k_ens_zt2d(const MemberDev* __restrict__ m, int n,
-                                                          int pass, int total, int per_xcd) {
-  __shared__ ZTile2HLds<CW, NR> sm;
-  const int item = xcd_logical(blockIdx.x, per_xcd);
-  if (item >= total) return;  // whole block, before any barrier
-  const MemberDev& md = m[member_of<1>(m, n, item)];
-  const DirArgs a = member_args(md, 1, pass & 1, pass >> 1);
-  const int local = item - md.z_start;
-  if (local >= md.z_ncol) return;  // dense z: z_ncol holds the member's blocks
-  dir_zt2d_tile<CW, NR>(a, Grid(md.nx, md.nz), local, sm, local == 0);
-}
-
-template <int CW, int NR>
-__global__ __launch_bounds__(CW * NR) __attribute__((amdgpu_waves_per_eu(6))) void k_ens_zt1d(
+template <int NR>
+__global__ __launch_bounds__(kZ1Cols * NR) __attribute__((amdgpu_waves_per_eu(6))) void k_ens_z1(
     const MemberDev* __restrict__ m, int n, int pass, int total, int per_xcd) {
-  __shared__ ZTile2HLds<CW, NR> sm;
-  const int item = xcd_logical(blockIdx.x, per_xcd);
-  if (item >= total) return;  // whole block, before any barrier
-  const MemberDev& md = m[member_of<1>(m, n, item)];
-  const DirArgs a = member_args(md, 1, pass & 1, pass >> 1);
-  const int local = item - md.z_start;
-  if (local >= md.z_ncol) return;  // dense z: z_ncol holds the member's blocks
-  dir_zt1d_tile<CW, NR>(a, Grid(md.nx, md.nz), local, sm, local == 0);
-}
-
-template <int CW, int NR>
-__global__ __launch_bounds__(CW * NR) __attribute__((amdgpu_waves_per_eu(6))) void k_ens_zt1(
-    const MemberDev* __restrict__ m, int n, int pass, int total, int per_xcd) {
-  __shared__ ZTile2HLds<CW, NR> sm;
+  __shared__ Z1Lds<NR> sm;
   const int item = xcd_logical(blockIdx.x, per_xcd);
   if (item >= total) return;  // whole block, before any barrier
   const MemberDev& md = m[member_of<1>(m, n, item)];
   const DirArgs a = member_args(md, 1, pass & 1, pass >> 1);
   const int local = item - md.z_start;
   if ((long long)(local / md.z_ncol) * (NR - 12) >= md.nz) return;  // as in k_ens_x
-  dir_zt2_tile<CW, NR, 1, true>(a, Grid(md.nx, md.nz), (local % md.z_ncol) * CW,
-                                (local / md.z_ncol) * (NR - 12), sm, local == 0);
+  dir_z1_tile<NR>(a, Grid(md.nx, md.nz), (local % md.z_ncol) * kZ1Cols,
+                  (local / md.z_ncol) * (NR - 12), sm, local == 0);
 }
 
-template <int CW, int NR>
-__global__ __launch_bounds__(CW * NR / 2) __attribute__((amdgpu_waves_per_eu(4))) void k_ens_zt2(const MemberDev* __restrict__ m, int n,
-                                                         int pass, int total, int per_xcd) {
-  __shared__ ZTile2HLds<CW, NR> sm;
+template <int NR>
+__global__ __launch_bounds__(kZ1Cols * NR) __attribute__((amdgpu_waves_per_eu(6))) void k_ens_z1d(
+    const MemberDev* __restrict__ m, int n, int pass, int total, int per_xcd) {
+  __shared__ Z1Lds<NR> sm;
   const int item = xcd_logical(blockIdx.x, per_xcd);
   if (item >= total) return;  // whole block, before any barrier
   const MemberDev& md = m[member_of<1>(m, n, item)];
   const DirArgs a = member_args(md, 1, pass & 1, pass >> 1);
   const int local = item - md.z_start;
-  if ((long long)(local / md.z_ncol) * (NR - 12) >= md.nz) return;  // as in k_ens_x
-  dir_zt2_tile<CW, NR>(a, Grid(md.nx, md.nz), (local % md.z_ncol) * CW,
-                       (local / md.z_ncol) * (NR - 12), sm, local == 0);
+  if (local >= md.z_ncol) return;  // dense z: z_ncol holds the member's blocks
+  dir_z1d_tile<NR>(a, Grid(md.nx, md.nz), local, sm, local == 0);
 }
 
-template <int CW, int NR>
-int launch_zt2(const DirArgs& a, Grid g, hipStream_t st, int members) {
-  constexpr int C = NR - 12;
-  const int ncolgrp = (g.nx + CW - 1) / CW;
-  const long long nreal = (long long)ncolgrp * ((g.nz + C - 1) / C);
-  const int per = (int)((nreal + kNumXcd - 1) / kNumXcd);
-  k_dir_zt2<CW, NR><<<dim3(per * kNumXcd, members), CW * NR / 2, 0, st>>>(a, g, ncolgrp,
-                                                                          (int)nreal, per);
-  PMW_CHECK_LAUNCH();
-  return PMW_OK;
-}
-
-template <int CW, int NR>
 int launch_zt1(const DirArgs& a, Grid g, hipStream_t st, int members) {
+  constexpr int NW = kZtWaves, NR = kZtRows;
+  const int ncol = (g.nx + kZtCols - 1) / kZtCols, ntile = ZTileRows<NR>::tiles(g.nz);
+  const int per = (ncol * ntile + kNumXcd - 1) / kNumXcd;
+  k_dir_zt1<NW, NR><<<dim3(per * kNumXcd, members), 64 * NW, 0, st>>>(a, g, ncol, ntile, per);
+  PMW_CHECK_LAUNCH();
+  return PMW_OK;
+}
+
+template <int NR>
+int launch_z1(const DirArgs& a, Grid g, hipStream_t st, int members) {
   constexpr int C = NR - 12;
-  const int ncolgrp = (g.nx + CW - 1) / CW;
+  const int ncolgrp = (g.nx + kZ1Cols - 1) / kZ1Cols;
   const long long nreal = (long long)ncolgrp * ((g.nz + C - 1) / C);
+  if (nreal > (1LL << 31) - 64) return PMW_EINVAL;
   const int per = (int)((nreal + kNumXcd - 1) / kNumXcd);
-  k_dir_zt1<CW, NR><<<dim3(per * kNumXcd, members), CW * NR, 0, st>>>(a, g, ncolgrp,
-                                                                      (int)nreal, per);
+  k_dir_z1<NR><<<dim3(per * kNumXcd, members), kZ1Cols * NR, 0, st>>>(a, g, ncolgrp, (int)nreal,
+                                                                      per);
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
 
-template <int CW, int NR>
-int launch_zt1d(const DirArgs& a, Grid g, hipStream_t st, int members) {
-  const int nreal = dense_z_blocks(g.nx, g.nz, CW, NR);
+template <int NR>
+int launch_z1d(const DirArgs& a, Grid g, hipStream_t st, int members) {
+  const int nreal = dense_z_blocks(g.nx, g.nz, kZ1Cols, NR);
   const int per = (nreal + kNumXcd - 1) / kNumXcd;
-  k_dir_zt1d<CW, NR><<<dim3(per * kNumXcd, members), CW * NR, 0, st>>>(a, g, nreal, per);
-  PMW_CHECK_LAUNCH();
-  return PMW_OK;
-}
-
-template <int CW, int NR>
-int launch_zt2d(const DirArgs& a, Grid g, hipStream_t st, int members) {
-  const int nreal = dense_z_blocks(g.nx, g.nz, CW, NR);
-  const int per = (nreal + kNumXcd - 1) / kNumXcd;
-  k_dir_zt2d<CW, NR><<<dim3(per * kNumXcd, members), CW * NR / 2, 0, st>>>(a, g, nreal, per);
+  k_dir_z1d<NR><<<dim3(per * kNumXcd, members), kZ1Cols * NR, 0, st>>>(a, g, nreal, per);
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
@@ -1583,29 +1020,6 @@ int launch_x(const DirArgs& a, Grid g, hipStream_t st, int members) {
   const int per = (nreal + kNumXcd - 1) / kNumXcd;
   k_dir_x<256 * K><<<dim3(per * kNumXcd, members, chunks), 64 * kXwWaves, 0, st>>>(
       a, g, E, rows, nreal, per);
-  PMW_CHECK_LAUNCH();
-  return PMW_OK;
-}
-
-template <int CW, int NT>
-int launch_zt(const DirArgs& a, Grid g, hipStream_t st, int members) {
-  constexpr int C = NT / CW - 12;
-  const int ncolgrp = (g.nx + CW - 1) / CW;
-  const long long nreal = (long long)ncolgrp * ((g.nz + C - 1) / C);
-  const int per = (int)((nreal + kNumXcd - 1) / kNumXcd);
-  k_dir_zt<CW, NT><<<dim3(per * kNumXcd, members), NT, 0, st>>>(a, g, ncolgrp, (int)nreal,
-                                                                 per);
-  PMW_CHECK_LAUNCH();
-  return PMW_OK;
-}
-
-template <int L>
-int launch_z(const DirArgs& a, Grid g, hipStream_t st, int members) {
-  const int ncolblk = (g.nx + 4 + 63) / 64;
-  const int nseg = (g.nz + L - 1) / L;
-  const long long nreal = (long long)ncolblk * nseg;
-  const int per = (int)((nreal + kNumXcd - 1) / kNumXcd);
-  k_dir_z<L><<<dim3(per * kNumXcd, members), 192, 0, st>>>(a, g, ncolblk, (int)nreal, per);
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
@@ -1632,13 +1046,28 @@ int fused_x_cells(int nt, long long cells) {
   return cells <= 300000 ? 1 : 2;
 }
 
-// z: 8..64 = rows per marching segment; columns*1000 + rows = LDS tiles:
-// 8064, 4128 (one cell per thread, RK init in LDS), 8096 (one cell per
-// thread, RK init in registers, stage state updated in place), 8128 (two
-// cells per thread); 18128 = 8128 as dense tiles (column groups end to end)
 bool fused_z_seg_ok(int seg) {
   return seg == 8 || seg == 16 || seg == 24 || seg == 32 || seg == 48 || seg == 64 ||
          seg == 8064 || seg == 4128 || seg == 8128 || seg == 18128 || seg == 8096 || seg == 18096;
+}
+
+// The z kernel of a launch over `cells` cells of grids whose smallest nz and
+// largest nx are given. Codes 18096 and 18128 force the dense one-cell tiles,
+// 8 to 64 the small ones; the others go by size. The three-row tiles need
+// edge tiles that reach past their own rows into the grid only (nz >= NR - 2)
+// and 32-bit offsets inside a tile; they win once their blocks fill the GPU.
+// Step time in us with one-cell tiles of 32 rows / of 96 rows / three-row
+// tiles: 100x50 12.7 / 13.9 / -, 200x100 13.4 / 15.1 / 18.1, 400x200 14.5 /
+// 17.5 / 21.0, 600x300 19.8 / 22.6 / 23.9, 800x400 26.4 / 26.6 / 28.0,
+// 1003x517 37.7 / 39.1 / 37.6, 2000x1000 108 / 99 / 92, 8192x4096 1800 / 1668
+// / 1452. Low columns (nz < 94) of large grids take the one-cell tile whose
+// rows fit them better.
+enum ZKernel { Z_ROWS3, Z_ONE96, Z_ONE32, Z_DENSE };
+ZKernel fused_z_kernel(int seg, long long cells, int min_nz, int max_nx) {
+  if (seg == 18096 || seg == 18128) return Z_DENSE;
+  if (seg <= 64 || cells < 500000) return Z_ONE32;
+  if (min_nz >= kZtRows - 2 && max_nx < (1 << 22)) return Z_ROWS3;
+  return min_nz > 40 ? Z_ONE96 : Z_ONE32;
 }
 
 int launch_dir_x(const DirArgs& a, Grid g, int nt, hipStream_t st, int members) {
@@ -1652,24 +1081,14 @@ int launch_dir_x(const DirArgs& a, Grid g, int nt, hipStream_t st, int members) 
 
 int launch_dir_z(const DirArgs& a, Grid g, int seg, hipStream_t st, int members) {
   if (members < 1 || members > 65535 || (members > 1 && a.mstride <= 0)) return PMW_EINVAL;
-  switch (seg) {
-    case 8: return launch_z<8>(a, g, st, members);
-    case 16: return launch_z<16>(a, g, st, members);
-    case 24: return launch_z<24>(a, g, st, members);
-    case 32: return launch_z<32>(a, g, st, members);
-    case 48: return launch_z<48>(a, g, st, members);
-    case 64: return launch_z<64>(a, g, st, members);
-    case 8064: return launch_zt<8, 512>(a, g, st, members);
-    case 4128: return launch_zt<4, 512>(a, g, st, members);
-    case 8128: return launch_zt2<8, 128>(a, g, st, members);
-    case 8096: return launch_zt1<8, 96>(a, g, st, members);
-    case 18128:
-      if (dense_z_rows(g.nx, g.nz, 8) > (1LL << 30)) return PMW_EINVAL;
-      return launch_zt2d<8, 128>(a, g, st, members);
-    case 18096:
-      if (dense_z_rows(g.nx, g.nz, 8) > (1LL << 30)) return PMW_EINVAL;
-      return launch_zt1d<8, 96>(a, g, st, members);
-    default: return PMW_EINVAL;
+  if (!fused_z_seg_ok(seg)) return PMW_EINVAL;
+  switch (fused_z_kernel(seg, (long long)g.nx * g.nz * members, g.nz, g.nx)) {
+    case Z_ROWS3: return launch_zt1(a, g, st, members);
+    case Z_ONE96: return launch_z1<96>(a, g, st, members);
+    case Z_ONE32: return launch_z1<32>(a, g, st, members);
+    default:
+      if (dense_z_rows(g.nx, g.nz, kZ1Cols) > (1LL << 30)) return PMW_EINVAL;
+      return launch_z1d<96>(a, g, st, members);
   }
 }
 
@@ -1680,14 +1099,21 @@ namespace {
 
 struct EnsPlan {
   int x_total, z_total;
-  int x_k;  // cells per lane of the x waves
+  int x_k;       // cells per lane of the x waves
+  int z_kernel;  // a pmw::ZKernel
 };
 
 int plan_members(const pmw_member* mem, int n, int x_nt, int z_seg, MemberDev* dev,
                  EnsPlan& plan) {
   long long xs = 0, zs = 0, cells = 0;
-  for (int q = 0; q < n; ++q) cells += (long long)mem[q].nx * mem[q].nz;
+  int min_nz = 1 << 30, max_nx = 0;
+  for (int q = 0; q < n; ++q) {
+    cells += (long long)mem[q].nx * mem[q].nz;
+    min_nz = std::min(min_nz, mem[q].nz);
+    max_nx = std::max(max_nx, mem[q].nx);
+  }
   plan.x_k = pmw::fused_x_cells(x_nt, cells);
+  plan.z_kernel = pmw::fused_z_kernel(z_seg, cells, min_nz, max_nx);
   for (int q = 0; q < n; ++q) {
     const pmw_member& m = mem[q];
     if (m.nx < 2 || m.nz < 2 || !m.state || !m.state_tmp || !m.state_work ||
@@ -1701,17 +1127,17 @@ int plan_members(const pmw_member* mem, int n, int x_nt, int z_seg, MemberDev* d
       return PMW_EINVAL;
     const int xt = xw_blocks(m.nx, m.nz, plan.x_k);
     int zc, zsg;
-    if (z_seg == 18128 || z_seg == 18096) {  // dense tiles: zc = the member's blocks, one "segment"
-      if (dense_z_rows(m.nx, m.nz, 8) > (1LL << 30)) return PMW_EINVAL;
-      zc = dense_z_blocks(m.nx, m.nz, 8, z_seg % 1000);
+    if (plan.z_kernel == pmw::Z_DENSE) {  // zc = the member's blocks, one row of tiles
+      if (dense_z_rows(m.nx, m.nz, kZ1Cols) > (1LL << 30)) return PMW_EINVAL;
+      zc = dense_z_blocks(m.nx, m.nz, kZ1Cols, 96);
       zsg = 1;
-    } else if (z_seg >= 1000) {  // LDS tiles: columns*1000 + rows (12 of them halo)
-      const int cw = z_seg / 1000, rows = z_seg % 1000 - 12;
-      zc = (m.nx + cw - 1) / cw;
-      zsg = (m.nz + rows - 1) / rows;
+    } else if (plan.z_kernel == pmw::Z_ROWS3) {
+      zc = (m.nx + kZtCols - 1) / kZtCols;
+      zsg = ZTileRows<kZtRows>::tiles(m.nz);
     } else {
-      zc = (m.nx + 4 + 63) / 64;
-      zsg = (m.nz + z_seg - 1) / z_seg;
+      const int rows = plan.z_kernel == pmw::Z_ONE96 ? 96 - 12 : 32 - 12;
+      zc = (m.nx + kZ1Cols - 1) / kZ1Cols;
+      zsg = (m.nz + rows - 1) / rows;
     }
     if (dev) {
       MemberDev& d = dev[q];
@@ -1803,74 +1229,30 @@ int launch_ens_x(const MemberDev* d, int n, int pass, int total, hipStream_t st)
   return PMW_OK;
 }
 
-template <int L>
-int launch_ens_z(const MemberDev* d, int n, int pass, int total, hipStream_t st) {
-  const int per = ens_per_xcd(total);
-  k_ens_z<L><<<per * kNumXcd, 192, 0, st>>>(d, n, pass, total, per);
-  PMW_CHECK_LAUNCH();
-  return PMW_OK;
-}
-
-template <int CW, int NR>
-int launch_ens_zt2d(const MemberDev* d, int n, int pass, int total, hipStream_t st) {
-  const int per = ens_per_xcd(total);
-  k_ens_zt2d<CW, NR><<<per * kNumXcd, CW * NR / 2, 0, st>>>(d, n, pass, total, per);
-  PMW_CHECK_LAUNCH();
-  return PMW_OK;
-}
-
-template <int CW, int NR>
-int launch_ens_zt1d(const MemberDev* d, int n, int pass, int total, hipStream_t st) {
-  const int per = ens_per_xcd(total);
-  k_ens_zt1d<CW, NR><<<per * kNumXcd, CW * NR, 0, st>>>(d, n, pass, total, per);
-  PMW_CHECK_LAUNCH();
-  return PMW_OK;
-}
-
-template <int CW, int NR>
-int launch_ens_zt1(const MemberDev* d, int n, int pass, int total, hipStream_t st) {
-  const int per = ens_per_xcd(total);
-  k_ens_zt1<CW, NR><<<per * kNumXcd, CW * NR, 0, st>>>(d, n, pass, total, per);
-  PMW_CHECK_LAUNCH();
-  return PMW_OK;
-}
-
-template <int CW, int NR>
-int launch_ens_zt2(const MemberDev* d, int n, int pass, int total, hipStream_t st) {
-  const int per = ens_per_xcd(total);
-  k_ens_zt2<CW, NR><<<per * kNumXcd, CW * NR / 2, 0, st>>>(d, n, pass, total, per);
-  PMW_CHECK_LAUNCH();
-  return PMW_OK;
-}
-
-template <int CW, int NT>
-int launch_ens_zt(const MemberDev* d, int n, int pass, int total, hipStream_t st) {
-  const int per = ens_per_xcd(total);
-  k_ens_zt<CW, NT><<<per * kNumXcd, NT, 0, st>>>(d, n, pass, total, per);
-  PMW_CHECK_LAUNCH();
-  return PMW_OK;
-}
-
-int launch_ens(int dir, int z_seg, const MemberDev* d, int n, int pass,
-               const EnsPlan& plan, hipStream_t st) {
-  if (dir == 0) {
-    return plan.x_k == 1 ? launch_ens_x<1>(d, n, pass, plan.x_total, st)
-                         : launch_ens_x<2>(d, n, pass, plan.x_total, st);
+int launch_ens_z(const MemberDev* d, int n, int pass, const EnsPlan& plan, hipStream_t st) {
+  const int total = plan.z_total, per = ens_per_xcd(total), nb = per * kNumXcd;
+  switch (plan.z_kernel) {
+    case pmw::Z_ROWS3:
+      k_ens_zt1<kZtWaves, kZtRows><<<nb, 64 * kZtWaves, 0, st>>>(d, n, pass, total, per);
+      break;
+    case pmw::Z_ONE96:
+      k_ens_z1<96><<<nb, kZ1Cols * 96, 0, st>>>(d, n, pass, total, per);
+      break;
+    case pmw::Z_ONE32:
+      k_ens_z1<32><<<nb, kZ1Cols * 32, 0, st>>>(d, n, pass, total, per);
+      break;
+    default:
+      k_ens_z1d<96><<<nb, kZ1Cols * 96, 0, st>>>(d, n, pass, total, per);
   }
-  switch (z_seg) {
-    case 8: return launch_ens_z<8>(d, n, pass, plan.z_total, st);
-    case 16: return launch_ens_z<16>(d, n, pass, plan.z_total, st);
-    case 24: return launch_ens_z<24>(d, n, pass, plan.z_total, st);
-    case 32: return launch_ens_z<32>(d, n, pass, plan.z_total, st);
-    case 48: return launch_ens_z<48>(d, n, pass, plan.z_total, st);
-    case 8064: return launch_ens_zt<8, 512>(d, n, pass, plan.z_total, st);
-    case 4128: return launch_ens_zt<4, 512>(d, n, pass, plan.z_total, st);
-    case 8128: return launch_ens_zt2<8, 128>(d, n, pass, plan.z_total, st);
-    case 8096: return launch_ens_zt1<8, 96>(d, n, pass, plan.z_total, st);
-    case 18128: return launch_ens_zt2d<8, 128>(d, n, pass, plan.z_total, st);
-    case 18096: return launch_ens_zt1d<8, 96>(d, n, pass, plan.z_total, st);
-    default: return launch_ens_z<64>(d, n, pass, plan.z_total, st);
-  }
+  PMW_CHECK_LAUNCH();
+  return PMW_OK;
+}
+
+int launch_ens(int dir, const MemberDev* d, int n, int pass, const EnsPlan& plan,
+               hipStream_t st) {
+  if (dir == 1) return launch_ens_z(d, n, pass, plan, st);
+  return plan.x_k == 1 ? launch_ens_x<1>(d, n, pass, plan.x_total, st)
+                       : launch_ens_x<2>(d, n, pass, plan.x_total, st);
 }
 
 }  // namespace
@@ -1959,7 +1341,7 @@ int pmw_ensemble_evolve(const pmw_member* members, int nmembers, const int* tuni
       }
       // state_tmp's interior: only the call's last direction keeps its stores
       const int keep_tmp = pass == 1 && step == nsteps - 1;
-      rc = launch_ens(dir, z_seg, d, nmembers, pass | keep_tmp << 1, plan, st);
+      rc = launch_ens(dir, d, nmembers, pass | keep_tmp << 1, plan, st);
       if (kernel_ms && rc == PMW_OK) {
         hipError_t e = hipEventRecord(ev[1], st);
         float ms = 0.f;

@@ -631,7 +631,7 @@ namespace {
 struct Tuning {
   int mode;   // 0: one fused launch per direction; 1: one launch per RK stage
   int x_nt;   // fused x: 256, 1512 force one or two cells per lane; 448, 512, 1256 by size
-  int z_seg;  // fused z: rows per marching segment (8..64) or LDS tile code (8064, 4128, 8096, 8128)
+  int z_seg;  // fused z: tile code (fused_z_kernel)
 };
 constexpr Tuning kDefaultTuning = {0, 512, 8096};
 
