@@ -752,8 +752,7 @@ int pmw_tape_forward(double* tape, long long tape_len, int members,
         a.out = gptr(tape + (q == 2LL * nsteps - 1 ? 6LL * nsteps : (q + 1) % 2) * slot);
         a.tmp_interior = false;
       }
-      a.d = dir == 0 ? dx : dz;
-      a.id = 1.0 / a.d;
+      set_spacing(a, dir == 0 ? dx : dz);
       a.hv = dir == 0 ? hv_coeff_x : hv_coeff_z;
       const int rc = dir == 0 ? launch_dir_x(a, g, x_nt, st, members)
                               : launch_dir_z(a, g, z_seg, st, members);

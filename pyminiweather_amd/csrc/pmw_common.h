@@ -1,10 +1,11 @@
 // pmw_common.h -- constants and pointwise device arithmetic shared by the
 // PyMiniWeather HIP kernels (gfx950).
 //
-// Every expression keeps the reference's floating-point operation order, and
-// the library is compiled with -ffp-contract=off, so that a face flux or a
-// cell update rounds exactly like the NumPy code it replaces. The only
-// expected differences from NumPy are last-bit differences of the powers
+// Reconstruction, pressure, tendency and update keep the reference's
+// floating-point operation order, and the library is compiled with
+// -ffp-contract=off, so that they round like the NumPy code they replace. The
+// expected differences from NumPy are fewer roundings in the fluxes' advective
+// and viscous terms (flux_x_face), last-bit differences of the powers
 // (pow_gamma of pmw_pow.h is correctly rounded in all but ~1e-7 of cases,
 // glibc's pow, which NumPy calls, in all but 8e-4) and of exp/cos in the
 // initial conditions.
@@ -12,6 +13,8 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <cmath>
 
 #include "pmw.h"
 #include "pmw_pow.h"
@@ -88,16 +91,24 @@ struct Grid {
   }
 };
 
-// a / b from y = RN(1/b): q = RN(a*y) is within an ulp of a/b and the
-// residual a - q*b is exact under fma, so q + r*y rounds to the IEEE
-// quotient (Markstein's correction; valid while a/b, a*y and the residual
-// neither overflow nor underflow, as for the fluxes and densities here).
-// Three instructions instead of a full division.
-__device__ __forceinline__ double div_rn(double a, double b, double y) {
-  const double q = a * y;
-  const double r = fma(-q, b, a);
-  return fma(r, y, q);
+// 1/b as y + yl, for quotients by b: y from v_rcp_f64 and one Newton step
+// (relative error e below 2^-46), yl = e y the remainder, so that y + yl is
+// 1/b to 2^-92, and a/b = RN(a y + RN(a yl)) is the correctly rounded
+// quotient except with probability ~2^-38: 5 instructions, and 2 per
+// quotient, instead of 10 for an IEEE reciprocal and 3. As with the division
+// by b, 0, infinite and NaN b give NaN quotients here.
+struct Recip {
+  double y, yl;
+};
+__device__ __forceinline__ Recip recip(double b) {
+  double y = __builtin_amdgcn_rcp(b);
+  y = fma(fma(-b, y, 1.0), y, y);
+  return {y, fma(-b, y, 1.0) * y};
 }
+__device__ __forceinline__ double quot(double a, Recip r) { return fma(a, r.y, a * r.yl); }
+
+// The remainder 1/d - id of a host reciprocal id = RN(1/d).
+inline double recip_lo(double d, double id) { return std::fma(-d, id, 1.0) * id; }
 
 // 4-tap reconstruction at one face: value and 3rd difference, accumulated
 // left to right like scipy.signal.convolve's direct method.
@@ -108,21 +119,25 @@ __device__ __forceinline__ void recon4(double s0, double s1, double s2,
 }
 
 // x-direction Euler flux with hyperviscosity (solve/interpolate.py:105-129).
+// The pressure's argument rho * t, t = (rho*theta) / rho, keeps the
+// reference's roundings (a last bit there is a last bit of a 1e5 Pa pressure).
+// The advective terms take the reconstructed momentum m = rho u itself instead
+// of rho * (m / rho), one product per term, and the products that are only
+// added into a flux are not rounded before: fewer roundings than the
+// reference's, which sit far below the pressure's last bit.
 __device__ __forceinline__ void flux_x_face(const double val[4],
                                             const double d3[4], double hyr,
                                             double hyt, double hv,
                                             double F[4]) {
   const double rho = val[0] + hyr;
-  const double ir = 1.0 / rho;
-  const double u = div_rn(val[1], rho, ir);
-  const double w = div_rn(val[2], rho, ir);
-  const double t = div_rn(val[3] + hyt, rho, ir);
+  const Recip r = recip(rho);
+  const double u = quot(val[1], r);
+  const double t = quot(val[3] + hyt, r);
   const double p = kC0 * pow_gamma(rho * t);
-  const double ru = rho * u;
-  F[0] = ru - hv * d3[0];
-  F[1] = (rho * (u * u) + p) - hv * d3[1];
-  F[2] = ru * w - hv * d3[2];
-  F[3] = ru * t - hv * d3[3];
+  F[0] = fma(-hv, d3[0], val[1]);
+  F[1] = fma(-hv, d3[1], fma(val[1], u, p));
+  F[2] = fma(-hv, d3[2], u * val[2]);
+  F[3] = fma(-hv, d3[3], val[1] * t);
 }
 
 // z-direction flux (solve/interpolate.py:153-186); `wall` marks faces k = 0
@@ -132,26 +147,23 @@ __device__ __forceinline__ void flux_z_face(const double val[4], double d3[4],
                                             double hyp, double hv, bool wall,
                                             double G[4]) {
   const double rho = val[0] + hyr;
-  const double ir = 1.0 / rho;
-  const double u = div_rn(val[1], rho, ir);
-  double w = div_rn(val[2], rho, ir);
-  const double t = div_rn(val[3] + hyt, rho, ir);
+  const Recip r = recip(rho);
+  const double m = wall ? 0.0 : val[2];  // rho w
+  const double w = quot(m, r);
+  const double t = quot(val[3] + hyt, r);
   const double p = kC0 * pow_gamma(rho * t) - hyp;
-  if (wall) {
-    w = 0.0;
-    d3[0] = 0.0;
-  }
-  const double rw = rho * w;
-  G[0] = rw - hv * d3[0];
-  G[1] = rw * u - hv * d3[1];
-  G[2] = (rho * (w * w) + p) - hv * d3[2];
-  G[3] = rw * t - hv * d3[3];
+  const double d0 = wall ? 0.0 : d3[0];
+  G[0] = fma(-hv, d0, m);
+  G[1] = fma(-hv, d3[1], w * val[1]);
+  G[2] = fma(-hv, d3[2], fma(m, w, p));
+  G[3] = fma(-hv, d3[3], m * t);
 }
 
-// Tendency from two face fluxes (solve/interpolate.py:209-215, 239-245).
-// id = RN(1/d).
-__device__ __forceinline__ double tend_of(double f_lo, double f_hi, double d, double id) {
-  return div_rn(-(f_hi - f_lo), d, id);
+// Tendency from two face fluxes (solve/interpolate.py:209-215, 239-245), with
+// id + idl = 1/d to 2^-106 (recip_lo): the correctly rounded quotient.
+__device__ __forceinline__ double tend_of(double f_lo, double f_hi, double id, double idl) {
+  const double x = f_lo - f_hi;
+  return fma(x, id, x * idl);
 }
 
 // Value the reference's set_bc_z leaves in z-halo row `prow` (0, 1, nz+2 or
@@ -160,7 +172,7 @@ __device__ __forceinline__ double tend_of(double f_lo, double f_hi, double d, do
 __device__ __forceinline__ double wall_halo(int v, double edge_val,
                                             double hy_edge, double hy_halo) {
   if (v == 2) return 0.0;
-  if (v == 1) return edge_val / hy_edge * hy_halo;
+  if (v == 1) return quot(edge_val, recip(hy_edge)) * hy_halo;
   return edge_val;
 }
 

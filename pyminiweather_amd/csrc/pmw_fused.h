@@ -17,9 +17,7 @@ struct DirArgs {
   const gdouble* hyt_int;   // hy_dens_theta_int (z faces)
   const gdouble* hyp_int;   // hy_pressure_int (z faces)
   const gdouble* src_w;     // (nz, nx) w source or nullptr
-  double d;                // dx or dz
-  double id;               // RN(1/d), set with d (a host division, so no
-                           // kernel spends an IEEE division on it)
+  double id, idl;          // 1/dx or 1/dz as a sum (set_spacing)
   double dt1, dt2, dt3;    // dt/3, dt/2, dt
   double hv;               // -hv_beta * d / (16 * dt_full)
   gdouble* s1 = nullptr;   // optional: receives the stage-1 interior
@@ -29,6 +27,11 @@ struct DirArgs {
   long long mstride = 0;   // batched launches: elements between members of
                            // in / st / out / tmp / s1 (member = blockIdx.y)
 };
+
+inline void set_spacing(DirArgs& a, double d) {
+  a.id = 1.0 / d;
+  a.idl = recip_lo(d, a.id);
+}
 
 bool fused_x_tile_ok(int nt);
 bool fused_z_seg_ok(int seg);

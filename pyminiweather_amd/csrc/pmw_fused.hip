@@ -108,9 +108,9 @@ __device__ __forceinline__ void wave_phase_done(int* wf, int P, int t) {
 // cells; 108 doubles of LDS traffic per cell and direction, here 12) the waves
 // are bound by FP64 issue in the steady state, with the start and the tail of
 // the launch on top (2.5 of 5 waves per SIMD on average). Per launch between
-// events, 512-thread LDS tiles / these waves: 2000 x 1000 52.3 / 42.5 us,
-// 8192 x 4096 740 / 599 us (3.6 TB/s of reads and writes; a 4 GB copy reaches
-// 4.6). The cheaper power alone took the tiles from 51 to 47 us, and they
+// events, 512-thread LDS tiles / these waves / with the reciprocal pairs of
+// recip() and tend_of(): 2000 x 1000 52.3 / 42.5 / 38.7 us, 8192 x 4096 740 /
+// 599 / 551 us (3.9 TB/s of reads and writes; a 4 GB copy reaches 4.6). The cheaper power alone took the tiles from 51 to 47 us, and they
 // stayed at 42 with the power left out of a timing copy altogether.
 template <int CTRL>
 __device__ __forceinline__ double dpp_f64(double x) {
@@ -196,7 +196,6 @@ __device__ __forceinline__ void dir_x_wave(const DirArgs& a, const Grid& g, unsi
     for (int v = 0; v < kNv; ++v) init[i * kNv + v][lane] = s[i][v];
   asm volatile("" ::: "memory");  // read back from LDS, not kept in registers
   const double hyr = a.hy_cell[prow], hyt = a.hyt_cell[prow];
-  const double id = a.id;
   const bool whole = inner && row_ok && K * lane >= 6 && K * lane + K <= W - 6;
 #pragma unroll
   for (int stage = 0; stage < 3; ++stage) {
@@ -211,7 +210,7 @@ __device__ __forceinline__ void dir_x_wave(const DirArgs& a, const Grid& g, unsi
     auto update = [&](int i, const double cell[4], const double flo[4], const double fhi[4]) {
       double td[4];
 #pragma unroll
-      for (int v = 0; v < kNv; ++v) td[v] = tend_of(flo[v], fhi[v], a.d, id);
+      for (int v = 0; v < kNv; ++v) td[v] = tend_of(flo[v], fhi[v], a.id, a.idl);
       if (a.src_w)
         td[2] = td[2] + a.src_w[(long long)(prow - kHs) * nx + wrap_cell(cell0 + i, nx)];
 #pragma unroll
@@ -338,7 +337,8 @@ __global__ __launch_bounds__(64 * kXwWaves)
 // which then meet in one XCD's L2).
 //
 // Measured (between events, one cell per thread with the RK init in registers
-// / this): 2000 x 1000 63.2 / 55 us, 8192 x 4096 980 / 867 us. Three rows per thread fit
+// / this / with the reciprocal pairs): 2000 x 1000 63.2 / 55 / 50 us, 8192 x
+// 4096 980 / 867 / 786 us. Three rows per thread fit
 // 128 VGPRs (4 waves per SIMD, two 66 KB blocks per CU). Same boxes, not kept:
 // 8 columns x 96 rows in 256 threads 58 and 1200 us (64-byte rows), 4 rows per
 // thread (x 24 row groups) 73 and 1190 us, 6 rows (2 waves per SIMD) 53 and 874
@@ -379,7 +379,6 @@ __device__ __forceinline__ void dir_zt1_tile(const DirArgs& a, const Grid& g, in
   const int base = first ? -2 : last ? nz + 2 - NR : CE + (tile - 1) * C - 6;
   const int own0 = first ? 0 : last ? nz - CE : base + 6;
   const int own1 = last ? nz : min(first ? CE : base + 6 + C, nz - CE);
-  wave_flags_init(sm.wf, NW, t);
   if (t < NR) {
     const int k = min(max(base + t, 0), nz);
     sm.hz[0][t] = a.hyr_int[k];
@@ -447,8 +446,7 @@ __device__ __forceinline__ void dir_zt1_tile(const DirArgs& a, const Grid& g, in
   };
   walls(a.st);
   publish();
-  const int tp = t >= CW ? t - CW : t, tn = t + CW < NT ? t + CW : t;  // rows before, after
-  const double id = a.id;
+  wave_flags_init(sm.wf, NW, t);
   __syncthreads();  // also publishes the flags
 #pragma unroll
   for (int stage = 0; stage < 3; ++stage) {
@@ -457,7 +455,7 @@ __device__ __forceinline__ void dir_zt1_tile(const DirArgs& a, const Grid& g, in
     auto update = [&](int j, const double cell[4], const double flo[4], const double fhi[4]) {
       double td[4];
 #pragma unroll
-      for (int v = 0; v < kNv; ++v) td[v] = tend_of(flo[v], fhi[v], a.d, id);
+      for (int v = 0; v < kNv; ++v) td[v] = tend_of(flo[v], fhi[v], a.id, a.idl);
       td[2] = td[2] - cell[0] * kGrav;
       if (a.src_w)
         td[2] = td[2] + a.src_w[(long long)min(max(k0 + j, 0), nz - 1) * nx + c0 + lcol];
@@ -469,6 +467,7 @@ __device__ __forceinline__ void dir_zt1_tile(const DirArgs& a, const Grid& g, in
           st_off(dst + v * g.plane + ubase + (long long)j * g.ld, lo, s[j][v]);
       }
     };
+    const int tp = t >= CW ? t - CW : t, tn = t + CW < NT ? t + CW : t;  // rows before, after
     double b2[4], b1[4], Fp[4];  // the two rows before, the flux behind
 #pragma unroll
     for (int v = 0; v < kNv; ++v) {
@@ -612,7 +611,6 @@ __device__ __forceinline__ void dir_z1_tile(const DirArgs& a, const Grid& g, int
     }
   }
   gdouble* const tmp_own = a.tmp_interior ? a.tmp : nullptr;
-  const double id = a.id;
   __syncthreads();  // also publishes the flags
 #pragma unroll
   for (int stage = 0; stage < 3; ++stage) {
@@ -631,7 +629,7 @@ __device__ __forceinline__ void dir_z1_tile(const DirArgs& a, const Grid& g, int
     if (colok && j >= e && j <= NR - e - 1 && k >= 0 && k < nz) {
       double td[4];
 #pragma unroll
-      for (int v = 0; v < kNv; ++v) td[v] = tend_of(fl[v][u], fl[v][u + CW], a.d, id);
+      for (int v = 0; v < kNv; ++v) td[v] = tend_of(fl[v][u], fl[v][u + CW], a.id, a.idl);
       td[2] = td[2] - s[0][u] * kGrav;
       if (a.src_w) td[2] = td[2] + src;
       double q[4];
@@ -770,7 +768,6 @@ __device__ __forceinline__ void dir_z1d_tile(const DirArgs& a, const Grid& g, in
     }
   }
   gdouble* const tmp_own = a.tmp_interior ? a.tmp : nullptr;
-  const double id = a.id;
   __syncthreads();  // also publishes the flags
 #pragma unroll
   for (int stage = 0; stage < 3; ++stage) {
@@ -789,7 +786,7 @@ __device__ __forceinline__ void dir_z1d_tile(const DirArgs& a, const Grid& g, in
     if (colok && j >= e && j <= NR - e - 1 && k >= 0 && k < nz) {
       double td[4];
 #pragma unroll
-      for (int v = 0; v < kNv; ++v) td[v] = tend_of(fl[v][u], fl[v][u + CW], a.d, id);
+      for (int v = 0; v < kNv; ++v) td[v] = tend_of(fl[v][u], fl[v][u + CW], a.id, a.idl);
       td[2] = td[2] - s[0][u] * kGrav;
       if (a.src_w) td[2] = td[2] + src;
       double q[4];
@@ -868,8 +865,8 @@ struct MemberDev {
   const double* hypi;  // hy_pressure_int
   const double* src;   // w source or nullptr
   int nx, nz;
-  double dx, dz, dt1, dt2, dt3, hvx, hvz;
-  double idx, idz;       // RN(1/dx), RN(1/dz)
+  double dt1, dt2, dt3, hvx, hvz;
+  double idx, idz, idxl, idzl;  // 1/dx, 1/dz as sums
   int x_start, z_start;  // first work item of this member in the x / z lists
   int x_blocks, z_ncol;  // blocks of the member's x waves, z column groups
 };
@@ -888,8 +885,8 @@ __device__ __forceinline__ DirArgs member_args(const MemberDev& m, int dir, int 
   a.hyt_int = gptr(m.hyti);
   a.hyp_int = gptr(m.hypi);
   a.src_w = m.src ? gptr(m.src) : nullptr;
-  a.d = dir == 0 ? m.dx : m.dz;
   a.id = dir == 0 ? m.idx : m.idz;
+  a.idl = dir == 0 ? m.idxl : m.idzl;
   a.dt1 = m.dt1;
   a.dt2 = m.dt2;
   a.dt3 = m.dt3;
@@ -1152,10 +1149,10 @@ int plan_members(const pmw_member* mem, int n, int x_nt, int z_seg, MemberDev* d
       d.src = m.src_w;
       d.nx = m.nx;
       d.nz = m.nz;
-      d.dx = m.dx;
-      d.dz = m.dz;
       d.idx = 1.0 / m.dx;
       d.idz = 1.0 / m.dz;
+      d.idxl = recip_lo(m.dx, d.idx);
+      d.idzl = recip_lo(m.dz, d.idz);
       d.dt1 = m.dt / 3;
       d.dt2 = m.dt / 2;
       d.dt3 = m.dt / 1;

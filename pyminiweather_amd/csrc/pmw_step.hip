@@ -170,7 +170,7 @@ __global__ void k_flux_z(const double* __restrict__ vals, double* __restrict__ d
 }
 
 __global__ void k_tend_x(const double* __restrict__ flux, double* __restrict__ tend,
-                         Grid g, double dx) {
+                         Grid g, double id, double idl) {
   const long long pt = (long long)g.nz * g.nx;
   const long long n = kNv * pt;
   const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -180,11 +180,12 @@ __global__ void k_tend_x(const double* __restrict__ flux, double* __restrict__ t
   const int v = (int)(idx / pt);
   const long long pf = (long long)(g.nz + 1) * (g.nx + 1);
   const double* f = flux + v * pf + (long long)k * (g.nx + 1) + i;
-  tend[idx] = tend_of(f[0], f[1], dx, 1.0 / dx);
+  tend[idx] = tend_of(f[0], f[1], id, idl);
 }
 
 __global__ void k_tend_z(const double* __restrict__ flux, const double* __restrict__ sf,
-                         double* __restrict__ tend, Grid g, double dz) {
+                         double* __restrict__ tend, Grid g, double id,
+                         double idl) {
   const long long pt = (long long)g.nz * g.nx;
   const long long n = kNv * pt;
   const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -194,7 +195,7 @@ __global__ void k_tend_z(const double* __restrict__ flux, const double* __restri
   const int v = (int)(idx / pt);
   const long long pf = (long long)(g.nz + 1) * (g.nx + 1);
   const double* f = flux + v * pf + (long long)k * (g.nx + 1) + i;
-  double t = tend_of(f[0], f[g.nx + 1], dz, 1.0 / dz);
+  double t = tend_of(f[0], f[g.nx + 1], id, idl);
   if (v == 2) t = t - sf[g.at(0, k + kHs, i + kHs)] * kGrav;
   tend[idx] = t;
 }
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(kXThreads) void k_stage_x(
     const double* init, double* forcing, double* out, double* __restrict__ tend,
     const double* __restrict__ hyr, const double* __restrict__ hyt,
     const double* __restrict__ src_w, int bc, const int* __restrict__ inj_rows,
-    Grid g, double dx, double dt, double hv) {
+    Grid g, double id, double idl, double dt, double hv) {
   __shared__ double sv[kNv][kXThreads];
   __shared__ double sf[kNv][kXThreads];
   const int t = threadIdx.x;
@@ -276,7 +277,7 @@ __global__ __launch_bounds__(kXThreads) void k_stage_x(
   if (t < kXCells && i < nx) {
     double td[4];
 #pragma unroll
-    for (int v = 0; v < kNv; ++v) td[v] = tend_of(sf[v][t], sf[v][t + 1], dx, 1.0 / dx);
+    for (int v = 0; v < kNv; ++v) td[v] = tend_of(sf[v][t], sf[v][t + 1], id, idl);
     const long long cell = (long long)k * nx + i;
     if (src_w) td[2] = td[2] + src_w[cell];
     if (MODE == 0) {
@@ -322,7 +323,8 @@ __global__ __launch_bounds__(kZtCols* kZtRows) void k_stage_z(
     const double* init, double* forcing, double* out, double* __restrict__ tend,
     const double* __restrict__ hy_cell, const double* __restrict__ hyr,
     const double* __restrict__ hyt, const double* __restrict__ hyp,
-    const double* __restrict__ src_w, Grid g, double dz, double dt, double hv, int ncolgrp,
+    const double* __restrict__ src_w, Grid g, double id, double idl, double dt, double hv,
+    int ncolgrp,
     int ntiles, int per_xcd) {
   constexpr int CW = kZtCols, NR = kZtRows, NT = CW * NR, C = NR - 4;
   const int nx = g.nx, nz = g.nz, t = threadIdx.x;
@@ -372,7 +374,7 @@ __global__ __launch_bounds__(kZtCols* kZtRows) void k_stage_z(
   if (colok && j >= 2 && j <= NR - 3 && k >= 0 && k < nz) {
     double td[4];
 #pragma unroll
-    for (int v = 0; v < kNv; ++v) td[v] = tend_of(fl[v][t], fl[v][t + CW], dz, 1.0 / dz);
+    for (int v = 0; v < kNv; ++v) td[v] = tend_of(fl[v][t], fl[v][t + CW], id, idl);
     td[2] = td[2] - s[0][t] * kGrav;
     const long long cell = (long long)k * nx + i;
     if (src_w) td[2] = td[2] + src_w[cell];
@@ -403,12 +405,13 @@ int launch_stage_x(int mode, const double* init, double* forcing, double* out,
                    const double* src_w, int bc, const int* inj_rows, Grid g,
                    double dx, double dt, double hv, hipStream_t st) {
   dim3 grid(blocks_for(g.nx, kXCells), g.nz);
+  const double id = 1.0 / dx, idl = recip_lo(dx, id);
   if (mode == 0)
     k_stage_x<0><<<grid, kXThreads, 0, st>>>(init, forcing, out, tend, hyr, hyt,
-                                            src_w, bc, inj_rows, g, dx, dt, hv);
+                                            src_w, bc, inj_rows, g, id, idl, dt, hv);
   else
     k_stage_x<1><<<grid, kXThreads, 0, st>>>(init, forcing, out, tend, hyr, hyt,
-                                            src_w, bc, inj_rows, g, dx, dt, hv);
+                                            src_w, bc, inj_rows, g, id, idl, dt, hv);
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
@@ -422,12 +425,13 @@ int launch_stage_z(int mode, const double* init, double* forcing, double* out,
   const int ntiles = ncolgrp * ((g.nz + kZtRows - 5) / (kZtRows - 4));
   const int per = (ntiles + kNumXcd - 1) / kNumXcd;
   const unsigned nblk = (unsigned)per * kNumXcd + blocks_for(g.ld, NT);  // + halo writers
+  const double id = 1.0 / dz, idl = recip_lo(dz, id);
   if (mode == 0)
     k_stage_z<0><<<nblk, NT, 0, st>>>(init, forcing, out, tend, hy_cell, hyr, hyt, hyp,
-                                      src_w, g, dz, dt, hv, ncolgrp, ntiles, per);
+                                      src_w, g, id, idl, dt, hv, ncolgrp, ntiles, per);
   else
     k_stage_z<1><<<nblk, NT, 0, st>>>(init, forcing, out, tend, hy_cell, hyr, hyt, hyp,
-                                      src_w, g, dz, dt, hv, ncolgrp, ntiles, per);
+                                      src_w, g, id, idl, dt, hv, ncolgrp, ntiles, per);
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
@@ -530,8 +534,9 @@ int pmw_compute_tend_x(const double* flux, double* tend, int nx, int nz,
                        double dx, void* stream) {
   if (!grid_ok(nx, nz) || bad_ptr(flux) || bad_ptr(tend)) return PMW_EINVAL;
   Grid g(nx, nz);
-  k_tend_x<<<blocks_for(4LL * nz * nx, 256), 256, 0, (hipStream_t)stream>>>(flux, tend,
-                                                                          g, dx);
+  const double id = 1.0 / dx;
+  k_tend_x<<<blocks_for(4LL * nz * nx, 256), 256, 0, (hipStream_t)stream>>>(
+      flux, tend, g, id, recip_lo(dx, id));
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
@@ -541,8 +546,9 @@ int pmw_compute_tend_z(const double* flux, const double* state_forcing,
   if (!grid_ok(nx, nz) || bad_ptr(flux) || bad_ptr(state_forcing) || bad_ptr(tend))
     return PMW_EINVAL;
   Grid g(nx, nz);
+  const double id = 1.0 / dz;
   k_tend_z<<<blocks_for(4LL * nz * nx, 256), 256, 0, (hipStream_t)stream>>>(
-      flux, state_forcing, tend, g, dz);
+      flux, state_forcing, tend, g, id, recip_lo(dz, id));
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
@@ -698,8 +704,7 @@ int evolve_impl(double* state, double* state_tmp, double* state_work,
         a.hyt_int = gptr(hy_dens_theta_int);
         a.hyp_int = gptr(hy_pressure_int);
         a.src_w = gptr(src_w);
-        a.d = dir == 0 ? dx : dz;
-        a.id = 1.0 / a.d;
+        set_spacing(a, dir == 0 ? dx : dz);
         a.dt1 = dts[0];
         a.dt2 = dts[1];
         a.dt3 = dts[2];
