@@ -180,9 +180,9 @@ int pmw_evolve(double* state, double* state_tmp, double* state_work,
 
 /* pmw_evolve with explicit kernel choice and optional per-launch timing.
  * `tuning` (HOST, 3 ints, NULL = defaults {0, 512, 8096}):
- *   [0] mode: 0 = one fused launch per direction (all three RK stages,
- *       periodic x only; the injection BC always uses mode 1), 1 = one
- *       launch per RK stage (the pmw_rk_stage kernels);
+ *   [0] mode: 0 = one fused launch per direction (all three RK stages; the
+ *       injection BC on fewer than 16 columns uses mode 1), 1 = one launch
+ *       per RK stage (the pmw_rk_stage kernels);
  *   [1] fused x kernel: waves over the rows laid end to end (each row with
  *       its 6 periodic cells per side) with one (256) or two (1512) cells
  *       per lane; 448, 512 and 1256 choose between them by the size of the

@@ -20,6 +20,8 @@ struct DirArgs {
   double id, idl;          // 1/dx or 1/dz as a sum (set_spacing)
   double dt1, dt2, dt3;    // dt/3, dt/2, dt
   double hv;               // -hv_beta * d / (16 * dt_full)
+  const PMW_GLOBAL int* inj_rows = nullptr;  // the inflow boundary's row mask: x
+                                             // is not periodic (launch_dir_x)
   gdouble* s1 = nullptr;   // optional: receives the stage-1 interior
   bool tmp_interior = true;  // false: tmp gets only its halo refresh (its
                              // interior is dead when the next direction of
@@ -32,6 +34,10 @@ inline void set_spacing(DirArgs& a, double d) {
   a.id = 1.0 / d;
   a.idl = recip_lo(d, a.id);
 }
+
+// The inflow boundary's fused x direction needs rows of at least this many
+// cells (its copy of the row's right end must not reach the left one).
+constexpr int kMinInflowCells = 16;
 
 bool fused_x_tile_ok(int nt);
 bool fused_z_seg_ok(int seg);

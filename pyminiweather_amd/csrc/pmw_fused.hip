@@ -138,24 +138,37 @@ struct XWaveLds {
 
 __host__ __device__ inline unsigned xw_row_slots(int nx, int K) { return (unsigned)(nx + 12 + K - 1) / K * K; }
 inline long long xw_slots(int nx, int nz, int K) { return (long long)xw_row_slots(nx, K) * nz; }
-inline int xw_blocks(int nx, int nz, int K) {
-  const long long waves = (xw_slots(nx, nz, K) - 13) / (64 * K - 12) + 1;
+inline int xw_blocks(int nx, int nz, int K, bool inflow = false) {
+  const long long waves = (xw_slots(nx, nz, K) - 13) / (64 * K - (inflow ? 16 : 12)) + 1;
   return (int)((waves + kXwWaves - 1) / kXwWaves);
 }
 
+// With the injection inflow (INFLOW, ics/bcs.py:37-64) x is not periodic: the
+// right halo is what the forcing buffer holds (state's in stage 1, state_tmp's
+// in stages 2 and 3; nothing writes it), and the left halo is the right end's
+// cells nx-2, nx-1 of each stage's state, with rho*u and (rho*theta)' set on
+// the inflow rows. A row's E slots are then: its cells nx-6 .. nx-1 once more
+// and the right halo (0-7: enough for nx-2, nx-1 to be right after two
+// stages), the left halo (8, 9), cells 0 .. nx-1, the right halo. The halo
+// slots are refreshed at the start of every stage, the left ones from 4 slots
+// before. Cell 0 depends on 10 slots before it: windows [10, W-6). A step at
+// 1003 x 517 takes 36 us, 66 with one launch per RK stage and the copies of
+// the right halo between them (60 launches and 20 copies per 10 steps became
+// 20 launches).
+//
 // Wave `b` of rows rbase .. rbase+nrows-1; E = xw_row_slots(nx, K).
-template <int K>
+template <int K, bool INFLOW>
 __device__ __forceinline__ void dir_x_wave(const DirArgs& a, const Grid& g, unsigned b,
                                            unsigned E, int rbase, int nrows,
                                            double (*init)[64]) {
-  constexpr int W = 64 * K, C = W - 12;
+  constexpr int W = 64 * K, LM = INFLOW ? 10 : 6, C = W - LM - 6;  // windows [LM, W-6)
   const int nx = g.nx, lane = threadIdx.x & 63;
   const unsigned slot0 = b * (unsigned)C;
   const unsigned row0 = __builtin_amdgcn_readfirstlane(slot0 / E);
   if ((int)row0 >= nrows) return;  // the last block's spare waves
   const unsigned rem = slot0 - row0 * E + (unsigned)(K * lane);
   const unsigned dr0 = rem / E;
-  const int cell0 = (int)(rem - dr0 * E) - 6;
+  const int cell0 = (int)(rem - dr0 * E) - LM;
   const bool row_ok = (int)(row0 + dr0) < nrows;  // else: past the last row, not written
   const unsigned dr = row_ok ? dr0 : (unsigned)nrows - 1 - row0;
   const int prow = rbase + (int)(row0 + dr) + kHs;
@@ -181,10 +194,12 @@ __device__ __forceinline__ void dir_x_wave(const DirArgs& a, const Grid& g, unsi
 #pragma unroll
     for (int i = 0; i < K; ++i) {
       const int c = cell0 + i;
-      const unsigned bw = (lrow + (unsigned)wrap_cell(c, nx)) * 8u;
+      // inflow: slots 0-5 hold cells nx-6 .. nx-1; halo slots are refreshed
+      const int cs = !INFLOW ? wrap_cell(c, nx) : c < -4 ? nx + 4 + c : min(max(c, 0), nx - 1);
+      const unsigned bw = (lrow + (unsigned)cs) * 8u;
 #pragma unroll
       for (int v = 0; v < kNv; ++v) s[i][v] = ld_off(a.in + v * g.plane + rowoff, bw);
-      if (row_ok && (c == -2 || c == -1 || c == nx || c == nx + 1)) {  // set_bc_x of stage 1
+      if (!INFLOW && row_ok && (c == -2 || c == -1 || c == nx || c == nx + 1)) {  // set_bc_x of stage 1
 #pragma unroll
         for (int v = 0; v < kNv; ++v) st_off(a.st + v * g.plane + rowoff, lo + 8u * i, s[i][v]);
       }
@@ -196,10 +211,52 @@ __device__ __forceinline__ void dir_x_wave(const DirArgs& a, const Grid& g, unsi
     for (int v = 0; v < kNv; ++v) init[i * kNv + v][lane] = s[i][v];
   asm volatile("" ::: "memory");  // read back from LDS, not kept in registers
   const double hyr = a.hy_cell[prow], hyt = a.hyt_cell[prow];
-  const bool whole = inner && row_ok && K * lane >= 6 && K * lane + K <= W - 6;
+  const bool whole = inner && row_ok && K * lane >= LM && K * lane + K <= W - 6;
+  const bool row_start =
+      INFLOW && __builtin_amdgcn_ballot_w64(cell0 <= -1 && cell0 + K > -2) != 0;
 #pragma unroll
   for (int stage = 0; stage < 3; ++stage) {
     const double dts = stage == 0 ? a.dt1 : stage == 1 ? a.dt2 : a.dt3;
+    if constexpr (INFLOW) {
+      gdouble* const halo = stage == 0 ? a.st : a.tmp;
+      if (row_start) {  // wave-uniform: the left halo from 4 slots before
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+          const int c = cell0 + i, sl = K * lane + i;
+          double q[4];
+#pragma unroll
+          for (int v = 0; v < kNv; ++v) {
+            q[v] = from_prev(from_prev(s[i][v]));
+            if (K == 1) q[v] = from_prev(from_prev(q[v]));
+          }
+          if (c == -2 || c == -1) {
+            if (a.inj_rows[prow - kHs]) {
+              const double r = q[0] + hyr;
+              q[1] = r * 50.0;
+              q[3] = r * 298.0 - hyt;
+            }
+            // stored where the row's slots 0 .. 9 lie in this wave
+            const bool put = stage != 1 && row_ok && sl >= c + LM;
+#pragma unroll
+            for (int v = 0; v < kNv; ++v) {
+              s[i][v] = q[v];
+              if (put) st_off(halo + v * g.plane + rowoff, lo + 8u * i, q[v]);
+            }
+          }
+        }
+      }
+      if (!inner) {
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+          const int c = cell0 + i, h = c < 0 ? c + 4 : c - nx;  // right halo 0, 1
+          if (h == 0 || h == 1) {
+#pragma unroll
+            for (int v = 0; v < kNv; ++v)
+              s[i][v] = ld_off(halo + v * g.plane + rowoff, (lrow + (unsigned)(nx + h)) * 8u);
+          }
+        }
+      }
+    }
     double b2[4], b1[4], nx1[4];  // cells -2, -1 and K of the lane's run
 #pragma unroll
     for (int v = 0; v < kNv; ++v) {
@@ -261,7 +318,7 @@ __device__ __forceinline__ void dir_x_wave(const DirArgs& a, const Grid& g, unsi
 #pragma unroll
         for (int i = 0; i < K; ++i) {
           const int c = cell0 + i, sl = K * lane + i;
-          if (sl >= 6 && sl < W - 6 && c >= 0 && c < nx) {
+          if (sl >= LM && sl < W - 6 && c >= 0 && c < nx) {
 #pragma unroll
             for (int v = 0; v < kNv; ++v)
               st_off(dst + v * g.plane + rowoff, lo + 8u * i, s[i][v]);
@@ -269,7 +326,7 @@ __device__ __forceinline__ void dir_x_wave(const DirArgs& a, const Grid& g, unsi
         }
       }
     }
-    if (stage == 1 && !inner && row_ok) {  // set_bc_x of stage 3 into tmp
+    if (!INFLOW && stage == 1 && !inner && row_ok) {  // set_bc_x of stage 3 into tmp
 #pragma unroll
       for (int i = 0; i < K; ++i) {
         const int c = cell0 + i, sl = K * lane + i;
@@ -312,8 +369,23 @@ __global__ __launch_bounds__(64 * kXwWaves)
   if (logical >= nreal) return;
   member_offset(a);
   const int rbase = (int)blockIdx.z * rows;
-  dir_x_wave<K>(a, g, xw_wave(logical), E, rbase, min(rows, g.nz - rbase),
-                sm.s[threadIdx.x >> 6]);
+  dir_x_wave<K, false>(a, g, xw_wave(logical), E, rbase, min(rows, g.nz - rbase),
+                       sm.s[threadIdx.x >> 6]);
+}
+
+// the same with the injection inflow
+template <int NS>
+__global__ __launch_bounds__(64 * kXwWaves)
+    __attribute__((amdgpu_waves_per_eu(xw_waves_per_simd(NS / 256)))) void k_dir_xi(
+        DirArgs a, Grid g, unsigned E, int rows, int nreal, int per_xcd) {
+  constexpr int K = NS / 256;
+  __shared__ XWaveLds<K> sm;
+  const int logical = xcd_logical(blockIdx.x, per_xcd);
+  if (logical >= nreal) return;
+  member_offset(a);
+  const int rbase = (int)blockIdx.z * rows;
+  dir_x_wave<K, true>(a, g, xw_wave(logical), E, rbase, min(rows, g.nz - rbase),
+                      sm.s[threadIdx.x >> 6]);
 }
 
 // ------------------------------------------------------------------ z ------
@@ -930,8 +1002,8 @@ __global__ __launch_bounds__(64 * kXwWaves)
   const DirArgs a = member_args(md, 0, pass & 1, pass >> 1);
   const int local = item - md.x_start;
   if (local >= md.x_blocks) return;  // a plan that is not the prepared one: stay in bounds
-  dir_x_wave<K>(a, Grid(md.nx, md.nz), xw_wave(local), xw_row_slots(md.nx, K), 0, md.nz,
-                sm.s[threadIdx.x >> 6]);
+  dir_x_wave<K, false>(a, Grid(md.nx, md.nz), xw_wave(local), xw_row_slots(md.nx, K), 0, md.nz,
+                       sm.s[threadIdx.x >> 6]);
 }
 
 template <int NW, int NR>
@@ -1013,10 +1085,13 @@ int launch_x(const DirArgs& a, Grid g, hipStream_t st, int members) {
   const int rows = (int)std::min<long long>(g.nz, std::max(1LL, (1LL << 31) / E));
   const int chunks = (g.nz + rows - 1) / rows;
   if (chunks > 65535) return PMW_EINVAL;
-  const int nreal = xw_blocks(g.nx, rows, K);
+  const int nreal = xw_blocks(g.nx, rows, K, a.inj_rows != nullptr);
   const int per = (nreal + kNumXcd - 1) / kNumXcd;
-  k_dir_x<256 * K><<<dim3(per * kNumXcd, members, chunks), 64 * kXwWaves, 0, st>>>(
-      a, g, E, rows, nreal, per);
+  const dim3 grid(per * kNumXcd, members, chunks);
+  if (a.inj_rows)
+    k_dir_xi<256 * K><<<grid, 64 * kXwWaves, 0, st>>>(a, g, E, rows, nreal, per);
+  else
+    k_dir_x<256 * K><<<grid, 64 * kXwWaves, 0, st>>>(a, g, E, rows, nreal, per);
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
@@ -1069,7 +1144,7 @@ ZKernel fused_z_kernel(int seg, long long cells, int min_nz, int max_nx) {
 
 int launch_dir_x(const DirArgs& a, Grid g, int nt, hipStream_t st, int members) {
   if (members < 1 || members > 65535 || (members > 1 && a.mstride <= 0)) return PMW_EINVAL;
-  if (!fused_x_tile_ok(nt)) return PMW_EINVAL;
+  if (!fused_x_tile_ok(nt) || (a.inj_rows && g.nx < kMinInflowCells)) return PMW_EINVAL;
   if (nt > 1000 && (long long)g.nz * (g.nx + 12) > (1LL << 30)) return PMW_EINVAL;
   return fused_x_cells(nt, (long long)g.nx * g.nz * members) == 1
              ? launch_x<1>(a, g, st, members)

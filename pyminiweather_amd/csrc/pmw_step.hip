@@ -675,8 +675,8 @@ int evolve_impl(double* state, double* state_tmp, double* state_work,
   Grid g(nx, nz);
   // stage dt as the reference computes them: dt/3, dt/2, dt/1 (step.py:111-141)
   const double dts[3] = {dt / 3, dt / 2, dt / 1};
-  // the injection inflow is only implemented by the per-stage kernels
-  const bool fused = tune.mode == 0 && bc == PMW_BC_PERIODIC;
+  // rows too narrow for the fused inflow take the per-stage kernels
+  const bool fused = tune.mode == 0 && (bc == PMW_BC_PERIODIC || nx >= kMinInflowCells);
   int launch = 0;
   auto rec = [&](int k, int dir) -> int {
     if (!ev) return PMW_OK;
@@ -704,6 +704,7 @@ int evolve_impl(double* state, double* state_tmp, double* state_work,
         a.hyt_int = gptr(hy_dens_theta_int);
         a.hyp_int = gptr(hy_pressure_int);
         a.src_w = gptr(src_w);
+        a.inj_rows = bc == PMW_BC_INJECTION ? gptr(inj_rows) : nullptr;
         set_spacing(a, dir == 0 ? dx : dz);
         a.dt1 = dts[0];
         a.dt2 = dts[1];

@@ -14,8 +14,9 @@ ctypes call into libpmw.so:
   reference (``fused=False`` runs the per-function kernels, which also fill
   the reference's intermediates).
 * ``evolve`` (solve/step.py:85-143): one launch per direction, each running
-  the three RK stages of that direction in LDS tiles (per-stage launches
-  for the injection BC, or when chosen by the tuning). The first direction
+  the three RK stages of that direction on chip (per-stage launches for the
+  injection BC on fewer than 16 columns, or when chosen by the tuning). The
+  first direction
   writes ``fields.state_work`` so no launch reads and writes one buffer;
   ``state`` and ``state_tmp`` end up exactly as the reference leaves them.
 
@@ -191,7 +192,7 @@ def discrete_step(params, fields, mesh, state_init, state_forcing, state_out, dt
               fields.nx, fields.nz, float(dt), _st(fields))
 
 
-# Kernel choice for evolve: (mode, fused x block size, fused z segment rows).
+# Kernel choice for evolve: (mode, x code, z code), see include/pmw.h.
 # mode 0 = one fused launch per direction, 1 = one launch per RK stage. The
 # per-grid entries are filled by pyminiweather_amd.autotune.
 DEFAULT_TUNING = (0, 512, 8096)
