@@ -63,26 +63,7 @@ __device__ __forceinline__ int wrapc(int c, int n) {
 
 // q^(gamma-1) for dp/dq = gamma C0 q^(gamma-1) (q = rho*theta at a face): a
 // derivative, so a few-ulp power.
-__device__ __forceinline__ double dpow(double q) { return pow_pos_fast(q, kGamma - 1.0); }
-
-// dpow(q) continued from dpow(q0) = p0 at a nearby q0: q^a = p0 (1 + e)^a,
-// e = (q - q0)/q0, by the binomial series to e^4 (truncation below 3e-17
-// for |e| <= 2^-10); ok is set false for larger changes (and NaN), where
-// the caller evaluates dpow(q) itself. 1/q0 is the hardware reciprocal
-// (2^29 ulp) with one Newton step, ~2^-46 relative, which moves the result
-// by less than 0.4 |e| 2^-46 < 4e-17. The adjoint tiles' later stages
-// reverse the same face.
-__device__ __forceinline__ double dpow_near(double q, double q0, double p0, bool& ok) {
-  double r = __builtin_amdgcn_rcp(q0);
-  r = fma(fma(-q0, r, 1.0), r, r);
-  const double e = (q - q0) * r;
-  ok = fabs(e) <= 0x1p-10;
-  double c = -0x1.54c5337464d59p-5;          // a(a-1)(a-2)(a-3)/24, a = gamma - 1
-  c = c * e + 0x1.0628bd48c9ba4p-4;          // a(a-1)(a-2)/6
-  c = c * e + -0x1.eba2540426299p-4;         // a(a-1)/2
-  c = c * e + 0x1.99e2b8f2ca162p-2;          // a
-  return p0 + p0 * (e * c);
-}
+__device__ __forceinline__ double dpow(double q) { return pow_gamma_minus_one(q); }
 
 // Primitive variables of a face and dp/dq (q = rho*theta, p = C0 q^gamma)
 // from pw = dpow(q): one division per face.
@@ -406,42 +387,45 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
     prow = p + kHs;
   }
   const bool own = inside && j >= H && j < H + C && (DIR == 0 ? p < nx : true);
-  // lam3 (zero outside the domain), lamS2 cleared
-  // acc: the init terms lam3 + lamS2 + lamS1, summed as the stages finish
-  double acc[4];
+  // Every load of the tile's start is issued before the first is waited for:
+  // lam3, S2 and the hydrostatic values of this thread's face (z) or row (x;
+  // the same for the three stages). Slots outside the domain load the nearest
+  // row and column inside it.
+  const long long cell_at =
+      DIR == 0 ? g.at(0, prow, pcol)
+               : g.at(0, min(max(p, 0), nz - 1) + kHs, min(pcol, nx + kHs - 1));
+  auto load_state = [&](const double* src, double q[4]) {
 #pragma unroll
-  for (int v = 0; v < kNv; ++v) {
-    acc[v] = inside ? a.lam[off + g.at(v, prow, pcol)] : 0.0;
-    sm.la[v][t] = acc[v];
-  }
-  // this thread's slot of a forcing state (wall halo rows rebuilt)
-  auto fetch_state = [&](const double* src, double q[4]) {
+    for (int v = 0; v < kNv; ++v) q[v] = src[off + v * g.plane + cell_at];
+  };
+  // the slot's value of a loaded forcing state (wall halo rows rebuilt)
+  auto slot_state = [&](double q[4]) {
+    if (DIR == 1 && !inside) {
 #pragma unroll
-    for (int v = 0; v < kNv; ++v) {
-      q[v] = 0.0;
-      if (inside)
-        q[v] = src[off + g.at(v, prow, pcol)];
-      else if (wall)
-        q[v] = wall_halo(v, src[off + g.at(v, pe, pcol)], a.hy_cell[pe], a.hy_cell[prow]);
+      for (int v = 0; v < kNv; ++v)
+        q[v] = wall ? wall_halo(v, q[v], a.hy_cell[pe], a.hy_cell[prow]) : 0.0;
     }
   };
-  {
-    double q[4];
-    fetch_state(a.s[2], q);
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) sm.st[v][t] = q[v];
-  }
-  // hydrostatic values of this thread's face (z) or row (x): the same for
-  // the three stages, loaded once
-  double hy_r = 0.0, hy_t = 0.0;
+  // acc: the init terms lam3 + lamS2 + lamS1, summed as the stages finish
+  double acc[4], q2[4];
+  load_state(a.lam, acc);
+  load_state(a.s[2], q2);
+  double hy_r, hy_t;
   if (DIR == 0) {
     hy_r = a.hy_cell[prow];
     hy_t = a.hyt_cell[prow];
-  } else if (pcol - kHs < nx && p >= 0 && p <= nz) {
-    hy_r = a.hyr_int[p];
-    hy_t = a.hyt_int[p];
+  } else {
+    const int kf = min(max(p, 0), nz);
+    hy_r = a.hyr_int[kf];
+    hy_t = a.hyt_int[kf];
   }
-  double q0 = 1.0, p0 = 1.0;  // this face's stage-3 power reference
+  slot_state(q2);
+#pragma unroll
+  for (int v = 0; v < kNv; ++v) {
+    if (!inside) acc[v] = 0.0;  // lam3 is zero outside the domain
+    sm.la[v][t] = acc[v];
+    sm.st[v][t] = q2[v];
+  }
   __syncthreads();
 #pragma unroll
   for (int m = 0; m < 3; ++m) {  // m = 0: stage 3 (forcing S2), 1: stage 2, 2: stage 1
@@ -452,38 +436,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
     // the next stage's forcing state, loaded now and stored to LDS once this
     // stage's faces are done, so the loads overlap the face arithmetic
     double nq[4];
-    if (m < 2) fetch_state(a.s[stage - 1], nq);
+    if (m < 2) load_state(a.s[stage - 1], nq);
     // faces at slots 2+2m .. NR-2-2m (z: faces outside 0..nz are zero)
     const bool zout = DIR == 1 && (p < 0 || p > nz);
-    bool pok = true;
     if (zout) {
 #pragma unroll
       for (int q = 0; q < kNv; ++q) sm.fw[q][t] = 0.0;
     } else if (j >= 2 + 2 * m && j <= NR - 2 - 2 * m && (DIR == 0 || col + (blk % nline) * CW < nx)) {
-      double val[4], lf[4], lv[4], ld[4];
-#pragma unroll
-      for (int v = 0; v < kNv; ++v)
-        val[v] = recon_val(sm.st[v][t - 2 * S], sm.st[v][t - S], sm.st[v][t], sm.st[v][t + S]);
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) lf[v] = sd * (lin[v][t] - lin[v][t - S]);
-      // the face's power: evaluated at stage 3, continued at stages 2 and 1
-      const double q = val[3] + hy_t;
-      double pw;
-      if (m == 0) {
-        pw = dpow(q);
-        q0 = q;
-        p0 = pw;
-      } else {
-        pw = dpow_near(q, q0, p0, pok);
-      }
-      if (DIR == 0)
-        adj_flux_x(val, hy_r, hy_t, a.hv, lf, lv, ld, pw);
-      else
-        adj_flux_z(val, hy_r, hy_t, a.hv, p == 0 || p == nz, lf, lv, ld, pw);
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) sm.fw[v][t] = lv[v];
-    }
-    if (!pok) {  // the face again with the power itself (rare)
       double val[4], lf[4], lv[4], ld[4];
 #pragma unroll
       for (int v = 0; v < kNv; ++v)
@@ -563,6 +522,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
     }
     if (m < 2) {
       // next forcing state; st is free once the faces are done
+      slot_state(nq);
 #pragma unroll
       for (int v = 0; v < kNv; ++v) sm.st[v][t] = nq[v];
       __syncthreads();  // every cell has read its neighbours' la

@@ -1,6 +1,7 @@
 // Host check of pow_gamma (pyminiweather_amd/csrc/pmw_pow.h) against a
 // 113-bit reference (quadmath powq, rounded once to double).
-// Usage: pow_gamma_check N lo hi -> prints "N not_correctly_rounded special_mismatches"
+// Usage: pow_gamma_check N lo hi -> prints "N not_correctly_rounded special_mismatches
+// max_relative_error_of_pow_gamma_minus_one"
 #include <quadmath.h>
 #include <cmath>
 #include <cstdint>
@@ -15,11 +16,14 @@ int main(int argc, char** argv) {
   const double lo = atof(argv[2]), hi = atof(argv[3]);
   uint64_t s = 0x9E3779B97F4A7C15ULL;
   long long bad = 0;
+  double m1 = 0.0;
   for (long long i = 0; i < n; ++i) {
     s ^= s << 13; s ^= s >> 7; s ^= s << 17;
     const double u = (double)(s >> 11) * 0x1p-53;
     const double x = exp(log(lo) + u * (log(hi) - log(lo)));
     bad += pmw::pow_gamma(x) != (double)powq((__float128)x, (__float128)kGam);
+    const __float128 ex = powq((__float128)x, (__float128)(kGam - 1.0));
+    m1 = fmax(m1, fabs((double)(((__float128)pmw::pow_gamma_minus_one(x) - ex) / ex)));
   }
   int special = 0;
   // signs, zeros, infinities, NaN, subnormals, the edges of overflow, and the
@@ -30,6 +34,8 @@ int main(int argc, char** argv) {
     const double a = pmw::pow_gamma(x);
     const double b = x < 0.0 && !std::isinf(x) ? NAN : (double)powq((__float128)x, (__float128)kGam);
     special += !same(a, b);
+    const double c = pmw::pow_gamma_minus_one(x);  // NaN unless positive and normal
+    special += std::isnan(c) == (x >= 0x1p-1022 && std::isfinite(x));
   }
   for (int e = -600; e <= 700; e += 25)
     for (int j = 0; j < 512; ++j)
@@ -38,6 +44,6 @@ int main(int argc, char** argv) {
         x = d < 0 ? nextafter(x, 0.0) : d > 0 ? nextafter(x, INFINITY) : x;
         bad += pmw::pow_gamma(x) != (double)powq((__float128)x, (__float128)kGam);
       }
-  printf("%lld %lld %d\n", n, bad, special);
+  printf("%lld %lld %d %.6g\n", n, bad, special, m1);
   return 0;
 }
