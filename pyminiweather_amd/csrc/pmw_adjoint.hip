@@ -31,6 +31,8 @@
 // with S_{k+1} in slot 6k+6; pmw_tape_adjoint sweeps the steps backwards
 // from it, one launch per direction (all three adjoint stages) for all
 // members.
+#include <algorithm>
+
 #include "pmw_common.h"
 #include "pmw_fused.h"
 
@@ -46,7 +48,7 @@ namespace {
 // The 4-tap face value alone (the adjoint's faces need no third
 // difference), symmetric taps summed first.
 __device__ __forceinline__ double recon_val(double s0, double s1, double s2, double s3) {
-  return (s0 + s3) * kW4a + (s1 + s2) * kW4b;
+  return fma(s0 + s3, kW4a, (s1 + s2) * kW4b);
 }
 
 constexpr double kW4[4] = {kW4a, kW4b, kW4b, kW4a};
@@ -85,10 +87,11 @@ __device__ __forceinline__ void adj_flux_x(const double val[4], double hyr, doub
                                            double ld[4], double pw) {
   double u, w, t, dp;
   face_prims(val, hyr, hyt, pw, u, w, t, dp);
-  lv[0] = -(u * u) * lf[1] - (u * w) * lf[2] - (u * t) * lf[3];
-  lv[1] = lf[0] + 2.0 * u * lf[1] + w * lf[2] + t * lf[3];
+  const double h = fma(t, lf[3], fma(w, lf[2], u * lf[1]));
+  lv[0] = -(u * h);
+  lv[1] = fma(u, lf[1], lf[0] + h);
   lv[2] = u * lf[2];
-  lv[3] = dp * lf[1] + u * lf[3];
+  lv[3] = fma(dp, lf[1], u * lf[3]);
 #pragma unroll
   for (int v = 0; v < kNv; ++v) ld[v] = -hv * lf[v];
 }
@@ -104,10 +107,11 @@ __device__ __forceinline__ void adj_flux_z(const double val[4], double hyr, doub
     lv[3] = dp * lf[2];
     ld[0] = 0.0;
   } else {
-    lv[0] = -(u * w) * lf[1] - (w * w) * lf[2] - (w * t) * lf[3];
+    const double h = fma(t, lf[3], fma(w, lf[2], u * lf[1]));
+    lv[0] = -(w * h);
     lv[1] = w * lf[1];
-    lv[2] = lf[0] + u * lf[1] + 2.0 * w * lf[2] + t * lf[3];
-    lv[3] = dp * lf[2] + w * lf[3];
+    lv[2] = fma(w, lf[2], lf[0] + h);
+    lv[3] = fma(dp, lf[2], w * lf[3]);
     ld[0] = -hv * lf[0];
   }
   ld[1] = -hv * lf[1];
@@ -315,25 +319,193 @@ int adj_stage(int dir, const double* f, const double* lam, double scale, const d
 }
 
 // ---- one RK3 direction in one launch --------------------------------------
-// A block holds a line tile: x = one row, NT cells along it (CW = 1); z = CW
-// columns x NR = NT/CW rows (slot t = j*CW + col). The three adjoint stages
-// run in LDS on a tile with a 7-cell halo (each stage widens the dependency
-// by 2 cells, plus 1 for the face before): lamS2 = dt T'(S2)^T lam3 on tile
-// slots 3..NR-4, lamS1 on 5..NR-6, lamS on 7..NR-8 (the NR-14 output cells).
-// Per cell and direction it reads S, S1, S2 and lam3 once and writes lamS.
 struct AdjDirArgs {
-  const double* s[3];  // forcing states of RK stages 1..3: S, S1, S2
-  const double* lam;   // cotangent of the direction's result
-  double* out;         // cotangent of its start state (must not alias lam)
-  const double* hy_cell;
-  const double* hyt_cell;
-  const double* hyr_int;
-  const double* hyt_int;
+  const gdouble* s[3];  // forcing states of RK stages 1..3: S, S1, S2
+  const gdouble* lam;   // cotangent of the direction's result
+  gdouble* out;         // cotangent of its start state (must not alias lam)
+  const gdouble* hy_cell;
+  const gdouble* hyt_cell;
+  const gdouble* hyr_int;
+  const gdouble* hyt_int;
   double dts[3];       // dt/3, dt/2, dt
-  double d, id, hv;
+  double id, hv;
   long long mstride;
 };
 
+// What one variable of face f, between cells f-1 and f, gives to the cells
+// f-2 .. f+1 it was reconstructed from: kW4[j] lv + kD3[j] ld.
+struct FaceTaps {
+  double m2, m1, p0, p1;
+};
+__device__ __forceinline__ FaceTaps face_taps(double lv, double ld) {
+  const double b = kW4b * lv;
+  return {fma(kW4a, lv, -ld), fma(3.0, ld, b), fma(-3.0, ld, b), fma(kW4a, lv, ld)};
+}
+
+// x: the waves of the forward x direction (K cells per lane in registers, the
+// rows laid end to end, neighbours by one-lane shifts), with windows of 7: a
+// stage widens the dependency by 2 cells, and by 1 for the face before. No LDS
+// and no barrier: bound by HBM and by the launch on one small grid. Per step of
+// the reverse sweep (both directions), LDS tiles of one cell per thread / these
+// waves: 400 x 200 20.2 / 18.4 us, 16 of them 130.2 / 123.0, 64 of 200 x 100
+// 140.7 / 133.0, 1003 x 517 62.0 / 59.2. Two cells per lane keep 8-byte loads:
+// 16-byte ones (inside rows only) spill and take 135 us where these take 123.
+constexpr int kAxWaves = 4;  // waves per block (they share nothing)
+constexpr int kAxH = 7;
+
+__host__ __device__ inline unsigned ax_row_slots(int nx, int K) {
+  return (unsigned)(nx + 2 * kAxH + K - 1) / K * K;
+}
+
+template <int K>
+__device__ __forceinline__ void adj_x_wave(const AdjDirArgs& a, const Grid& g, unsigned b,
+                                           unsigned E, int rbase, int nrows) {
+#pragma clang fp contract(off)  // the same bits for every K
+  constexpr int W = 64 * K, C = W - 2 * kAxH;
+  const int nx = g.nx, lane = threadIdx.x & 63;
+  const unsigned slot0 = b * (unsigned)C;
+  const unsigned row0 = __builtin_amdgcn_readfirstlane(slot0 / E);
+  if ((int)row0 >= nrows) return;  // the last block's spare waves
+  const unsigned rem = slot0 - row0 * E + (unsigned)(K * lane);
+  const unsigned dr0 = rem / E;
+  const int cell0 = (int)(rem - dr0 * E) - kAxH;
+  const bool row_ok = (int)(row0 + dr0) < nrows;  // else: past the last row, not written
+  const unsigned dr = row_ok ? dr0 : (unsigned)nrows - 1 - row0;
+  const int prow = rbase + (int)(row0 + dr) + kHs;
+  const long long rowoff = (long long)(rbase + (int)row0 + kHs) * g.ld +
+                           (long long)blockIdx.y * a.mstride;  // wave-uniform
+  const unsigned lrow = dr * (unsigned)g.ld + kHs;             // the lane's row
+  const bool inner = cell0 >= 0 && cell0 + K <= nx;
+  unsigned lo[K];
+#pragma unroll
+  for (int i = 0; i < K; ++i) lo[i] = (lrow + (unsigned)wrap_cell(cell0 + i, nx)) * 8u;
+  auto load = [&](const gdouble* src, double q[K][4]) {
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) {
+      const gdouble* base = src + v * g.plane + rowoff;
+#pragma unroll
+      for (int i = 0; i < K; ++i) q[i][v] = ld_off(base, lo[i]);
+    }
+  };
+  // every load of the first stage is issued before the first is waited for,
+  // each later stage's state while the stage before is computed
+  double acc[K][4], la[K][4], q[K][4], nq[K][4];
+  load(a.lam, la);
+  load(a.s[2], q);
+  load(a.s[1], nq);
+  const double hyr = a.hy_cell[prow], hyt = a.hyt_cell[prow];
+#pragma unroll
+  for (int i = 0; i < K; ++i)
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) acc[i][v] = la[i][v];  // lam3 + lamS2 + lamS1
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {  // m = 0: stage 3 (forcing S2), 1: stage 2, 2: stage 1
+    const double sd = a.dts[2 - m] * a.id;
+    double b2[4], b1[4], nx1[4], lb[4];  // cells -2, -1, K of the lane's run; lam of -1
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) {
+      b1[v] = from_prev(q[K - 1][v]);
+      b2[v] = K == 1 ? from_prev(b1[v]) : from_prev(q[0][v]);
+      nx1[v] = from_next(q[0][v]);
+      lb[v] = from_prev(la[K - 1][v]);
+    }
+    FaceTaps ft[K][4];
+#pragma unroll
+    for (int j = 0; j < K; ++j) {  // face between cells j-1 and j
+      double val[4], lf[4], lv[4], ld[4];
+#pragma unroll
+      for (int v = 0; v < kNv; ++v) {
+        const double c0 = q[j][v], c1 = j + 1 < K ? q[K - 1][v] : nx1[v];
+        val[v] = recon_val(j == 0 ? b2[v] : b1[v], j == 0 ? b1[v] : q[0][v], c0, c1);
+        lf[v] = sd * (la[j][v] - (j == 0 ? lb[v] : la[0][v]));
+      }
+      adj_flux_x(val, hyr, hyt, a.hv, lf, lv, ld, dpow(val[3] + hyt));
+#pragma unroll
+      for (int v = 0; v < kNv; ++v) ft[j][v] = face_taps(lv[v], ld[v]);
+    }
+    double l[K][4];
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) {
+      const double t = from_prev(ft[K - 1][v].p1);
+      if constexpr (K == 1) {
+        const double r = from_next(ft[0][v].m1 + from_next(ft[0][v].m2));
+        l[0][v] = (ft[0][v].p0 + t) + r;
+      } else {
+        const double r = from_next(ft[0][v].m1 + ft[K - 1][v].m2);
+        l[0][v] = (ft[0][v].p0 + t) + (ft[K - 1][v].m1 + from_next(ft[0][v].m2));
+        l[K - 1][v] = (ft[K - 1][v].p0 + ft[0][v].p1) + r;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < K; ++i)
+#pragma unroll
+      for (int v = 0; v < kNv; ++v) {
+        la[i][v] = l[i][v];
+        acc[i][v] = acc[i][v] + l[i][v];
+        q[i][v] = nq[i][v];
+      }
+    if (m == 0) load(a.s[0], nq);
+  }
+  if (inner && row_ok && K * lane >= kAxH && K * lane + K <= W - kAxH) {
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) {
+      PMW_GLOBAL char* p =
+          (PMW_GLOBAL char*)sgpr64((unsigned long long)(a.out + v * g.plane + rowoff)) + lo[0];
+      if constexpr (K == 2)
+        *(PMW_GLOBAL dpair*)p = dpair{acc[0][v], acc[K - 1][v]};
+      else
+        *(gdouble*)p = acc[0][v];
+    }
+  } else if (row_ok) {
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      const int c = cell0 + i, sl = K * lane + i;
+      if (sl >= kAxH && sl < W - kAxH && c >= 0 && c < nx) {
+#pragma unroll
+        for (int v = 0; v < kNv; ++v) st_off(a.out + v * g.plane + rowoff, lo[i], acc[i][v]);
+      }
+    }
+  }
+}
+
+template <int K>
+__global__ __launch_bounds__(64 * kAxWaves) __attribute__((amdgpu_waves_per_eu(K == 1 ? 6 : 4)))
+void k_adj_xw(AdjDirArgs a, Grid g, unsigned E, int rows, int nreal, int per_xcd) {
+  const int logical = xcd_logical(blockIdx.x, per_xcd);
+  if (logical >= nreal) return;
+  const int rbase = (int)blockIdx.z * rows;
+  adj_x_wave<K>(a, g, __builtin_amdgcn_readfirstlane((unsigned)logical * kAxWaves + (threadIdx.x >> 6)),
+                E, rbase, min(rows, g.nz - rbase));
+}
+
+// Cells per lane: tuning 384 forces two; 256 goes by size, as the forward x
+// waves do and for the same reasons. Per step of the sweep, one / two cells:
+// 400 x 200 18.4 / 18.8 us, 700 x 350 34.0 / 35.4, 800 x 400 44.0 / 43.5, 64 of
+// 200 x 100 134.9 / 133.0.
+int adj_x_cells(int nt, long long cells) { return nt == 256 && cells <= 300000 ? 1 : 2; }
+
+template <int K>
+int launch_adj_x(const AdjDirArgs& a, Grid g, int members, hipStream_t st) {
+  const unsigned E = ax_row_slots(g.nx, K);
+  // slots are 32-bit: rows beyond 2^31 of them go to further blockIdx.z
+  const int rows = (int)std::min<long long>(g.nz, std::max(1LL, (1LL << 31) / E));
+  const int chunks = (g.nz + rows - 1) / rows;
+  if (chunks > 65535) return PMW_EINVAL;
+  // the last slot that any row owns is 7 slots before the rows' end
+  const long long waves = ((long long)E * rows - 2 * kAxH - 1) / (64 * K - 2 * kAxH) + 1;
+  const int nreal = (int)((waves + kAxWaves - 1) / kAxWaves);
+  const int per = (nreal + kNumXcd - 1) / kNumXcd;
+  k_adj_xw<K><<<dim3(per * kNumXcd, members, chunks), 64 * kAxWaves, 0, st>>>(a, g, E, rows,
+                                                                             nreal, per);
+  PMW_CHECK_LAUNCH();
+  return PMW_OK;
+}
+
+// z: a block holds CW columns x NR = NT/CW rows (slot t = j*CW + col). The
+// three adjoint stages run in LDS on a tile with a 7-cell halo: lamS2 = dt
+// T'(S2)^T lam3 on tile rows 3..NR-4, lamS1 on 5..NR-6, lamS on 7..NR-8 (the
+// NR-14 output rows). Per cell and direction it reads S, S1, S2 and lam3 once
+// and writes lamS.
 // la holds lam3, then lamS2, then lamS1, each stage's result written in
 // place after its faces are done: a stage's faces read only slots the stage
 // before wrote (faces 2+2m..NR-2-2m read slots 1+2m..NR-2-2m, inside the
@@ -349,58 +521,35 @@ struct AdjDirLds {
   double la[kNv][NT];  // lam3, then lamS2, then lamS1
 };
 
-// Consecutive tiles (neighbouring columns / row segments) go to the same XCD
-// so that the cache lines they share are fetched into one L2.
-__device__ __forceinline__ int adj_xcd_logical(int b, int per_xcd) {
-  return (b % 8) * per_xcd + b / 8;
-}
-
-template <int DIR, int CW, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_adj_dir(
-    AdjDirArgs a, Grid g, int nline, int nreal,
-                                                int per_xcd) {
-  constexpr int NR = NT / CW, H = 7, C = NR - 2 * H, S = DIR == 0 ? 1 : CW;
+template <int CW, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_adj_zt(
+    AdjDirArgs a, Grid g, int nline, int nreal, int per_xcd) {
+  constexpr int NR = NT / CW, H = 7, C = NR - 2 * H, S = CW;
   __shared__ AdjDirLds<NT> sm;
-  const int blk = adj_xcd_logical(blockIdx.x, per_xcd);
+  const int blk = xcd_logical(blockIdx.x, per_xcd);
   if (blk >= nreal) return;  // whole block, before any barrier
   const long long off = (long long)blockIdx.y * a.mstride;
   const int nx = g.nx, nz = g.nz, t = threadIdx.x;
   const int j = t / CW, col = t % CW;
-  // line and position along it
-  int prow = 0, pcol = 0, p;
-  bool inside, wall = false;
-  int pe = 0;  // z wall slots: padded edge row
-  if (DIR == 0) {
-    const int k = blk / nline;
-    p = (blk % nline) * C - H + j;
-    prow = k + kHs;
-    pcol = wrapc(p, nx) + kHs;
-    inside = true;
-  } else {
-    const int i = (blk % nline) * CW + col;
-    p = (blk / nline) * C - H + j;
-    pcol = i + kHs;
-    const bool colok = i < nx;
-    inside = colok && p >= 0 && p < nz;
-    wall = colok && (p == -2 || p == -1 || p == nz || p == nz + 1);
-    pe = p < 0 ? kHs : nz + kHs - 1;
-    prow = p + kHs;
-  }
-  const bool own = inside && j >= H && j < H + C && (DIR == 0 ? p < nx : true);
+  const int i = (blk % nline) * CW + col;
+  const int p = (blk / nline) * C - H + j;
+  const int pcol = i + kHs, prow = p + kHs;
+  const bool colok = i < nx;
+  const bool inside = colok && p >= 0 && p < nz;
+  const bool wall = colok && (p == -2 || p == -1 || p == nz || p == nz + 1);
+  const int pe = p < 0 ? kHs : nz + kHs - 1;  // wall slots: padded edge row
+  const bool own = inside && j >= H && j < H + C;
   // Every load of the tile's start is issued before the first is waited for:
-  // lam3, S2 and the hydrostatic values of this thread's face (z) or row (x;
-  // the same for the three stages). Slots outside the domain load the nearest
+  // lam3, S2 and the hydrostatic values of this thread's face. Slots outside the domain load the nearest
   // row and column inside it.
-  const long long cell_at =
-      DIR == 0 ? g.at(0, prow, pcol)
-               : g.at(0, min(max(p, 0), nz - 1) + kHs, min(pcol, nx + kHs - 1));
-  auto load_state = [&](const double* src, double q[4]) {
+  const long long cell_at = g.at(0, min(max(p, 0), nz - 1) + kHs, min(pcol, nx + kHs - 1));
+  auto load_state = [&](const gdouble* src, double q[4]) {
 #pragma unroll
     for (int v = 0; v < kNv; ++v) q[v] = src[off + v * g.plane + cell_at];
   };
   // the slot's value of a loaded forcing state (wall halo rows rebuilt)
   auto slot_state = [&](double q[4]) {
-    if (DIR == 1 && !inside) {
+    if (!inside) {
 #pragma unroll
       for (int v = 0; v < kNv; ++v)
         q[v] = wall ? wall_halo(v, q[v], a.hy_cell[pe], a.hy_cell[prow]) : 0.0;
@@ -410,15 +559,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
   double acc[4], q2[4];
   load_state(a.lam, acc);
   load_state(a.s[2], q2);
-  double hy_r, hy_t;
-  if (DIR == 0) {
-    hy_r = a.hy_cell[prow];
-    hy_t = a.hyt_cell[prow];
-  } else {
-    const int kf = min(max(p, 0), nz);
-    hy_r = a.hyr_int[kf];
-    hy_t = a.hyt_int[kf];
-  }
+  const int kf = min(max(p, 0), nz);
+  const double hy_r = a.hyr_int[kf], hy_t = a.hyt_int[kf];
   slot_state(q2);
 #pragma unroll
   for (int v = 0; v < kNv; ++v) {
@@ -437,12 +579,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
     // stage's faces are done, so the loads overlap the face arithmetic
     double nq[4];
     if (m < 2) load_state(a.s[stage - 1], nq);
-    // faces at slots 2+2m .. NR-2-2m (z: faces outside 0..nz are zero)
-    const bool zout = DIR == 1 && (p < 0 || p > nz);
+    // faces at slots 2+2m .. NR-2-2m (those outside 0..nz are zero)
+    const bool zout = p < 0 || p > nz;
     if (zout) {
 #pragma unroll
       for (int q = 0; q < kNv; ++q) sm.fw[q][t] = 0.0;
-    } else if (j >= 2 + 2 * m && j <= NR - 2 - 2 * m && (DIR == 0 || col + (blk % nline) * CW < nx)) {
+    } else if (j >= 2 + 2 * m && j <= NR - 2 - 2 * m && colok) {
       double val[4], lf[4], lv[4], ld[4];
 #pragma unroll
       for (int v = 0; v < kNv; ++v)
@@ -450,10 +592,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
 #pragma unroll
       for (int v = 0; v < kNv; ++v) lf[v] = sd * (lin[v][t] - lin[v][t - S]);
       const double pw = dpow(val[3] + hy_t);
-      if (DIR == 0)
-        adj_flux_x(val, hy_r, hy_t, a.hv, lf, lv, ld, pw);
-      else
-        adj_flux_z(val, hy_r, hy_t, a.hv, p == 0 || p == nz, lf, lv, ld, pw);
+      adj_flux_z(val, hy_r, hy_t, a.hv, p == 0 || p == nz, lf, lv, ld, pw);
 #pragma unroll
       for (int v = 0; v < kNv; ++v) sm.fw[v][t] = lv[v];
     }
@@ -468,13 +607,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
       // and sl, at position fp): -hv lamF, lamF formed as the face phase
       // forms it; zero outside 0..nz and for rho' at the walls (z)
       auto ldf = [&](int sl, int fp, int v) {
-        if (DIR == 1 && (fp < 0 || fp > nz || (v == 0 && (fp == 0 || fp == nz)))) return 0.0;
+        if (fp < 0 || fp > nz || (v == 0 && (fp == 0 || fp == nz))) return 0.0;
         return -a.hv * (sd * (lin[v][sl] - lin[v][sl - S]));
       };
-      // Away from the walls (all of x) the four faces' d3 cotangents sum
+      // Away from the walls the four faces' d3 cotangents sum
       // to -hv sd times the fourth difference of lambda at the cell
       // (kD3 = -1, 3, -3, 1 over differences of neighbours).
-      const bool interior = DIR == 0 || (p >= 2 && p <= nz - 3);
+      const bool interior = p >= 2 && p <= nz - 3;
       const double c4 = -a.hv * sd;
 #pragma unroll
       for (int v = 0; v < kNv; ++v) {
@@ -498,27 +637,25 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
           l[v] = w;
         }
       }
-      if (DIR == 1) {
-        if (p == 0 || p == nz - 1) {
-          // the wall halo rows of this edge row: positions -2, -1 or nz, nz+1
-          const int r0w = p == 0 ? -2 : nz;
-          for (int r = r0w; r < r0w + 2; ++r) {
-            double h[4] = {0.0, 0.0, 0.0, 0.0};
+      if (p == 0 || p == nz - 1) {
+        // the wall halo rows of this edge row: positions -2, -1 or nz, nz+1
+        const int r0w = p == 0 ? -2 : nz;
+        for (int r = r0w; r < r0w + 2; ++r) {
+          double h[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int f = r + 2 - q;
-              if (f < 0 || f > nz) continue;
-              const int sl = t + (f - p) * S;
+          for (int q = 0; q < 4; ++q) {
+            const int f = r + 2 - q;
+            if (f < 0 || f > nz) continue;
+            const int sl = t + (f - p) * S;
 #pragma unroll
-              for (int v = 0; v < kNv; ++v) h[v] += kW4[q] * sm.fw[v][sl] + kD3[q] * ldf(sl, f, v);
-            }
-            l[0] += h[0];
-            l[1] += h[1] * a.hy_cell[r + kHs] / a.hy_cell[prow];
-            l[3] += h[3];
+            for (int v = 0; v < kNv; ++v) h[v] += kW4[q] * sm.fw[v][sl] + kD3[q] * ldf(sl, f, v);
           }
+          l[0] += h[0];
+          l[1] += h[1] * a.hy_cell[r + kHs] / a.hy_cell[prow];
+          l[3] += h[3];
         }
-        l[0] += -kGrav * (sc * lw);
       }
+      l[0] += -kGrav * (sc * lw);
     }
     if (m < 2) {
       // next forcing state; st is free once the faces are done
@@ -543,21 +680,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
   }
 }
 
-template <int DIR, int CW, int NT>
-int launch_adj_dir(const AdjDirArgs& a, Grid g, int members, hipStream_t st) {
+template <int CW, int NT>
+int launch_adj_zt(const AdjDirArgs& a, Grid g, int members, hipStream_t st) {
   constexpr int C = NT / CW - 14;
-  int nline;
-  long long nreal;
-  if (DIR == 0) {
-    nline = (g.nx + C - 1) / C;
-    nreal = (long long)nline * g.nz;
-  } else {
-    nline = (g.nx + CW - 1) / CW;
-    nreal = (long long)nline * ((g.nz + C - 1) / C);
-  }
+  const int nline = (g.nx + CW - 1) / CW;
+  const long long nreal = (long long)nline * ((g.nz + C - 1) / C);
   if (nreal > (1LL << 31) - 64) return PMW_EINVAL;
   const int per = (int)((nreal + 7) / 8);
-  k_adj_dir<DIR, CW, NT><<<dim3((unsigned)per * 8, members), NT, 0, st>>>(a, g, nline,
+  k_adj_zt<CW, NT><<<dim3((unsigned)per * kNumXcd, members), NT, 0, st>>>(a, g, nline,
                                                                           (int)nreal, per);
   PMW_CHECK_LAUNCH();
   return PMW_OK;
@@ -745,10 +875,10 @@ int pmw_tape_adjoint(const double* tape, long long tape_len, int members, double
   Grid g(nx, nz);
   hipStream_t st = (hipStream_t)stream;
   AdjDirArgs a;
-  a.hy_cell = hy_dens_cell;
-  a.hyt_cell = hy_dens_theta_cell;
-  a.hyr_int = hy_dens_int;
-  a.hyt_int = hy_dens_theta_int;
+  a.hy_cell = gptr(hy_dens_cell);
+  a.hyt_cell = gptr(hy_dens_theta_cell);
+  a.hyr_int = gptr(hy_dens_int);
+  a.hyt_int = gptr(hy_dens_theta_int);
   a.dts[0] = dt / 3;
   a.dts[1] = dt / 2;
   a.dts[2] = dt / 1;
@@ -761,23 +891,21 @@ int pmw_tape_adjoint(const double* tape, long long tape_len, int members, double
     for (int pass = 1; pass >= 0; --pass) {
       const int dir = pass == 0 ? first : 1 - first;
       const double* s0 = tape + (6LL * k + 3 * pass) * slot;
-      a.s[0] = s0;
-      a.s[1] = s0 + slot;
-      a.s[2] = s0 + 2 * slot;
-      a.lam = bufs[pass == 1 ? 0 : 1];
-      a.out = bufs[pass == 1 ? 1 : 0];
-      a.d = dir == 0 ? dx : dz;
-      a.id = 1.0 / a.d;
+      for (int s = 0; s < 3; ++s) a.s[s] = gptr(s0 + s * slot);
+      a.lam = gptr(bufs[pass == 1 ? 0 : 1]);
+      a.out = gptr(bufs[pass == 1 ? 1 : 0]);
+      a.id = 1.0 / (dir == 0 ? dx : dz);
       a.hv = dir == 0 ? hv_coeff_x : hv_coeff_z;
       int rc;
       if (dir == 0)
-        rc = x_nt == 256 ? launch_adj_dir<0, 1, 256>(a, g, members, st)
-                         : launch_adj_dir<0, 1, 384>(a, g, members, st);
+        rc = adj_x_cells(x_nt, (long long)nx * nz * members) == 1
+                 ? launch_adj_x<1>(a, g, members, st)
+                 : launch_adj_x<2>(a, g, members, st);
       else
-        rc = z_tile == 4256   ? launch_adj_dir<1, 4, 256>(a, g, members, st)
-             : z_tile == 4384 ? launch_adj_dir<1, 4, 384>(a, g, members, st)
-             : z_tile == 8512 ? launch_adj_dir<1, 8, 512>(a, g, members, st)
-                              : launch_adj_dir<1, 2, 256>(a, g, members, st);
+        rc = z_tile == 4256   ? launch_adj_zt<4, 256>(a, g, members, st)
+             : z_tile == 4384 ? launch_adj_zt<4, 384>(a, g, members, st)
+             : z_tile == 8512 ? launch_adj_zt<8, 512>(a, g, members, st)
+                              : launch_adj_zt<2, 256>(a, g, members, st);
       if (rc) return rc;
     }
   }
