@@ -342,7 +342,7 @@ __global__ __launch_bounds__(64 * kXwWaves)
 // phases are ordered by the waves' flags (wave_phase_done).
 //
 // Rows of the tiles: the first holds rows -2 .. NR-3 of the column, the last
-// rows nz+2-NR .. nz+1, so that a wall's halo rows share a thread with their
+// rows nz+2-NR .. nz+1 (nz >= NR - 2), so that a wall's halo rows share a thread with their
 // edge row and set_bc_z between the stages stays in one thread's registers;
 // the tiles between start 6 rows before the first row they own. Next to a wall nothing is lost to the
 // stencil, so the first and last own NR - 8 rows, the others NR - 12. Tiles
@@ -369,21 +369,43 @@ struct ZTileLds {
   int wf[NW + 2];      // wave phase flags
 };
 
-constexpr int kZtCols = 16, kZtK = 3, kZtWaves = 8, kZtRows = 96;
+constexpr int kZtCols = 16, kZtK = 3;
 
-template <int NR>
-struct ZTileRows {
-  static constexpr int C = NR - 12, CE = NR - 8;  // rows owned: inside, at a wall
-  static __host__ __device__ int tiles(int nz) {
-    return nz <= 2 * CE ? 2 : 2 + (nz - 2 * CE + C - 1) / C;
-  }
-};
+// Tiles of 12 nw rows (nw waves) a column of nz >= 12 nw - 2 rows takes; they
+// own 12 nw - 12 rows each inside and 12 nw - 8 at a wall.
+__host__ __device__ inline int zt_tiles(int nz, int nw) {
+  const int c = 12 * nw - 12, ce = 12 * nw - 8;
+  return nz <= 2 * ce ? 2 : 2 + (nz - 2 * ce + c - 1) / c;
+}
+inline long long zt_blocks(int nx, int nz, int nw) {
+  return (long long)((nx + kZtCols - 1) / kZtCols) * zt_tiles(nz, nw);
+}
+constexpr int kZtMinRows = 12 * 4 - 2;
+
+// Waves per tile, 4 or 8, for a launch that takes b4 or b8 tiles of them. Four
+// waves give more and smaller blocks (four per CU instead of two) but share
+// less: a tile of 48 rows owns 36. The GPU holds 4096 of these waves either
+// way, so a launch costs about its rounds of 4096 waves, half of that for the
+// part of the last round that is filled and half for the round; at equal
+// rounds four waves are 10 % faster (blocks start and end earlier). z time per
+// step in us, 8 / 4 waves: 800x400 17.7 / 17.1, 2100x260 21.7 / 21.4, 1600x400
+// (500 blocks of 8, just one round) 22.0 / 24.4, 1003x517 21.4 / 20.7, 3000x200
+// 28.7 / 25.8, 1500x750 34.3 / 33.3, 2000x1000 50.7 / 53.8, 8192x4096 791 /
+// 908; a step of 64 of 200x100 127.8 / 110.6, of 16 of 400x200 103.7 / 101.0;
+// four steps of 48 grids of 200x100 to 800x400 1605 / 1567. Five to seven waves
+// spread unevenly over a CU's four SIMDs: slower throughout (2000x1000 64.5,
+// 64, 58).
+int zt_waves(int min_nz, long long b4, long long b8) {
+  constexpr long long kResident = 4096;
+  auto cost = [](long long w) { return w + (w + kResident - 1) / kResident * kResident; };
+  return min_nz < 12 * 8 - 2 || 10 * cost(4 * b4) <= 11 * cost(8 * b8) ? 4 : 8;
+}
 
 template <int NW, int NR>
 __device__ __forceinline__ void dir_zt1_tile(const DirArgs& a, const Grid& g, int tile, int ntile,
                                              int c0, ZTileLds<NW, NR>& sm, bool corners) {
   constexpr int NT = 64 * NW, CW = kZtCols, K = kZtK, NG = NT / CW;
-  constexpr int C = ZTileRows<NR>::C, CE = ZTileRows<NR>::CE;
+  constexpr int C = NR - 12, CE = NR - 8;  // rows owned: inside, at a wall
   static_assert(NG * K == NR && NT >= NR, "three rows per thread");
   const int nx = g.nx, nz = g.nz, t = threadIdx.x;
   const int col = t % CW, rg = t / CW;
@@ -943,7 +965,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   if (item >= total) return;  // whole block, before any barrier
   const MemberDev& md = m[member_of<1>(m, n, item)];
   const DirArgs a = member_args(md, 1, pass & 1, pass >> 1);
-  const int local = item - md.z_start, ntile = ZTileRows<NR>::tiles(md.nz);
+  const int local = item - md.z_start, ntile = zt_tiles(md.nz, NW);
   if (local >= md.z_ncol * ntile) return;  // as in k_ens_x
   dir_zt1_tile<NW, NR>(a, Grid(md.nx, md.nz), local / md.z_ncol, ntile,
                        (local % md.z_ncol) * kZtCols, sm, local == 0);
@@ -976,9 +998,10 @@ __global__ __launch_bounds__(kZ1Cols * NR) __attribute__((amdgpu_waves_per_eu(6)
   dir_z1d_tile<NR>(a, Grid(md.nx, md.nz), local, sm, local == 0);
 }
 
+template <int NW>
 int launch_zt1(const DirArgs& a, Grid g, hipStream_t st, int members) {
-  constexpr int NW = kZtWaves, NR = kZtRows;
-  const int ncol = (g.nx + kZtCols - 1) / kZtCols, ntile = ZTileRows<NR>::tiles(g.nz);
+  constexpr int NR = 12 * NW;
+  const int ncol = (g.nx + kZtCols - 1) / kZtCols, ntile = zt_tiles(g.nz, NW);
   const int per = (ncol * ntile + kNumXcd - 1) / kNumXcd;
   k_dir_zt1<NW, NR><<<dim3(per * kNumXcd, members), 64 * NW, 0, st>>>(a, g, ncol, ntile, per);
   PMW_CHECK_LAUNCH();
@@ -1055,19 +1078,19 @@ bool fused_z_seg_ok(int seg) {
 // The z kernel of a launch over `cells` cells of grids whose smallest nz and
 // largest nx are given. Codes 18096 and 18128 force the dense one-cell tiles,
 // 8 to 64 the small ones; the others go by size. The three-row tiles need
-// edge tiles that reach past their own rows into the grid only (nz >= NR - 2)
-// and 32-bit offsets inside a tile; they win once their blocks fill the GPU.
-// Step time in us with one-cell tiles of 32 rows / of 96 rows / three-row
-// tiles: 100x50 12.7 / 13.9 / -, 200x100 13.4 / 15.1 / 18.1, 400x200 14.5 /
-// 17.5 / 21.0, 600x300 19.8 / 22.6 / 23.9, 800x400 26.4 / 26.6 / 28.0,
-// 1003x517 37.7 / 39.1 / 37.6, 2000x1000 108 / 99 / 92, 8192x4096 1800 / 1668
-// / 1452. Low columns (nz < 94) of large grids take the one-cell tile whose
-// rows fit them better.
+// edge tiles that reach past their own rows into the grid only (nz >= 46 for
+// their smallest) and 32-bit offsets inside a tile; they win once their blocks
+// fill the GPU. Step time in us, one-cell tiles of 32 rows / three-row tiles of
+// 48: 600x300 18.3 / 20.3, 700x350 22.2 / 21.2, 1000x300 24.8 / 25.9, 800x400
+// 25.4 / 24.6, 2000x200 29.9 / 29.2, 4000x100 31.3 / 30.0, 900x500 31.1 / 29.5.
+// Against one-cell tiles of 96 rows, which remain for columns and rows outside
+// those bounds: 10000x50 40.1 / 40.1, x60 43.3 / 41.4, x80 45.4 / 42.3, x93
+// 66.4 / 53.0.
 enum ZKernel { Z_ROWS3, Z_ONE96, Z_ONE32, Z_DENSE };
 ZKernel fused_z_kernel(int seg, long long cells, int min_nz, int max_nx) {
   if (seg == 18096 || seg == 18128) return Z_DENSE;
-  if (seg <= 64 || cells < 500000) return Z_ONE32;
-  if (min_nz >= kZtRows - 2 && max_nx < (1 << 22)) return Z_ROWS3;
+  if (seg <= 64 || cells <= 300000) return Z_ONE32;
+  if (min_nz >= kZtMinRows && max_nx < (1 << 22)) return Z_ROWS3;
   return min_nz > 40 ? Z_ONE96 : Z_ONE32;
 }
 
@@ -1084,7 +1107,11 @@ int launch_dir_z(const DirArgs& a, Grid g, int seg, hipStream_t st, int members)
   if (members < 1 || members > 65535 || (members > 1 && a.mstride <= 0)) return PMW_EINVAL;
   if (!fused_z_seg_ok(seg)) return PMW_EINVAL;
   switch (fused_z_kernel(seg, (long long)g.nx * g.nz * members, g.nz, g.nx)) {
-    case Z_ROWS3: return launch_zt1(a, g, st, members);
+    case Z_ROWS3:
+      return zt_waves(g.nz, zt_blocks(g.nx, g.nz, 4) * members,
+                      zt_blocks(g.nx, g.nz, 8) * members) == 4
+                 ? launch_zt1<4>(a, g, st, members)
+                 : launch_zt1<8>(a, g, st, members);
     case Z_ONE96: return launch_z1<96>(a, g, st, members);
     case Z_ONE32: return launch_z1<32>(a, g, st, members);
     default:
@@ -1102,19 +1129,23 @@ struct EnsPlan {
   int x_total, z_total;
   int x_k;       // cells per lane of the x waves
   int z_kernel;  // a pmw::ZKernel
+  int z_waves;   // of Z_ROWS3
 };
 
 int plan_members(const pmw_member* mem, int n, int x_nt, int z_seg, MemberDev* dev,
                  EnsPlan& plan) {
-  long long xs = 0, zs = 0, cells = 0;
+  long long xs = 0, zs = 0, cells = 0, zb4 = 0, zb8 = 0;
   int min_nz = 1 << 30, max_nx = 0;
   for (int q = 0; q < n; ++q) {
     cells += (long long)mem[q].nx * mem[q].nz;
+    zb4 += zt_blocks(mem[q].nx, mem[q].nz, 4);
+    zb8 += zt_blocks(mem[q].nx, mem[q].nz, 8);
     min_nz = std::min(min_nz, mem[q].nz);
     max_nx = std::max(max_nx, mem[q].nx);
   }
   plan.x_k = pmw::fused_x_cells(x_nt, cells);
   plan.z_kernel = pmw::fused_z_kernel(z_seg, cells, min_nz, max_nx);
+  plan.z_waves = zt_waves(min_nz, zb4, zb8);
   for (int q = 0; q < n; ++q) {
     const pmw_member& m = mem[q];
     if (m.nx < 2 || m.nz < 2 || !m.state || !m.state_tmp || !m.state_work ||
@@ -1134,7 +1165,7 @@ int plan_members(const pmw_member* mem, int n, int x_nt, int z_seg, MemberDev* d
       zsg = 1;
     } else if (plan.z_kernel == pmw::Z_ROWS3) {
       zc = (m.nx + kZtCols - 1) / kZtCols;
-      zsg = ZTileRows<kZtRows>::tiles(m.nz);
+      zsg = zt_tiles(m.nz, plan.z_waves);
     } else {
       const int rows = plan.z_kernel == pmw::Z_ONE96 ? 96 - 12 : 32 - 12;
       zc = (m.nx + kZ1Cols - 1) / kZ1Cols;
@@ -1234,7 +1265,10 @@ int launch_ens_z(const MemberDev* d, int n, int pass, const EnsPlan& plan, hipSt
   const int total = plan.z_total, per = ens_per_xcd(total), nb = per * kNumXcd;
   switch (plan.z_kernel) {
     case pmw::Z_ROWS3:
-      k_ens_zt1<kZtWaves, kZtRows><<<nb, 64 * kZtWaves, 0, st>>>(d, n, pass, total, per);
+      if (plan.z_waves == 4)
+        k_ens_zt1<4, 48><<<nb, 256, 0, st>>>(d, n, pass, total, per);
+      else
+        k_ens_zt1<8, 96><<<nb, 512, 0, st>>>(d, n, pass, total, per);
       break;
     case pmw::Z_ONE96:
       k_ens_z1<96><<<nb, kZ1Cols * 96, 0, st>>>(d, n, pass, total, per);
