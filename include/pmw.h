@@ -320,8 +320,9 @@ int pmw_tape_forward(double* tape, long long tape_len, int members,
  * then its first; each direction is one launch for all members that runs
  * the three stage adjoints (the formulas of pmw_adjoint_stage) on chip.
  * workspace: 1 slot. tuning: NULL (= {256, 8512}) or {x waves (256: cells per
- * lane by size | 384: two), z tile (columns*1000 + threads: 4256, 4384, 2256, 8512)}. Every
- * choice gives the same result bit for bit. No reference counterpart. */
+ * lane by size | 384: two), z tile (8512: by size | 4256, 4384: 8
+ * columns x 32 rows | 2256: 8 x 64)}. Every choice gives the same result bit for
+ * bit. No reference counterpart. */
 int pmw_tape_adjoint(const double* tape, long long tape_len, int members, double* lam,
                      double* workspace, long long workspace_len, const double* hy_dens_cell,
                      const double* hy_dens_theta_cell, const double* hy_dens_int,

@@ -44,8 +44,8 @@ from ._lib import ptr, stream_of
 from .ics import Directions, check_state
 
 RHOT = 3
-# adjoint kernels: x block threads (256, 384), z tile (columns * 1000 +
-# threads: 4256, 4384, 2256, 8512)
+# adjoint kernels: x waves (256 by size, 384 two cells per lane), z tile (8512
+# by size, 4256 and 4384 8 columns x 32 rows, 2256 8 x 64)
 ADJ_DEFAULT_TUNING = (256, 8512)
 ADJ_TUNINGS = ((256, 4256), (384, 4384), (256, 2256), (256, 8512))
 

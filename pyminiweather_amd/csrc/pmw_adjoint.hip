@@ -502,160 +502,162 @@ int launch_adj_x(const AdjDirArgs& a, Grid g, int members, hipStream_t st) {
 }
 
 // z: a block holds CW columns x NR = NT/CW rows (slot t = j*CW + col). The
-// three adjoint stages run in LDS on a tile with a 7-cell halo: lamS2 = dt
-// T'(S2)^T lam3 on tile rows 3..NR-4, lamS1 on 5..NR-6, lamS on 7..NR-8 (the
-// NR-14 output rows). Per cell and direction it reads S, S1, S2 and lam3 once
-// and writes lamS.
-// la holds lam3, then lamS2, then lamS1, each stage's result written in
-// place after its faces are done: a stage's faces read only slots the stage
-// before wrote (faces 2+2m..NR-2-2m read slots 1+2m..NR-2-2m, inside the
-// cells 3+2(m-1)..NR-4-2(m-1) of stage m-1), and slots outside the domain
-// keep the zero they were loaded with.
-// The face cotangents of the third differences are -hv lamF, so only those
-// of the reconstructed values are kept; a cell forms the others from la
-// (96 B of LDS per slot).
+// three adjoint stages run on a tile with a 7-row halo: lamS2 = dt T'(S2)^T
+// lam3 on tile rows 3..NR-4, lamS1 on 5..NR-6, lamS on 7..NR-8 (the NR-14
+// output rows). Per cell and direction it reads S, S1, S2 and lam3 once and
+// writes lamS.
+// LDS holds the running cotangent la (lam3, then lamS2, then lamS1) and the
+// face cotangents fw of the reconstructed values; those of the third
+// differences are -hv lamF, which a cell forms from la. A stage's faces read
+// only slots the stage before wrote (faces 2+2m..NR-2-2m read slots
+// 1+2m..NR-2-2m, inside the cells 3+2(m-1)..NR-4-2(m-1) of stage m-1), and
+// slots outside the domain keep the zero they were loaded with.
+//
+// Bound by the memory's latency and by its own chain of phases: 24 waves per
+// CU (96 B of LDS per slot, 76 VGPRs) move 384 MB in about 100 us at 2000 x
+// 1000, with the FP64 pipes a third busy. The wall rows are part of every
+// launch's longest blocks: gathered face by face, with a division per halo row
+// and stage / as corrections of the inside formula (below), a step of the sweep
+// takes 200 x 100 16.7 / 12.9 us, 400 x 200 18.4 / 16.4, 16 of them 122.9 /
+// 112.0, 64 of 200 x 100 132.5 / 120.2, 2000 x 1000 177 / 169. Not faster: wave
+// flags instead of the barriers, forcing rows read from memory by each face
+// that needs them (64 KB of taps in LDS, 16 waves per CU: 136 us for the 16),
+// two or three rows per thread (131, 137), loads of the needed rows only.
 template <int NT>
-struct AdjDirLds {
+struct AdjZtLds {
   double st[kNv][NT];  // forcing state of the stage being reversed
-  double fw[kNv][NT];  // face cotangents of the reconstructed values
-  double la[kNv][NT];  // lam3, then lamS2, then lamS1
+  double fw[kNv][NT];
+  double la[kNv][NT];
 };
 
 template <int CW, int NT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_adj_zt(
-    AdjDirArgs a, Grid g, int nline, int nreal, int per_xcd) {
-  constexpr int NR = NT / CW, H = 7, C = NR - 2 * H, S = CW;
-  __shared__ AdjDirLds<NT> sm;
+    AdjDirArgs a, Grid g, int ncol, int nreal, int per_xcd) {
+#pragma clang fp contract(off)  // the same bits in every instance
+  constexpr int NR = NT / CW, H = kAxH, C = NR - 2 * H, S = CW;
+  __shared__ AdjZtLds<NT> sm;
   const int blk = xcd_logical(blockIdx.x, per_xcd);
   if (blk >= nreal) return;  // whole block, before any barrier
-  const long long off = (long long)blockIdx.y * a.mstride;
   const int nx = g.nx, nz = g.nz, t = threadIdx.x;
-  const int j = t / CW, col = t % CW;
-  const int i = (blk % nline) * CW + col;
-  const int p = (blk / nline) * C - H + j;
-  const int pcol = i + kHs, prow = p + kHs;
-  const bool colok = i < nx;
-  const bool inside = colok && p >= 0 && p < nz;
-  const bool wall = colok && (p == -2 || p == -1 || p == nz || p == nz + 1);
-  const int pe = p < 0 ? kHs : nz + kHs - 1;  // wall slots: padded edge row
+  const int j = t / CW, i = (blk % ncol) * CW + t % CW;
+  const int p = (blk / ncol) * C - H + j;
+  const bool colok = i < nx, inside = colok && p >= 0 && p < nz;
   const bool own = inside && j >= H && j < H + C;
-  // Every load of the tile's start is issued before the first is waited for:
-  // lam3, S2 and the hydrostatic values of this thread's face. Slots outside the domain load the nearest
-  // row and column inside it.
-  const long long cell_at = g.at(0, min(max(p, 0), nz - 1) + kHs, min(pcol, nx + kHs - 1));
+  // Slots outside the domain load the nearest row and column inside it.
+  const int pin = min(max(p, 0), nz - 1);
+  const long long cell_at = (long long)blockIdx.y * a.mstride + g.at(0, pin + kHs, min(i, nx - 1) + kHs);
   auto load_state = [&](const gdouble* src, double q[4]) {
 #pragma unroll
-    for (int v = 0; v < kNv; ++v) q[v] = src[off + v * g.plane + cell_at];
+    for (int v = 0; v < kNv; ++v) q[v] = src[v * g.plane + cell_at];
   };
   // the slot's value of a loaded forcing state (wall halo rows rebuilt)
   auto slot_state = [&](double q[4]) {
-    if (!inside) {
+    if (p < 0 || p >= nz) {
+      const bool wall = p >= -2 && p <= nz + 1;
 #pragma unroll
       for (int v = 0; v < kNv; ++v)
-        q[v] = wall ? wall_halo(v, q[v], a.hy_cell[pe], a.hy_cell[prow]) : 0.0;
+        q[v] = wall ? wall_halo(v, q[v], a.hy_cell[pin + kHs], a.hy_cell[p + kHs]) : 0.0;
     }
   };
+  // Every load of the tile's start is issued before the first is waited for.
   // acc: the init terms lam3 + lamS2 + lamS1, summed as the stages finish
-  double acc[4], q2[4];
+  double acc[4], q[4];
   load_state(a.lam, acc);
-  load_state(a.s[2], q2);
+  load_state(a.s[2], q);
   const int kf = min(max(p, 0), nz);
   const double hy_r = a.hyr_int[kf], hy_t = a.hyt_int[kf];
-  slot_state(q2);
+  // rho*u of the halo rows -1, -2 or nz, nz+1 follows the edge row's
+  double edge1 = 0.0, edge2 = 0.0;
+  if (p == 0 || p == nz - 1) {
+    const int out = p == 0 ? -1 : 1;
+    const double ir = 1.0 / a.hy_cell[p + kHs];
+    edge1 = a.hy_cell[p + out + kHs] * ir;
+    edge2 = a.hy_cell[p + 2 * out + kHs] * ir;
+  }
+  slot_state(q);
 #pragma unroll
   for (int v = 0; v < kNv; ++v) {
     if (!inside) acc[v] = 0.0;  // lam3 is zero outside the domain
     sm.la[v][t] = acc[v];
-    sm.st[v][t] = q2[v];
+    sm.st[v][t] = q[v];
   }
   __syncthreads();
 #pragma unroll
   for (int m = 0; m < 3; ++m) {  // m = 0: stage 3 (forcing S2), 1: stage 2, 2: stage 1
-    const int stage = 2 - m;
-    double (*lin)[NT] = sm.la;
-    const double sc = a.dts[stage];
-    const double sd = sc * a.id;
-    // the next stage's forcing state, loaded now and stored to LDS once this
-    // stage's faces are done, so the loads overlap the face arithmetic
+    const double sc = a.dts[2 - m], sd = sc * a.id;
+    // the next stage's forcing state, stored to LDS once this stage's faces
+    // are done: the loads overlap the face arithmetic
     double nq[4];
-    if (m < 2) load_state(a.s[stage - 1], nq);
+    if (m < 2) load_state(a.s[1 - m], nq);
     // faces at slots 2+2m .. NR-2-2m (those outside 0..nz are zero)
-    const bool zout = p < 0 || p > nz;
-    if (zout) {
+    if (p < 0 || p > nz) {
 #pragma unroll
-      for (int q = 0; q < kNv; ++q) sm.fw[q][t] = 0.0;
+      for (int v = 0; v < kNv; ++v) sm.fw[v][t] = 0.0;
     } else if (j >= 2 + 2 * m && j <= NR - 2 - 2 * m && colok) {
       double val[4], lf[4], lv[4], ld[4];
 #pragma unroll
-      for (int v = 0; v < kNv; ++v)
+      for (int v = 0; v < kNv; ++v) {
         val[v] = recon_val(sm.st[v][t - 2 * S], sm.st[v][t - S], sm.st[v][t], sm.st[v][t + S]);
-#pragma unroll
-      for (int v = 0; v < kNv; ++v) lf[v] = sd * (lin[v][t] - lin[v][t - S]);
-      const double pw = dpow(val[3] + hy_t);
-      adj_flux_z(val, hy_r, hy_t, a.hv, p == 0 || p == nz, lf, lv, ld, pw);
+        lf[v] = sd * (sm.la[v][t] - sm.la[v][t - S]);
+      }
+      adj_flux_z(val, hy_r, hy_t, a.hv, p == 0 || p == nz, lf, lv, ld, dpow(val[3] + hy_t));
 #pragma unroll
       for (int v = 0; v < kNv; ++v) sm.fw[v][t] = lv[v];
     }
     __syncthreads();
-    // gravity needs lin[w] at this slot: read before lin may be overwritten
-    const double lw = lin[2][t];
     // cells at slots 3+2m .. NR-4-2m
     double l[4] = {0.0, 0.0, 0.0, 0.0};
     const bool cell = inside && j >= 3 + 2 * m && j <= NR - 4 - 2 * m;
     if (cell) {
-      // d3 cotangent of the face at slot sl (the face between slots sl-S
-      // and sl, at position fp): -hv lamF, lamF formed as the face phase
-      // forms it; zero outside 0..nz and for rho' at the walls (z)
-      auto ldf = [&](int sl, int fp, int v) {
-        if (fp < 0 || fp > nz || (v == 0 && (fp == 0 || fp == nz))) return 0.0;
-        return -a.hv * (sd * (lin[v][sl] - lin[v][sl - S]));
-      };
-      // Away from the walls the four faces' d3 cotangents sum
-      // to -hv sd times the fourth difference of lambda at the cell
-      // (kD3 = -1, 3, -3, 1 over differences of neighbours).
-      const bool interior = p >= 2 && p <= nz - 3;
+      // The four faces' d3 cotangents sum to c4 = -hv sd times the fourth
+      // difference of lambda (kD3 = -1, 3, -3, 1 over differences of
+      // neighbours), at the walls too: lambda and the faces outside are zero.
       const double c4 = -a.hv * sd;
 #pragma unroll
       for (int v = 0; v < kNv; ++v) {
-        double lam[5];  // lin at slots t-2S .. t+2S
+        double lam[5];  // rows p-2 .. p+2
 #pragma unroll
-        for (int i = 0; i < 5; ++i) lam[i] = lin[v][t + (i - 2) * S];
+        for (int i = 0; i < 5; ++i) lam[i] = sm.la[v][t + (i - 2) * S];
         // transposed 4-tap reconstruction (kW4 = a, b, b, a)
-        double w = kW4a * (sm.fw[v][t + 2 * S] + sm.fw[v][t - S]) +
-                   kW4b * (sm.fw[v][t + S] + sm.fw[v][t]);
-        if (interior) {
-          // sum_q kD3[q] (lam[4-q] - lam[3-q]) = 4 (l1 + l3) - (l0 + l4) - 6 l2
-          const double d4 = (4.0 * (lam[1] + lam[3]) - (lam[0] + lam[4])) - 6.0 * lam[2];
-          l[v] = w + c4 * d4;
-        } else {
+        const double w = fma(kW4a, sm.fw[v][t + 2 * S] + sm.fw[v][t - S],
+                             kW4b * (sm.fw[v][t + S] + sm.fw[v][t]));
+        const double d4 = fma(-6.0, lam[2], fma(4.0, lam[1] + lam[3], -(lam[0] + lam[4])));
+        l[v] = fma(c4, d4, w);
+        if (p < 2 || p >= nz - 2) {
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {  // face at slot t+(2-q)S, position p+2-q
-            const int fp = p + 2 - q;
-            const bool zero = fp < 0 || fp > nz || (v == 0 && (fp == 0 || fp == nz));
-            if (!zero) w += kD3[q] * (c4 * (lam[4 - q] - lam[3 - q]));
+          for (int side = 0; side < 2; ++side) {
+            // the difference of lambda at the wall face is +- the edge row's
+            const int d = side == 0 ? p : nz - 1 - p;  // rows from the edge
+            const double e = c4 * lam[2];
+            if (v == 0) {  // rho' has no d3 at the wall face: taken out again
+              if (d == 0) l[0] = fma(3.0, e, l[0]);
+              if (d == 1) l[0] = l[0] - c4 * (side == 0 ? lam[1] : lam[3]);
+            }
+            if (d == 0) {
+              // the halo rows' cotangents fold back onto the edge row
+              // (set_bc_z): next to it h1, beyond h2
+              const double in = c4 * (side == 0 ? lam[3] : lam[1]);
+              const double fo = sm.fw[v][side == 0 ? t : t + S];  // the wall face
+              const double fi = sm.fw[v][side == 0 ? t + S : t];  // the next one inside
+              double h1 = fma(kW4a, fi, e - in), h2 = 0.0;
+              if (v == 3) {  // the wall face passes p alone
+                h1 = fma(kW4b, fo, h1);
+                h2 = kW4a * fo;
+              }
+              if (v != 0) {
+                h1 = fma(3.0, e, h1);
+                h2 = h2 - e;
+              }
+              if (v == 1) {
+                h1 = h1 * edge1;
+                h2 = h2 * edge2;
+              }
+              if (v != 2) l[v] = l[v] + (h1 + h2);
+            }
           }
-          l[v] = w;
         }
       }
-      if (p == 0 || p == nz - 1) {
-        // the wall halo rows of this edge row: positions -2, -1 or nz, nz+1
-        const int r0w = p == 0 ? -2 : nz;
-        for (int r = r0w; r < r0w + 2; ++r) {
-          double h[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int f = r + 2 - q;
-            if (f < 0 || f > nz) continue;
-            const int sl = t + (f - p) * S;
-#pragma unroll
-            for (int v = 0; v < kNv; ++v) h[v] += kW4[q] * sm.fw[v][sl] + kD3[q] * ldf(sl, f, v);
-          }
-          l[0] += h[0];
-          l[1] += h[1] * a.hy_cell[r + kHs] / a.hy_cell[prow];
-          l[3] += h[3];
-        }
-      }
-      l[0] += -kGrav * (sc * lw);
+      l[0] = fma(-kGrav * sc, sm.la[2][t], l[0]);  // T_w -= rho'_forcing * g
     }
     if (m < 2) {
       // next forcing state; st is free once the faces are done
@@ -667,28 +669,36 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
 #pragma unroll
         for (int v = 0; v < kNv; ++v) {
           sm.la[v][t] = l[v];  // in place: this stage's faces are done
-          acc[v] += l[v];
+          acc[v] = acc[v] + l[v];
         }
       }
       __syncthreads();
     } else if (own) {
 #pragma unroll
-      for (int v = 0; v < kNv; ++v) {
-        a.out[off + g.at(v, prow, pcol)] = l[v] + acc[v];
-      }
+      for (int v = 0; v < kNv; ++v) a.out[v * g.plane + cell_at] = l[v] + acc[v];
     }
   }
 }
 
+// z tile: 8 columns x 32 rows or x 64. Tunings 4256 and 4384 force the small
+// one, 2256 the large; 8512 goes by size: small tiles while a launch takes
+// little longer than one block. Per step of the sweep in us, 32 / 64 rows:
+// 100x50 12.5 / 13.6, 200x100 12.9 / 14.7, 4 of 100x50 13.1 / 14.8, 300x150
+// 14.1 / 15.1, 400x200 17.0 / 16.5, 600x300 26.5 / 26.0. Tiles of 4 and 2
+// columns, 16 columns, 96 rows: slower on every size.
+bool adj_z_small(int tile, long long cells) {
+  return tile == 8512 ? cells <= 60000 : tile != 2256;
+}
+
 template <int CW, int NT>
 int launch_adj_zt(const AdjDirArgs& a, Grid g, int members, hipStream_t st) {
-  constexpr int C = NT / CW - 14;
-  const int nline = (g.nx + CW - 1) / CW;
-  const long long nreal = (long long)nline * ((g.nz + C - 1) / C);
+  const int ncol = (g.nx + CW - 1) / CW;
+  constexpr int C = NT / CW - 2 * kAxH;
+  const long long nreal = (long long)ncol * ((g.nz + C - 1) / C);
   if (nreal > (1LL << 31) - 64) return PMW_EINVAL;
-  const int per = (int)((nreal + 7) / 8);
-  k_adj_zt<CW, NT><<<dim3((unsigned)per * kNumXcd, members), NT, 0, st>>>(a, g, nline,
-                                                                          (int)nreal, per);
+  const int per = (int)((nreal + kNumXcd - 1) / kNumXcd);
+  k_adj_zt<CW, NT><<<dim3((unsigned)per * kNumXcd, members), NT, 0, st>>>(
+      a, g, ncol, (int)nreal, per);
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
@@ -902,10 +912,9 @@ int pmw_tape_adjoint(const double* tape, long long tape_len, int members, double
                  ? launch_adj_x<1>(a, g, members, st)
                  : launch_adj_x<2>(a, g, members, st);
       else
-        rc = z_tile == 4256   ? launch_adj_zt<4, 256>(a, g, members, st)
-             : z_tile == 4384 ? launch_adj_zt<4, 384>(a, g, members, st)
-             : z_tile == 8512 ? launch_adj_zt<8, 512>(a, g, members, st)
-                              : launch_adj_zt<2, 256>(a, g, members, st);
+        rc = adj_z_small(z_tile, (long long)nx * nz * members)
+                 ? launch_adj_zt<8, 256>(a, g, members, st)
+                 : launch_adj_zt<8, 512>(a, g, members, st);
       if (rc) return rc;
     }
   }

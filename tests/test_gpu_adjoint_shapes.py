@@ -59,3 +59,11 @@ def test_x_waves_match_stages(nx, tuning):
     """Rows shorter than a wave, of one wave's cells and one more or less,
     several rows and members per block, one and two cells per lane."""
     _check(nx, 5, 2, tuning)
+
+
+@pytest.mark.parametrize("tuning", [(256, 8512), (256, 4256), (256, 2256)])
+@pytest.mark.parametrize("nz", [2, 3, 4, 17, 18, 19, 36, 37, 49, 50, 51, 100, 101])
+def test_z_tiles_match_stages(nz, tuning):
+    """Columns of a few rows (both walls in one thread's reach), of one tile's
+    rows and one more or less, of two tiles, with a ragged last column group."""
+    _check(21, nz, 2, tuning)
