@@ -102,18 +102,24 @@ def load():
 
 def call(name, *args):
     """Call an int-returning entry point and raise PMWError on failure."""
-    lib = load()
+    lib = _lib or load()
     rc = getattr(lib, name)(*args)
     if rc != 0:
         raise PMWError(name, rc, lib.pmw_error_string(rc).decode())
     return rc
 
 
+# Addresses and streams are passed as plain integers: every signature above
+# declares its arguments, and building a c_void_p for each, with torch's Stream
+# object on top, took a third of the host time of a small call.
 def ptr(t):
     """Device address of a tensor (None passes NULL)."""
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def stream_of(device=None):
     """hipStream_t handle of torch's current stream on `device`."""
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    index = getattr(device, "index", None)
+    if index is not None and device.type == "cuda":
+        return torch._C._cuda_getCurrentRawStream(index)
+    return torch.cuda.current_stream(device).cuda_stream

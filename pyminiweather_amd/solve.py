@@ -41,10 +41,13 @@ from .ics import BC_INJECTION, Directions, bc_code, check_state, set_bc_x, set_b
 reverse_direction: bool = False
 
 
+_HV_BETA = Constants.hv_beta.value
+
+
 def hv_coeff(d, dt_full):
     """Hyperviscosity coefficient -hv_beta * d / (16 * dt) with the FULL
     timestep params["dt"] (solve/interpolate.py:99-101, 147-149)."""
-    return -Constants.hv_beta.value * d / (16 * dt_full)
+    return -_HV_BETA * d / (16 * dt_full)
 
 
 def _st(fields):
