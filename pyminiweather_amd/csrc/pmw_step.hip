@@ -96,69 +96,103 @@ __global__ void k_halo_z(double* __restrict__ s, Grid g,
 
 // --------------------------------------------------------- per function --
 
-__global__ void k_interp_x(const double* __restrict__ s, double* __restrict__ vals,
-                           double* __restrict__ d3, Grid g) {
-  const int nf = g.nx + 1;
-  const long long n = (long long)kNv * g.nz * nf;
-  const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= n) return;
-  const int i = (int)(idx % nf);
-  const int k = (int)((idx / nf) % g.nz);
-  const int v = (int)(idx / ((long long)nf * g.nz));
-  const double* r = s + g.at(v, k + kHs, i);
-  double a, b;
-  recon4(r[0], r[1], r[2], r[3], a, b);
-  vals[idx] = a;
-  d3[idx] = b;
-}
+// A thread's element (row k of `total`, column i of n), all four variables (or
+// blockIdx.y's): the lanes run through the rows laid end to end, so rows of any
+// width fill them. These kernels are bound by memory and, on small grids, by
+// the launch; a 64-bit flat index over the variables too took two divisions of
+// about 100 instructions per element, this one a 32-bit one per four. Rows
+// beyond 2^31 elements go to further blockIdx.z. The chain of both directions,
+// before / now: 800 x 400 58.5 / 53.7 us, 333 x 4111 195 / 186, 2000 x 1000 267
+// / 265. Rows from blockIdx and columns from the lanes instead: 333 x 4111 222
+// us (lanes past the row's end).
+struct Flat {
+  unsigned n;
+  int total, rows;
+  __device__ __forceinline__ bool at(int& k, int& i) const {
+    const unsigned idx = blockIdx.x * 256u + threadIdx.x;
+    const unsigned r = idx / n;
+    i = (int)(idx - r * n);
+    k = (int)blockIdx.z * rows + (int)r;
+    return (int)r < rows && k < total;
+  }
+};
 
-__global__ void k_interp_z(const double* __restrict__ s, double* __restrict__ vals,
-                           double* __restrict__ d3, Grid g) {
-  const int nfz = g.nz + 1;
-  const long long n = (long long)kNv * nfz * g.nx;
-  const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= n) return;
-  const int i = (int)(idx % g.nx);
-  const int k = (int)((idx / g.nx) % nfz);
-  const int v = (int)(idx / ((long long)g.nx * nfz));
-  const double* c = s + g.at(v, k, i + kHs);
-  double a, b;
-  recon4(c[0], c[g.ld], c[2 * g.ld], c[3 * g.ld], a, b);
-  vals[idx] = a;
-  d3[idx] = b;
-}
-
-__global__ void k_flux_x(const double* __restrict__ vals, const double* __restrict__ d3,
-                         const double* __restrict__ hyr, const double* __restrict__ hyt,
-                         double* __restrict__ flux, Grid g, double hv) {
-  const int nf = g.nx + 1;
-  const long long pv = (long long)g.nz * nf;          // plane of vals/d3
-  const long long pf = (long long)(g.nz + 1) * nf;    // plane of flux
-  const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= pv) return;
-  const int k = (int)(idx / nf);
-  double a[4], b[4], F[4];
+__global__ __launch_bounds__(256) void k_interp_x(const double* __restrict__ s,
+                                                  double* __restrict__ vals,
+                                                  double* __restrict__ d3, Grid g, Flat f) {
+  int k, i;
+  if (!f.at(k, i)) return;
+  const long long pv = (long long)g.nz * f.n, o = (long long)k * f.n + i;
+  const double* r = s + g.at(0, k + kHs, i);
+#pragma unroll
   for (int v = 0; v < kNv; ++v) {
-    a[v] = vals[v * pv + idx];
-    b[v] = d3[v * pv + idx];
+    const double* q = r + v * g.plane;
+    double a, b;
+    recon4(q[0], q[1], q[2], q[3], a, b);
+    vals[v * pv + o] = a;
+    d3[v * pv + o] = b;
+  }
+}
+
+// kInterpRows faces of a column per thread: kInterpRows + 3 loads instead of 4
+// per face. The chain at 800 x 400 / 333 x 4111 with 1, 2, 4, 8 faces: 57.0,
+// 54.7, 53.9, 53.7 / 197, 192, 190, 186 us.
+constexpr int kInterpRows = 8;
+
+__global__ __launch_bounds__(256) void k_interp_z(const double* __restrict__ s,
+                                                  double* __restrict__ vals,
+                                                  double* __restrict__ d3, Grid g, Flat f) {
+  int kg, i;
+  if (!f.at(kg, i)) return;
+  const int v = blockIdx.y, k0 = kg * kInterpRows, nfz = g.nz + 1;
+  const double* c = s + g.at(v, k0, i + kHs);
+  double q[kInterpRows + 3];
+#pragma unroll
+  for (int j = 0; j < kInterpRows + 3; ++j)
+    if (k0 + j < g.nz + 2 * kHs) q[j] = c[j * (long long)g.ld];
+  const long long o = ((long long)v * nfz + k0) * g.nx + i;
+#pragma unroll
+  for (int j = 0; j < kInterpRows; ++j) {
+    if (k0 + j >= nfz) break;
+    double a, b;
+    recon4(q[j], q[j + 1], q[j + 2], q[j + 3], a, b);
+    vals[o + j * (long long)g.nx] = a;
+    d3[o + j * (long long)g.nx] = b;
+  }
+}
+
+__global__ __launch_bounds__(256) void k_flux_x(
+    const double* __restrict__ vals, const double* __restrict__ d3,
+    const double* __restrict__ hyr, const double* __restrict__ hyt, double* __restrict__ flux,
+    Grid g, Flat f, double hv) {
+  int k, i;
+  if (!f.at(k, i)) return;
+  const long long pv = (long long)g.nz * f.n;          // plane of vals/d3
+  const long long pf = (long long)(g.nz + 1) * f.n;    // plane of flux
+  const long long o = (long long)k * f.n + i;
+  double a[4], b[4], F[4];
+#pragma unroll
+  for (int v = 0; v < kNv; ++v) {
+    a[v] = vals[v * pv + o];
+    b[v] = d3[v * pv + o];
   }
   flux_x_face(a, b, hyr[k + kHs], hyt[k + kHs], hv, F);
-  for (int v = 0; v < kNv; ++v) flux[v * pf + idx] = F[v];
+#pragma unroll
+  for (int v = 0; v < kNv; ++v) flux[v * pf + o] = F[v];
 }
 
-__global__ void k_flux_z(const double* __restrict__ vals, double* __restrict__ d3,
-                         const double* __restrict__ hyr, const double* __restrict__ hyt,
-                         const double* __restrict__ hyp, double* __restrict__ flux,
-                         Grid g, double hv) {
-  const int nfz = g.nz + 1;
-  const long long pv = (long long)nfz * g.nx;
+__global__ __launch_bounds__(256) void k_flux_z(
+    const double* __restrict__ vals, double* __restrict__ d3, const double* __restrict__ hyr,
+    const double* __restrict__ hyt, const double* __restrict__ hyp, double* __restrict__ flux,
+    Grid g, Flat f, double hv) {
+  int k, i;
+  if (!f.at(k, i)) return;
+  const long long pv = (long long)(g.nz + 1) * g.nx;
   const long long pf = (long long)(g.nz + 1) * (g.nx + 1);
-  const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= pv) return;
-  const int k = (int)(idx / g.nx);
-  const int i = (int)(idx % g.nx);
+  const long long idx = (long long)k * g.nx + i;
   const bool wall = (k == 0 || k == g.nz);
   double a[4], b[4], G[4];
+#pragma unroll
   for (int v = 0; v < kNv; ++v) {
     a[v] = vals[v * pv + idx];
     b[v] = d3[v * pv + idx];
@@ -166,38 +200,39 @@ __global__ void k_flux_z(const double* __restrict__ vals, double* __restrict__ d
   flux_z_face(a, b, hyr[k], hyt[k], hyp[k], hv, wall, G);
   if (wall) d3[idx] = 0.0;  // d3_vals_z[rho'] zeroed in place (interpolate.py:172-173)
   const long long o = (long long)k * (g.nx + 1) + i;
+#pragma unroll
   for (int v = 0; v < kNv; ++v) flux[v * pf + o] = G[v];
 }
 
-__global__ void k_tend_x(const double* __restrict__ flux, double* __restrict__ tend,
-                         Grid g, double id, double idl) {
+__global__ __launch_bounds__(256) void k_tend_x(const double* __restrict__ flux,
+                                                double* __restrict__ tend, Grid g, Flat f,
+                                                double id, double idl) {
+  int k, i;
+  if (!f.at(k, i)) return;
   const long long pt = (long long)g.nz * g.nx;
-  const long long n = kNv * pt;
-  const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= n) return;
-  const int i = (int)(idx % g.nx);
-  const int k = (int)((idx / g.nx) % g.nz);
-  const int v = (int)(idx / pt);
   const long long pf = (long long)(g.nz + 1) * (g.nx + 1);
-  const double* f = flux + v * pf + (long long)k * (g.nx + 1) + i;
-  tend[idx] = tend_of(f[0], f[1], id, idl);
+  const double* q = flux + (long long)k * (g.nx + 1) + i;
+  double* t = tend + (long long)k * g.nx + i;
+#pragma unroll
+  for (int v = 0; v < kNv; ++v) t[v * pt] = tend_of(q[v * pf], q[v * pf + 1], id, idl);
 }
 
-__global__ void k_tend_z(const double* __restrict__ flux, const double* __restrict__ sf,
-                         double* __restrict__ tend, Grid g, double id,
-                         double idl) {
+__global__ __launch_bounds__(256) void k_tend_z(const double* __restrict__ flux,
+                                                const double* __restrict__ sf,
+                                                double* __restrict__ tend, Grid g, Flat f,
+                                                double id, double idl) {
+  int k, i;
+  if (!f.at(k, i)) return;
   const long long pt = (long long)g.nz * g.nx;
-  const long long n = kNv * pt;
-  const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= n) return;
-  const int i = (int)(idx % g.nx);
-  const int k = (int)((idx / g.nx) % g.nz);
-  const int v = (int)(idx / pt);
   const long long pf = (long long)(g.nz + 1) * (g.nx + 1);
-  const double* f = flux + v * pf + (long long)k * (g.nx + 1) + i;
-  double t = tend_of(f[0], f[g.nx + 1], id, idl);
-  if (v == 2) t = t - sf[g.at(0, k + kHs, i + kHs)] * kGrav;
-  tend[idx] = t;
+  const double* q = flux + (long long)k * (g.nx + 1) + i;
+  double* o = tend + (long long)k * g.nx + i;
+#pragma unroll
+  for (int v = 0; v < kNv; ++v) {
+    double t = tend_of(q[v * pf], q[v * pf + g.nx + 1], id, idl);
+    if (v == 2) t = t - sf[g.at(0, k + kHs, i + kHs)] * kGrav;
+    o[v * pt] = t;
+  }
 }
 
 __global__ void k_add_w(double* __restrict__ tend, const double* __restrict__ src,
@@ -207,16 +242,19 @@ __global__ void k_add_w(double* __restrict__ tend, const double* __restrict__ sr
   tend[2 * n + idx] = tend[2 * n + idx] + src[idx];
 }
 
-__global__ void k_rk_update(const double* init, const double* __restrict__ tend,
-                            double* out, Grid g, double dt) {
+__global__ __launch_bounds__(256) void k_rk_update(const double* init,
+                                                   const double* __restrict__ tend, double* out,
+                                                   Grid g, Flat f, double dt) {
+  int k, i;
+  if (!f.at(k, i)) return;
   const long long pt = (long long)g.nz * g.nx;
-  const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= kNv * pt) return;
-  const int i = (int)(idx % g.nx);
-  const int k = (int)((idx / g.nx) % g.nz);
-  const int v = (int)(idx / pt);
-  const long long o = g.at(v, k + kHs, i + kHs);
-  out[o] = init[o] + dt * tend[idx];
+  const long long o = g.at(0, k + kHs, i + kHs);
+  const double* t = tend + (long long)k * g.nx + i;
+  double q[4];
+#pragma unroll
+  for (int v = 0; v < kNv; ++v) q[v] = init[o + v * g.plane] + dt * t[v * pt];
+#pragma unroll
+  for (int v = 0; v < kNv; ++v) out[o + v * g.plane] = q[v];
 }
 
 // ------------------------------------------------------------ fused x ----
@@ -392,6 +430,15 @@ __global__ __launch_bounds__(kZtCols* kZtRows) void k_stage_z(
   }
 }
 
+Flat flat_of(int n, int total) {
+  const int rows = (int)std::min<long long>(total, std::max(1LL, (1LL << 31) / n));
+  return Flat{(unsigned)n, total, rows};
+}
+dim3 flat_grid(const Flat& f, int vars = 1) {
+  return dim3((unsigned)(((long long)f.rows * f.n + 255) / 256), vars,
+              (f.total + f.rows - 1) / f.rows);
+}
+
 inline unsigned blocks_for(long long n, int per) { return (unsigned)((n + per - 1) / per); }
 
 bool grid_ok(int nx, int nz) {
@@ -482,8 +529,9 @@ int pmw_interpolate_x(const double* state, double* vals_x, double* d3_vals_x,
   if (!grid_ok(nx, nz) || bad_ptr(state) || bad_ptr(vals_x) || bad_ptr(d3_vals_x))
     return PMW_EINVAL;
   Grid g(nx, nz);
-  k_interp_x<<<blocks_for(4LL * nz * (nx + 1), 256), 256, 0, (hipStream_t)stream>>>(
-      state, vals_x, d3_vals_x, g);
+  const Flat f = flat_of(nx + 1, nz);
+  k_interp_x<<<flat_grid(f), 256, 0, (hipStream_t)stream>>>(
+      state, vals_x, d3_vals_x, g, f);
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
@@ -493,8 +541,9 @@ int pmw_interpolate_z(const double* state, double* vals_z, double* d3_vals_z,
   if (!grid_ok(nx, nz) || bad_ptr(state) || bad_ptr(vals_z) || bad_ptr(d3_vals_z))
     return PMW_EINVAL;
   Grid g(nx, nz);
-  k_interp_z<<<blocks_for(4LL * (nz + 1) * nx, 256), 256, 0, (hipStream_t)stream>>>(
-      state, vals_z, d3_vals_z, g);
+  const Flat f = flat_of(nx, (nz + kInterpRows) / kInterpRows);
+  k_interp_z<<<flat_grid(f, 4), 256, 0, (hipStream_t)stream>>>(
+      state, vals_z, d3_vals_z, g, f);
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
@@ -507,8 +556,9 @@ int pmw_compute_flux_x(const double* vals_x, const double* d3_vals_x,
       bad_ptr(hy_dens_cell) || bad_ptr(hy_dens_theta_cell) || bad_ptr(flux))
     return PMW_EINVAL;
   Grid g(nx, nz);
-  k_flux_x<<<blocks_for((long long)nz * (nx + 1), 256), 256, 0, (hipStream_t)stream>>>(
-      vals_x, d3_vals_x, hy_dens_cell, hy_dens_theta_cell, flux, g, hv_coeff);
+  const Flat f = flat_of(nx + 1, nz);
+  k_flux_x<<<flat_grid(f), 256, 0, (hipStream_t)stream>>>(
+      vals_x, d3_vals_x, hy_dens_cell, hy_dens_theta_cell, flux, g, f, hv_coeff);
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
@@ -523,8 +573,9 @@ int pmw_compute_flux_z(const double* vals_z, double* d3_vals_z,
       bad_ptr(hy_pressure_int) || bad_ptr(flux))
     return PMW_EINVAL;
   Grid g(nx, nz);
-  k_flux_z<<<blocks_for((long long)(nz + 1) * nx, 256), 256, 0, (hipStream_t)stream>>>(
-      vals_z, d3_vals_z, hy_dens_int, hy_dens_theta_int, hy_pressure_int, flux, g,
+  const Flat f = flat_of(nx, nz + 1);
+  k_flux_z<<<flat_grid(f), 256, 0, (hipStream_t)stream>>>(
+      vals_z, d3_vals_z, hy_dens_int, hy_dens_theta_int, hy_pressure_int, flux, g, f,
       hv_coeff);
   PMW_CHECK_LAUNCH();
   return PMW_OK;
@@ -535,8 +586,9 @@ int pmw_compute_tend_x(const double* flux, double* tend, int nx, int nz,
   if (!grid_ok(nx, nz) || bad_ptr(flux) || bad_ptr(tend)) return PMW_EINVAL;
   Grid g(nx, nz);
   const double id = 1.0 / dx;
-  k_tend_x<<<blocks_for(4LL * nz * nx, 256), 256, 0, (hipStream_t)stream>>>(
-      flux, tend, g, id, recip_lo(dx, id));
+  const Flat f = flat_of(nx, nz);
+  k_tend_x<<<flat_grid(f), 256, 0, (hipStream_t)stream>>>(
+      flux, tend, g, f, id, recip_lo(dx, id));
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
@@ -547,8 +599,9 @@ int pmw_compute_tend_z(const double* flux, const double* state_forcing,
     return PMW_EINVAL;
   Grid g(nx, nz);
   const double id = 1.0 / dz;
-  k_tend_z<<<blocks_for(4LL * nz * nx, 256), 256, 0, (hipStream_t)stream>>>(
-      flux, state_forcing, tend, g, id, recip_lo(dz, id));
+  const Flat f = flat_of(nx, nz);
+  k_tend_z<<<flat_grid(f), 256, 0, (hipStream_t)stream>>>(
+      flux, state_forcing, tend, g, f, id, recip_lo(dz, id));
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
@@ -568,8 +621,9 @@ int pmw_rk_update(const double* state_init, const double* tend,
   if (!grid_ok(nx, nz) || bad_ptr(state_init) || bad_ptr(tend) || bad_ptr(state_out))
     return PMW_EINVAL;
   Grid g(nx, nz);
-  k_rk_update<<<blocks_for(4LL * nz * nx, 256), 256, 0, (hipStream_t)stream>>>(
-      state_init, tend, state_out, g, dt_stage);
+  const Flat f = flat_of(nx, nz);
+  k_rk_update<<<flat_grid(f), 256, 0, (hipStream_t)stream>>>(
+      state_init, tend, state_out, g, f, dt_stage);
   PMW_CHECK_LAUNCH();
   return PMW_OK;
 }
