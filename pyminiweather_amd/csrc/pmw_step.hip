@@ -259,6 +259,8 @@ __global__ __launch_bounds__(256) void k_rk_update(const double* init,
 
 // ------------------------------------------------------------ fused x ----
 // MODE 0: full RK stage (writes out). MODE 1: tendency only (writes tend).
+// Bound by memory; every load is issued before the first wait: 2000 x 1000, the
+// stage from one buffer 25.4 -> 22.2 us, the tendency 22.0 -> 20.8.
 template <int MODE>
 __global__ __launch_bounds__(kXThreads) void k_stage_x(
     const double* init, double* forcing, double* out, double* __restrict__ tend,
@@ -273,6 +275,15 @@ __global__ __launch_bounds__(kXThreads) void k_stage_x(
   const int nx = g.nx;
   const int prow = k + kHs;
   const int c = i0 + t;                 // padded column loaded by this thread
+  const int i = i0 + t;                 // interior cell written by it
+  const bool own = t < kXCells && i < nx;
+  // every load is issued before the first is waited for
+  double S[4] = {0.0, 0.0, 0.0, 0.0};
+  if (MODE == 0 && own) {
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) S[v] = init[g.at(v, prow, i + kHs)];
+  }
+  const double hr = hyr[prow], ht = hyt[prow];
   if (c < nx + 4) {
     int src = c;
     bool halo = false;
@@ -290,9 +301,9 @@ __global__ __launch_bounds__(kXThreads) void k_stage_x(
     for (int v = 0; v < kNv; ++v) q[v] = forcing[g.at(v, prow, src)];
     if (halo) {
       if (bc == PMW_BC_INJECTION && inj_rows[k]) {
-        const double r = q[0] + hyr[prow];
+        const double r = q[0] + hr;
         q[1] = r * 50.0;
-        q[3] = r * 298.0 - hyt[prow];
+        q[3] = r * 298.0 - ht;
       }
 #pragma unroll
       for (int v = 0; v < kNv; ++v) forcing[g.at(v, prow, c)] = q[v];
@@ -306,13 +317,12 @@ __global__ __launch_bounds__(kXThreads) void k_stage_x(
 #pragma unroll
     for (int v = 0; v < kNv; ++v)
       recon4(sv[v][t], sv[v][t + 1], sv[v][t + 2], sv[v][t + 3], a[v], b[v]);
-    flux_x_face(a, b, hyr[prow], hyt[prow], hv, F);
+    flux_x_face(a, b, hr, ht, hv, F);
 #pragma unroll
     for (int v = 0; v < kNv; ++v) sf[v][t] = F[v];
   }
   __syncthreads();
-  const int i = i0 + t;
-  if (t < kXCells && i < nx) {
+  if (own) {
     double td[4];
 #pragma unroll
     for (int v = 0; v < kNv; ++v) td[v] = tend_of(sf[v][t], sf[v][t + 1], id, idl);
@@ -321,8 +331,7 @@ __global__ __launch_bounds__(kXThreads) void k_stage_x(
     if (MODE == 0) {
 #pragma unroll
       for (int v = 0; v < kNv; ++v) {
-        const long long o = g.at(v, prow, i + kHs);
-        out[o] = init[o] + dt * td[v];
+        out[g.at(v, prow, i + kHs)] = S[v] + dt * td[v];
       }
     } else {
       const long long pt = (long long)g.nz * nx;
@@ -392,6 +401,11 @@ __global__ __launch_bounds__(kZtCols* kZtRows) void k_stage_z(
   const int k = (tile / ncolgrp) * C - 2 + j;  // this slot's row, face and cell
   const bool colok = i < nx;
   const int pcol = i + kHs;
+  const bool own = colok && j >= 2 && j <= NR - 3 && k >= 0 && k < nz;
+  // the face's profiles are on their way before the first wait (init is not:
+  // its registers cost two waves per SIMD and 0.9 of 29.3 us at 2000 x 1000)
+  const int kf = min(max(k, 0), nz);
+  const double hr = hyr[kf], ht = hyt[kf], hp = hyp[kf];
   double q[4] = {0.0, 0.0, 0.0, 0.0};
   if (colok && k >= -2 && k <= nz + 1) load_z_row(forcing, g, hy_cell, k, pcol, q);
 #pragma unroll
@@ -403,13 +417,13 @@ __global__ __launch_bounds__(kZtCols* kZtRows) void k_stage_z(
 #pragma unroll
     for (int v = 0; v < kNv; ++v)
       recon4(s[v][t - 2 * CW], s[v][t - CW], s[v][t], s[v][t + CW], a[v], b[v]);
-    flux_z_face(a, b, hyr[k], hyt[k], hyp[k], hv, k == 0 || k == nz, G);
+    flux_z_face(a, b, hr, ht, hp, hv, k == 0 || k == nz, G);
 #pragma unroll
     for (int v = 0; v < kNv; ++v) fl[v][t] = G[v];
   }
   __syncthreads();
   // cell k from faces k and k+1 (tile rows 2..NR-3: the C output rows)
-  if (colok && j >= 2 && j <= NR - 3 && k >= 0 && k < nz) {
+  if (own) {
     double td[4];
 #pragma unroll
     for (int v = 0; v < kNv; ++v) td[v] = tend_of(fl[v][t], fl[v][t + CW], id, idl);
