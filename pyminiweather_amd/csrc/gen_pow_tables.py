@@ -10,13 +10,17 @@ decimal module at 60 digits and rounded to doubles.
   4th entry, 2^(j/64)).
 * gamma: for j = 0..511, c_j = 1/(1 + (j + 1/2)/512) rounded to 10 bits, so
   that r = m*c_j - 1 is exact in one fma for m in [1 + j/512, 1 + (j+1)/512)
-  (|r| <= 2^-9), c_j^-gamma as a double-double and c_j^(1-gamma); and for
-  every biased exponent e of a double 2^((e-1023) gamma) as a double-double
-  (up to the largest whose power stays finite, then one NaN) and
-  2^((e-1023) (gamma-1)).
+  (|r| <= 2^-9); for the four binades from 2^6, entry 512 o + j: the power
+  (2^(6+o) / c_j)^gamma as a double and a float of its rest, and c_j as a float
+  (kGamQ); and for other binades, whose significands use the entries of binade
+  6 + (e-6) mod 4, 2^(4 (i-258) gamma) for i = 1.. as a double-double (0 for
+  i = 0, times 2^64 for i < 100, up to the largest that is finite, then one NaN).
+* gamma - 1: c_j^(1-gamma) and c_j (kGamM), and for every biased exponent e of
+  a double 2^((e-1023) (gamma-1)) (kGamD).
   gamma is the double nearest to the physical constant.
 """
 import math
+import struct
 from decimal import Decimal, getcontext
 
 getcontext().prec = 60
@@ -30,6 +34,10 @@ def rn(d):
 def dd(d):
     h = rn(d)
     return h, rn(d - Decimal(h))
+
+
+def f32(d):
+    return struct.unpack("f", struct.pack("f", float(d)))[0]  # rounds to nearest
 
 
 def round_bits(d, bits):
@@ -53,20 +61,27 @@ def main():
         th.append(h); tl.append(l)
 
     gamma = Decimal(GAMMA)
-    gm = []  # c, hi and lo of c^-gamma, c^(1-gamma)
-    for j in range(512):
+    ln2 = Decimal(2).ln()
+    gq, gm = [], []
+    for i in range(2048):
+        o, j = divmod(i, 512)
         c = round_bits(1 / (1 + (Decimal(j) + Decimal("0.5")) / 512), 10)
         for m in (1 + Decimal(j) / 512, 1 + Decimal(j + 1) / 512):
             assert abs(m * c - 1) <= Decimal(2) ** -9
-        lc = c.ln()
-        gm += [rn(c), *dd((-gamma * lc).exp()), rn(((1 - gamma) * lc).exp())]
-    ln2 = Decimal(2).ln()
+        lx = (6 + o) * ln2 - c.ln()
+        h, l = dd((gamma * lx).exp())
+        gq.append((h, f32(l), f32(c)))
+        assert Decimal(f32(c)) == c
+        if o == 0:
+            gm += [rn(((1 - gamma) * c.ln()).exp()), rn(c)]
     ge, gd = [], []
+    for i in range(513):
+        k = 4 * (i - 258)
+        if k * gamma < 1024:
+            lift = 64 * ln2 if i < 100 else 0  # clear of subnormal factors
+            ge += dd((k * gamma * ln2 + lift).exp()) if i else (0.0, 0.0)
     for e in range(2048):
-        k = e - 1023
-        if e <= 1023 + 731:  # 2^(731 gamma) is the last below 2^1024
-            ge += dd((k * gamma * ln2).exp()) if e else (0.0, 0.0)
-        gd.append(rn((k * (gamma - 1) * ln2).exp()))
+        gd.append(rn(((e - 1023) * (gamma - 1) * ln2).exp()))
 
     last = len(ge) // 2
     ge += (math.nan, math.nan)
@@ -86,7 +101,11 @@ def main():
     arr("kLogLo", ll)
     arr("kExpHi", th)
     arr("kExpLo", tl)
-    arr("kGamC", gm, align=True)
+    out.append("struct alignas(16) GamQ {\n  double h;\n  float l, c;\n};")
+    out.append(f"constexpr GamQ kGamQ[{len(gq)}] = {{")
+    out.extend("    {%s, %sf, %sf}," % tuple(float.hex(v) for v in q) for q in gq)
+    out.append("};")
+    arr("kGamM", gm, align=True)
     arr("kGamE", ge, align=True)
     arr("kGamD", gd, align=True)
     out.append(f"constexpr unsigned kGamELast = {last};")

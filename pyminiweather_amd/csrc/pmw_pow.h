@@ -299,23 +299,29 @@ PMW_HD double significand(double x) {
 
 // x^gamma for gamma = kGamma's double (pmw_common.h), the exponent of the
 // tables. x = 2^(e-1023) m; j = m's first 9 fraction bits; r = m c_j - 1,
-// exact; x^gamma = 2^((e-1023) gamma) c_j^-gamma (1 + r)^gamma. The linear
-// term of the series and both table factors are double-double; the quadratic
-// and later terms (< 2^-19.8) are doubles, whose rounding sets the error of
-// the value before the last rounding: host maximum 3.7e-22 relative against
-// 113-bit quadmath (pow_pos: 4.5e-22), so all but ~1e-6 of results are the
-// correctly rounded ones. Powers that overflow give inf; other arguments as
-// pow(x, gamma): +-0 -> 0, +-inf -> inf, negative and NaN -> NaN; subnormal
-// arguments, whose power is below the smallest double, give 0.
+// exact; x^gamma = (2^(e-1023) / c_j)^gamma (1 + r)^gamma. For 64 <= x < 1024
+// (rho*theta of any atmosphere) one 16-byte table entry holds c_j and the first
+// factor as a double and a float; elsewhere the entry of the binade 6 + (e-6)
+// mod 4 is scaled by a second, double-double factor. The linear term of the
+// series is double-double; the quadratic and later terms (< 2^-19.8) are
+// doubles, whose rounding sets the error of the value before the last
+// rounding: all but ~1e-6 of results are the correctly rounded ones. Powers
+// that overflow give inf; other arguments as pow(x, gamma): +-0 -> 0, +-inf ->
+// inf, negative and NaN -> NaN; subnormal arguments, whose power is below the
+// smallest double, give 0.
+//
+// The entry is a gather, and the flux kernels pay for its bytes. Three loads of
+// 40 bytes a lane (c_j and double-doubles of c_j^-gamma and of every binade's
+// factor) / this one of 16: a step of 2000 x 1000 84.5 / 82.7 us, of 8192 x
+// 4096 1315 / 1277, of 1003 x 517 33.8 / 33.0. With uniform loads (a timing
+// copy, wrong values) 2000 x 1000 takes 75.1.
 PMW_HD double pow_gamma(double x) {
   using namespace powt;
   const unsigned hi = high_word(x);
-  const double* t = kGamC + 4u * ((hi >> 11) & 511u);
-  // the last entry (NaN) serves x >= 2^732, NaN and a set sign
-  const unsigned e = hi >> 20;
-  const double* te = kGamE + 2u * (e < kGamELast ? e : kGamELast);
-  const double c = t[0], th = t[1], tl = t[2], eh = te[0], el = te[1];
-  const double r = fma(significand(x), c, -1.0);     // exact
+  const unsigned k = (hi >> 11) - (1029u << 9);      // < 2048: 64 <= x < 1024
+  const GamQ t = kGamQ[k & 2047u];
+  const double r = fma(significand(x), (double)t.c, -1.0);  // exact
+  const double th = t.h, tl = t.l;
   // c_k = gamma (gamma-1) ... (gamma-k+1) / k!, k = 7..2; c_8 r^8 < 2^-80
   double q = fma_c(-0x1.2cfc9a75b3dd8p-8, r, 0x1.ca0d127e7ec8ep-8);
   q = fma_c(q, r, -0x1.7dbd21dc9384dp-7);
@@ -329,25 +335,31 @@ PMW_HD double pow_gamma(double x) {
   const double a = th * ph;
   const double s = th + a;                           // Fast2Sum: th > |a|
   const double l = (((th - s) + a) + fma(th, ph, -a)) + fma(th, pl, fma(tl, ph, tl));
-  // (s + l)(eh + el)
-  const double h = s * eh;
-  const double res = h + fma(l, eh, fma(s, el, fma(s, eh, -h)));
-  const double inf = __builtin_inf();
-  if (__builtin_expect(!(res < inf), 0)) {
+  if (__builtin_expect(k >= 2048u, 0)) {
+    // the last entry (NaN) serves powers past the largest, NaN and a set sign
+    const unsigned e = ((hi >> 20) + 3u) >> 2;
+    const double* te = kGamE + 2u * (e < kGamELast ? e : kGamELast);
+    const double eh = te[0], el = te[1];
+    const double h = s * eh;                         // (s + l)(eh + el)
+    const double up = h + fma(l, eh, fma(s, el, fma(s, eh, -h)));
+    const double res = e < 100u ? up * 0x1p-64 : up;  // as the table's entries
+    const double inf = __builtin_inf();
+    if (res < inf) return res;
     return x == 0.0 ? 0.0 : (x > 0.0 || x == -inf) ? inf : __builtin_nan("");
   }
-  return res;
+  return s + l;
 }
 
-// x^(gamma-1) to 4e-16 relative for positive normal x, from the same tables in
+// x^(gamma-1) to 4e-16 relative for positive normal x, by the same steps in
 // plain double arithmetic: for the adjoint's dp/dq = gamma C0 q^(gamma-1),
-// where a derivative needs no last bit. Other x give NaN. 18 VALU
-// instructions and 3 loads (pow_pos_fast: 45 and two dependent rounds).
+// where a derivative needs no last bit. Other x give NaN. Two loads and no
+// branch: with one entry per binade and the rare path in a branch the adjoint
+// kernels, at their register limits, spill (16 of 400 x 200 112 -> 166 us).
 PMW_HD double pow_gamma_minus_one(double x) {
   using namespace powt;
   const unsigned hi = high_word(x);
-  const double* t = kGamC + 4u * ((hi >> 11) & 511u);
-  const double c = t[0], d = t[3], e = kGamD[(hi >> 20) & 2047u];
+  const double* t = kGamM + 2u * ((hi >> 11) & 511u);
+  const double d = t[0], c = t[1], e = kGamD[(hi >> 20) & 2047u];
   const double r = fma(significand(x), c, -1.0);  // exact, |r| <= 2^-9
   // c_k = a (a-1) ... (a-k+1) / k!, a = gamma - 1; c_6 r^6 < 2^-60
   double q = fma_c(0x1.eaabd5fa7fe8cp-6, r, -0x1.54c5337464d59p-5);
