@@ -562,6 +562,120 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   dir_zt1_tile<NW, NR>(a, g, logical / ncol, ntile, (logical % ncol) * kZtCols, sm, logical == 0);
 }
 
+// ---- z, one column per wave (k_dir_zw), for grids whose column waves are at
+// most one per SIMD: lane = row, the x waves turned by 90 degrees. Neighbouring
+// rows come by one-lane shifts; no LDS, no barrier, no flag. A lane's loads and
+// stores touch a cache line each (the block's other column and its neighbours
+// on the XCD share them): such a launch waits for latency, not for bandwidth.
+// Tiles of a column: the first holds rows -2 .. 61, the last rows nz-62 ..
+// nz+1, those between start 6 rows before the first row they own. A column of
+// up to 60 rows is one wave. Step in us with one-cell tiles of 32 rows / this:
+// 37x5 11.8 / 9.9, 100x50 11.9 / 10.3, 200x100 12.3 / 11.2, 300x150 (900 waves)
+// 12.4 / 12.0, 1000x60 13.7 / 13.1; beyond, 350x175 (1400) 13.5 / 13.9, 400x200
+// 13.8 / 14.6. Blocks of 1, 2, 4, 8, 16 columns at 200x100: 11.2, 11.2, 11.4,
+// 12.0, 14.8.
+constexpr int kZwWaves = 2;  // columns per block (the waves share nothing)
+constexpr long long kZwMaxWaves = 1024;  // one per SIMD
+
+__host__ __device__ inline int zw_tiles(int nz) {
+  return nz <= 60 ? 1 : nz <= 112 ? 2 : 2 + (nz - 112 + 51) / 52;
+}
+
+__device__ __forceinline__ void dir_z_wave(const DirArgs& a, const Grid& g, int tile, int ntile,
+                                           int c, bool corners) {
+  const int nx = g.nx, nz = g.nz, lane = threadIdx.x & 63;
+  if (c >= nx) return;
+  const bool first = tile == 0, last = tile == ntile - 1;
+  const int base = first ? -2 : last ? nz - 62 : 50 + (tile - 1) * 52;
+  const int own0 = first ? 0 : last ? nz - 56 : base + 6;
+  const int own1 = last ? nz : min(first ? 56 : base + 58, nz - 56);
+  const int k = base + lane;
+  const gdouble* hy = a.hy_cell;
+  const int plo = kHs, phi = nz + kHs - 1;
+  const bool own = k >= own0 && k < own1;
+  const int kc = min(max(k, 0), nz - 1), kf = min(max(k, 0), nz);
+  const long long at = (long long)(kc + kHs) * g.ld + c + kHs;  // clamped row
+  // every load is issued before the first is waited for
+  double S[4], s[4];
+#pragma unroll
+  for (int v = 0; v < kNv; ++v) S[v] = a.in[v * g.plane + at];
+  const double hyr = a.hyr_int[kf], hyt = a.hyt_int[kf], hyp = a.hyp_int[kf];
+  const bool low = k == -2 || k == -1, high = k == nz || k == nz + 1;
+  const bool wall = low || high;
+  const double hye = hy[low ? plo : phi], hyh = hy[wall ? k + kHs : phi];
+  const double src = a.src_w ? a.src_w[(long long)kc * nx + c] : 0.0;
+  if (corners && threadIdx.x < 8) {
+    // corner columns (padded 0, 1, nx+2, nx+3) of the halo rows of st, tmp
+    const int t = threadIdx.x;
+    gdouble* buf = t < 4 ? a.st : a.tmp;
+    const int qq = t & 3;
+    const int cc = qq < 2 ? qq : nx + qq;
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) {
+      const double e = buf[g.at(v, plo, cc)];
+      buf[g.at(v, 0, cc)] = wall_halo(v, e, hy[plo], hy[0]);
+      buf[g.at(v, 1, cc)] = wall_halo(v, e, hy[plo], hy[1]);
+      const double f = buf[g.at(v, phi, cc)];
+      buf[g.at(v, nz + 2, cc)] = wall_halo(v, f, hy[phi], hy[nz + 2]);
+      buf[g.at(v, nz + 3, cc)] = wall_halo(v, f, hy[phi], hy[nz + 3]);
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < kNv; ++v) s[v] = S[v];
+#pragma unroll
+  for (int stage = 0; stage < 3; ++stage) {
+    const double dts = stage == 0 ? a.dt1 : stage == 1 ? a.dt2 : a.dt3;
+    if (base < 0 || base + 63 >= nz) {  // wall halo rows, stored by set_bc_z of stages 1 and 3
+      gdouble* const halo = stage == 0 ? a.st : a.tmp;
+#pragma unroll
+      for (int v = 0; v < kNv; ++v) {
+        double e;
+        if (stage == 0) {
+          e = s[v];  // loaded from the edge row
+        } else {
+          const double n1 = from_next(s[v]), p1 = from_prev(s[v]);
+          const double n2 = from_next(n1), p2 = from_prev(p1);
+          e = low ? (k == -1 ? n1 : n2) : (k == nz ? p1 : p2);
+        }
+        if (wall) {
+          s[v] = wall_halo(v, e, hye, hyh);
+          if (stage != 1 && (low ? first : last))
+            halo[v * g.plane + (long long)(k + kHs) * g.ld + c + kHs] = s[v];
+        }
+      }
+    }
+    double v4[4], d3[4], F[4];
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) {
+      const double b1 = from_prev(s[v]);
+      recon4(from_prev(b1), b1, s[v], from_next(s[v]), v4[v], d3[v]);
+    }
+    flux_z_face(v4, d3, hyr, hyt, hyp, a.hv, k == 0 || k == nz, F);
+    double td[4];
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) td[v] = tend_of(F[v], from_next(F[v]), a.id, a.idl);
+    td[2] = td[2] - s[0] * kGrav;
+    if (a.src_w) td[2] = td[2] + src;
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) s[v] = S[v] + dts * td[v];
+    gdouble* const dst = stage == 0 ? a.s1 : stage == 1 ? (a.tmp_interior ? a.tmp : nullptr) : a.out;
+    if (dst && own) {
+#pragma unroll
+      for (int v = 0; v < kNv; ++v) dst[v * g.plane + at] = s[v];
+    }
+  }
+}
+
+__global__ __launch_bounds__(64 * kZwWaves) void k_dir_zw(DirArgs a, Grid g, int ncol, int ntile,
+                                                          int per_xcd) {
+  const int logical = xcd_logical(blockIdx.x, per_xcd);
+  if (logical >= ncol * ntile) return;
+  member_offset(a);
+  dir_z_wave(a, g, logical / ncol, ntile,
+             (logical % ncol) * kZwWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6),
+             logical == 0);
+}
+
 // ---- z, one cell per thread, for small grids and low columns.
 // A block holds 8 columns x NR rows (slot t = row*8 + col, tile row j =
 // logical row r0-6+j; NR-12 rows are written), the RK init in registers and
@@ -1008,6 +1122,14 @@ int launch_zt1(const DirArgs& a, Grid g, hipStream_t st, int members) {
   return PMW_OK;
 }
 
+int launch_zw(const DirArgs& a, Grid g, hipStream_t st, int members) {
+  const int ncol = (g.nx + kZwWaves - 1) / kZwWaves, ntile = zw_tiles(g.nz);
+  const int per = (ncol * ntile + kNumXcd - 1) / kNumXcd;
+  k_dir_zw<<<dim3(per * kNumXcd, members), 64 * kZwWaves, 0, st>>>(a, g, ncol, ntile, per);
+  PMW_CHECK_LAUNCH();
+  return PMW_OK;
+}
+
 template <int NR>
 int launch_z1(const DirArgs& a, Grid g, hipStream_t st, int members) {
   constexpr int C = NR - 12;
@@ -1113,7 +1235,11 @@ int launch_dir_z(const DirArgs& a, Grid g, int seg, hipStream_t st, int members)
                  ? launch_zt1<4>(a, g, st, members)
                  : launch_zt1<8>(a, g, st, members);
     case Z_ONE96: return launch_z1<96>(a, g, st, members);
-    case Z_ONE32: return launch_z1<32>(a, g, st, members);
+    case Z_ONE32:
+      // the codes that do not force a kernel: columns as waves if they fit
+      if (seg > 64 && (long long)g.nx * zw_tiles(g.nz) * members <= kZwMaxWaves)
+        return launch_zw(a, g, st, members);
+      return launch_z1<32>(a, g, st, members);
     default:
       if (dense_z_rows(g.nx, g.nz, kZ1Cols) > (1LL << 30)) return PMW_EINVAL;
       return launch_z1d<96>(a, g, st, members);

@@ -1,4 +1,4 @@
-"""The three-row z tiles against the per-stage kernels, bit for bit."""
+"""The z tiles and column waves against the per-stage kernels, bit for bit."""
 import ctypes
 
 import numpy as np
@@ -51,6 +51,26 @@ def test_three_row_tiles_bitwise_equal_per_stage(nx, nz, ic):
                                                device="cuda", generator=g)
     want = _run(p, start, (1, 256, 8096), 2)
     got = _run(p, start, (0, 512, 8096), 2)
+    assert all(np.all(np.isfinite(w)) for w in want)
+    np.testing.assert_array_equal(got[0], want[0])
+    np.testing.assert_array_equal(got[1], want[1])
+
+
+# one wave per column up to 60 rows, two to 112, then one more every 52; 1024
+# columns of 60 rows are the most waves taken, 1025 one too many
+@pytest.mark.parametrize("nx,nz", [(17, nz) for nz in (2, 3, 4, 57, 58, 59, 60, 61, 62, 63, 111,
+                                                       112, 113, 164, 165, 217)] +
+                         [(2, 9), (3, 70), (1024, 60), (1025, 60)])
+@pytest.mark.parametrize("ic", ["collision", "gravity"])
+def test_column_waves_bitwise_equal_per_stage(nx, nz, ic):
+    """Three steps from random states with nonzero halos, as above."""
+    p = O.make_params(nx, nz, ic, cfl=1.0, max_speed=450.0)
+    g = torch.Generator(device="cuda").manual_seed(nx * 1000 + nz)
+    scale = torch.tensor([1e-3, 2.0, 2.0, 0.5], dtype=torch.float64, device="cuda")
+    start = scale[:, None, None] * torch.randn((4, nz + 4, nx + 4), dtype=torch.float64,
+                                               device="cuda", generator=g)
+    want = _run(p, start, (1, 256, 8096), 3)
+    got = _run(p, start, (0, 512, 8096), 3)
     assert all(np.all(np.isfinite(w)) for w in want)
     np.testing.assert_array_equal(got[0], want[0])
     np.testing.assert_array_equal(got[1], want[1])
