@@ -562,29 +562,43 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   dir_zt1_tile<NW, NR>(a, g, logical / ncol, ntile, (logical % ncol) * kZtCols, sm, logical == 0);
 }
 
-// ---- z, one column per wave (k_dir_zw), for grids whose column waves are at
-// most one per SIMD: lane = row, the x waves turned by 90 degrees. Neighbouring
-// rows come by one-lane shifts; no LDS, no barrier, no flag. A lane's loads and
-// stores touch a cache line each (the block's other column and its neighbours
-// on the XCD share them): such a launch waits for latency, not for bandwidth.
+// ---- z, one column per wave, for small grids: lane = row, the x waves turned
+// by 90 degrees. Neighbouring rows come by one-lane shifts, no flags, no LDS
+// between the stages: such a launch waits for latency, not for bandwidth.
 // Tiles of a column: the first holds rows -2 .. 61, the last rows nz-62 ..
 // nz+1, those between start 6 rows before the first row they own. A column of
-// up to 60 rows is one wave. Step in us with one-cell tiles of 32 rows / this:
-// 37x5 11.8 / 9.9, 100x50 11.9 / 10.3, 200x100 12.3 / 11.2, 300x150 (900 waves)
-// 12.4 / 12.0, 1000x60 13.7 / 13.1; beyond, 350x175 (1400) 13.5 / 13.9, 400x200
-// 13.8 / 14.6. Blocks of 1, 2, 4, 8, 16 columns at 200x100: 11.2, 11.2, 11.4,
-// 12.0, 14.8.
-constexpr int kZwWaves = 2;  // columns per block (the waves share nothing)
-constexpr long long kZwMaxWaves = 1024;  // one per SIMD
+// up to 60 rows is one wave.
+// k_dir_zw, up to 512 waves: blocks of two columns that share nothing; a lane's
+// loads and stores touch a cache line each. k_dir_zs, up to 4096 (four per
+// SIMD): blocks of four columns whose loads and stores pass through LDS, rows
+// of 32 bytes. Step in us with one-cell tiles of 32 rows / k_dir_zw / k_dir_zs:
+// 37x5 11.8 / 9.9 / -, 100x50 12.0 / 10.4 / 10.8, 200x100 (400 waves) 12.3 /
+// 10.9 / 11.4, 333x61 (666) 12.3 / 11.3 / 11.1, 300x150 (900) 12.4 / 11.8 /
+// 11.3, 1000x60 13.7 / 13.1 / 12.5, 400x200 (1600) 13.7 / 14.6 / 13.0, 500x250
+// 15.9 / - / 15.0, 600x300 (3600) 17.9 / - / 17.5, 4000x70 (8000) 27.3 / - /
+// 30.0. Columns per block, k_dir_zw at 200x100 with 1, 2, 4, 8, 16: 11.2, 11.2,
+// 11.4, 12.0, 14.8; k_dir_zs at 400x200 with 4, 8, 16: 13.0, 13.7, 15.7.
+constexpr int kZwWaves = 2, kZsWaves = 4;  // columns per block
+constexpr long long kZwMaxWaves = 512, kZsMaxWaves = 4096;
 
 __host__ __device__ inline int zw_tiles(int nz) {
   return nz <= 60 ? 1 : nz <= 112 ? 2 : 2 + (nz - 112 + 51) / 52;
 }
 
+template <int NC>
+struct ZwLds {
+  double b[2][kNv][64][NC + 1];
+};
+
+// STAGED: the block's NC columns pass through LDS, so that loads and stores
+// are rows of 8 NC bytes.
+template <int NC, bool STAGED>
 __device__ __forceinline__ void dir_z_wave(const DirArgs& a, const Grid& g, int tile, int ntile,
-                                           int c, bool corners) {
+                                           int c0, int w, ZwLds<NC>* sm, bool corners) {
   const int nx = g.nx, nz = g.nz, lane = threadIdx.x & 63;
-  if (c >= nx) return;
+  const bool colok = c0 + w < nx;  // wave-uniform
+  if (!STAGED && !colok) return;
+  const int c = colok ? c0 + w : nx - 1;
   const bool first = tile == 0, last = tile == ntile - 1;
   const int base = first ? -2 : last ? nz - 62 : 50 + (tile - 1) * 52;
   const int own0 = first ? 0 : last ? nz - 56 : base + 6;
@@ -597,8 +611,21 @@ __device__ __forceinline__ void dir_z_wave(const DirArgs& a, const Grid& g, int 
   const long long at = (long long)(kc + kHs) * g.ld + c + kHs;  // clamped row
   // every load is issued before the first is waited for
   double S[4], s[4];
+  // STAGED: this thread's row and column of the block's loads and stores
+  const int ri = threadIdx.x / NC, ci = threadIdx.x % NC, kr = base + ri;
+  const long long rat = (long long)(min(max(kr, 0), nz - 1) + kHs) * g.ld + min(c0 + ci, nx - 1) + kHs;
+  const bool rown = kr >= own0 && kr < own1 && c0 + ci < nx;
+  int buf = 0;
+  if constexpr (STAGED) {
+    double q[4];
 #pragma unroll
-  for (int v = 0; v < kNv; ++v) S[v] = a.in[v * g.plane + at];
+    for (int v = 0; v < kNv; ++v) q[v] = a.in[v * g.plane + rat];
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) sm->b[0][v][ri][ci] = q[v];
+  } else {
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) S[v] = a.in[v * g.plane + at];
+  }
   const double hyr = a.hyr_int[kf], hyt = a.hyt_int[kf], hyp = a.hyp_int[kf];
   const bool low = k == -2 || k == -1, high = k == nz || k == nz + 1;
   const bool wall = low || high;
@@ -620,6 +647,11 @@ __device__ __forceinline__ void dir_z_wave(const DirArgs& a, const Grid& g, int 
       buf[g.at(v, nz + 3, cc)] = wall_halo(v, f, hy[phi], hy[nz + 3]);
     }
   }
+  if constexpr (STAGED) {
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < kNv; ++v) S[v] = sm->b[0][v][lane][w];
+  }
 #pragma unroll
   for (int v = 0; v < kNv; ++v) s[v] = S[v];
 #pragma unroll
@@ -639,7 +671,7 @@ __device__ __forceinline__ void dir_z_wave(const DirArgs& a, const Grid& g, int 
         }
         if (wall) {
           s[v] = wall_halo(v, e, hye, hyh);
-          if (stage != 1 && (low ? first : last))
+          if (stage != 1 && colok && (low ? first : last))
             halo[v * g.plane + (long long)(k + kHs) * g.ld + c + kHs] = s[v];
         }
       }
@@ -659,7 +691,21 @@ __device__ __forceinline__ void dir_z_wave(const DirArgs& a, const Grid& g, int 
 #pragma unroll
     for (int v = 0; v < kNv; ++v) s[v] = S[v] + dts * td[v];
     gdouble* const dst = stage == 0 ? a.s1 : stage == 1 ? (a.tmp_interior ? a.tmp : nullptr) : a.out;
-    if (dst && own) {
+    if constexpr (STAGED) {
+      if (dst) {  // the same for the whole block
+        // Two buffers in turn: when a wave writes a buffer again it has passed
+        // the barrier of the store between, and with it every wave its reads.
+        auto& b = sm->b[buf];
+        buf ^= 1;
+#pragma unroll
+        for (int v = 0; v < kNv; ++v) b[v][lane][w] = s[v];
+        __syncthreads();
+        if (rown) {
+#pragma unroll
+          for (int v = 0; v < kNv; ++v) dst[v * g.plane + rat] = b[v][ri][ci];
+        }
+      }
+    } else if (dst && own) {
 #pragma unroll
       for (int v = 0; v < kNv; ++v) dst[v * g.plane + at] = s[v];
     }
@@ -671,9 +717,19 @@ __global__ __launch_bounds__(64 * kZwWaves) void k_dir_zw(DirArgs a, Grid g, int
   const int logical = xcd_logical(blockIdx.x, per_xcd);
   if (logical >= ncol * ntile) return;
   member_offset(a);
-  dir_z_wave(a, g, logical / ncol, ntile,
-             (logical % ncol) * kZwWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6),
-             logical == 0);
+  dir_z_wave<kZwWaves, false>(a, g, logical / ncol, ntile, (logical % ncol) * kZwWaves,
+                              __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nullptr,
+                              logical == 0);
+}
+
+__global__ __launch_bounds__(64 * kZsWaves) void k_dir_zs(DirArgs a, Grid g, int ncol, int ntile,
+                                                          int per_xcd) {
+  __shared__ ZwLds<kZsWaves> sm;
+  const int logical = xcd_logical(blockIdx.x, per_xcd);
+  if (logical >= ncol * ntile) return;  // whole block, before any barrier
+  member_offset(a);
+  dir_z_wave<kZsWaves, true>(a, g, logical / ncol, ntile, (logical % ncol) * kZsWaves,
+                             __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), &sm, logical == 0);
 }
 
 // ---- z, one cell per thread, for small grids and low columns.
@@ -1112,6 +1168,14 @@ __global__ __launch_bounds__(kZ1Cols * NR) __attribute__((amdgpu_waves_per_eu(6)
   dir_z1d_tile<NR>(a, Grid(md.nx, md.nz), local, sm, local == 0);
 }
 
+int launch_zs(const DirArgs& a, Grid g, hipStream_t st, int members) {
+  const int ncol = (g.nx + kZsWaves - 1) / kZsWaves, ntile = zw_tiles(g.nz);
+  const int per = (ncol * ntile + kNumXcd - 1) / kNumXcd;
+  k_dir_zs<<<dim3(per * kNumXcd, members), 64 * kZsWaves, 0, st>>>(a, g, ncol, ntile, per);
+  PMW_CHECK_LAUNCH();
+  return PMW_OK;
+}
+
 template <int NW>
 int launch_zt1(const DirArgs& a, Grid g, hipStream_t st, int members) {
   constexpr int NR = 12 * NW;
@@ -1236,9 +1300,11 @@ int launch_dir_z(const DirArgs& a, Grid g, int seg, hipStream_t st, int members)
                  : launch_zt1<8>(a, g, st, members);
     case Z_ONE96: return launch_z1<96>(a, g, st, members);
     case Z_ONE32:
-      // the codes that do not force a kernel: columns as waves if they fit
-      if (seg > 64 && (long long)g.nx * zw_tiles(g.nz) * members <= kZwMaxWaves)
-        return launch_zw(a, g, st, members);
+      if (seg > 64) {  // no code that forces a kernel: columns as waves if they fit
+        const long long waves = (long long)g.nx * zw_tiles(g.nz) * members;
+        if (waves <= kZwMaxWaves) return launch_zw(a, g, st, members);
+        if (waves <= kZsMaxWaves) return launch_zs(a, g, st, members);
+      }
       return launch_z1<32>(a, g, st, members);
     default:
       if (dense_z_rows(g.nx, g.nz, kZ1Cols) > (1LL << 30)) return PMW_EINVAL;

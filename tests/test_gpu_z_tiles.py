@@ -56,11 +56,13 @@ def test_three_row_tiles_bitwise_equal_per_stage(nx, nz, ic):
     np.testing.assert_array_equal(got[1], want[1])
 
 
-# one wave per column up to 60 rows, two to 112, then one more every 52; 1024
-# columns of 60 rows are the most waves taken, 1025 one too many
+# one wave per column up to 60 rows, two to 112, then one more every 52; up to
+# 512 waves share nothing, up to 4096 pass their columns through LDS four by
+# four (the last group ragged), 4097 are one too many
 @pytest.mark.parametrize("nx,nz", [(17, nz) for nz in (2, 3, 4, 57, 58, 59, 60, 61, 62, 63, 111,
                                                        112, 113, 164, 165, 217)] +
-                         [(2, 9), (3, 70), (1024, 60), (1025, 60)])
+                         [(2, 9), (3, 70), (512, 60), (513, 60), (307, 61), (515, 113), (271, 217),
+                          (4096, 60), (4097, 60)])
 @pytest.mark.parametrize("ic", ["collision", "gravity"])
 def test_column_waves_bitwise_equal_per_stage(nx, nz, ic):
     """Three steps from random states with nonzero halos, as above."""
