@@ -187,12 +187,12 @@ int pmw_evolve(double* state, double* state_tmp, double* state_work,
  *       its 6 periodic cells per side) with one (256) or two (1512) cells
  *       per lane; 448, 512 and 1256 choose between them by the size of the
  *       grid (or of all members);
- *   [2] fused z kernel: LDS tiles. 18096 and 18128 = one cell per thread, 8
+ *   [2] fused z kernel: 18096 and 18128 = one cell per thread, 8
  *       columns x 96 rows over the column groups laid end to end; 8, 16, 24,
  *       32, 48 and 64 = one cell per thread, 8 columns x 32 rows; 8064, 8096,
  *       8128 and 4128 choose by the size of the grid (or of all members)
- *       between the latter, 8 x 96 and 16 columns x 96 rows with three rows
- *       per thread.
+ *       between columns as waves (single and batched grids), the latter, 8 x
+ *       96, and 16 columns x 48 or 96 rows with three rows per thread.
  * Both modes leave bit-identical `state` and `state_tmp`.
  * `kernel_ms` (HOST, 2 doubles, or NULL): if given, a HIP event is recorded
  * around every launch, the call blocks until they finish, and each launch's

@@ -20,8 +20,9 @@
 //  * x (k_dir_x<NS>): independent waves over the rows laid end to end, K cells
 //    per lane in registers, neighbours by one-lane shifts; the periodic cells
 //    are part of the extended rows.
-//  * z, LDS tiles: k_dir_zt1<NW,NR> with three rows per thread in registers,
-//    k_dir_z1<NR> with one cell per thread (small grids, low columns) and
+//  * z: k_dir_zt1<NW,NR>, LDS tiles with three rows per thread in registers,
+//    for large grids; k_dir_zw and k_dir_zs, columns as waves, for small ones;
+//    k_dir_z1<NR>, LDS tiles with one cell per thread, between them, and
 //    k_dir_z1d<NR>, the same over the column groups laid end to end. The wall
 //    halo rows of every stage state are rebuilt from its edge row.
 //  * k_ens_*: the same over the flattened tile list of an ensemble.
@@ -60,9 +61,11 @@ namespace {
 // are bound by FP64 issue in the steady state, with the start and the tail of
 // the launch on top (2.5 of 5 waves per SIMD on average). Per launch between
 // events, 512-thread LDS tiles / these waves / with the reciprocal pairs of
-// recip() and tend_of(): 2000 x 1000 52.3 / 42.5 / 38.7 us, 8192 x 4096 740 /
-// 599 / 551 us (3.9 TB/s of reads and writes; a 4 GB copy reaches 4.6). The cheaper power alone took the tiles from 51 to 47 us, and they
-// stayed at 42 with the power left out of a timing copy altogether.
+// recip() and tend_of() / with one table entry per power: 2000 x 1000 52.3 /
+// 42.5 / 38.7 / 37.3 us, 8192 x 4096 740 / 599 / 551 / 526 us (4.1 TB/s of reads
+// and writes; a 4 GB copy reaches 4.6). The cheaper power alone took the tiles
+// from 51 to 47 us, and they stayed at 42 with the power left out of a timing
+// copy altogether.
 constexpr int kXwWaves = 4;  // waves per block (they share nothing)
 
 template <int K>
@@ -86,8 +89,8 @@ inline int xw_blocks(int nx, int nz, int K, bool inflow = false) {
 // stages), the left halo (8, 9), cells 0 .. nx-1, the right halo. The halo
 // slots are refreshed at the start of every stage, the left ones from 4 slots
 // before. Cell 0 depends on 10 slots before it: windows [10, W-6). A step at
-// 1003 x 517 takes 36 us, 66 with one launch per RK stage and the copies of
-// the right halo between them (60 launches and 20 copies per 10 steps became
+// 1003 x 517 took 36 us (33 now), 66 with one launch per RK stage and the copies
+// of the right halo between them (60 launches and 20 copies per 10 steps became
 // 20 launches).
 //
 // Wave `b` of rows rbase .. rbase+nrows-1; E = xw_row_slots(nx, K).
@@ -351,13 +354,15 @@ __global__ __launch_bounds__(64 * kXwWaves)
 // which then meet in one XCD's L2).
 //
 // Measured (between events, one cell per thread with the RK init in registers
-// / this / with the reciprocal pairs): 2000 x 1000 63.2 / 55 / 50 us, 8192 x
-// 4096 980 / 867 / 786 us. Three rows per thread fit
-// 128 VGPRs (4 waves per SIMD, two 66 KB blocks per CU). Same boxes, not kept:
-// 8 columns x 96 rows in 256 threads 58 and 1200 us (64-byte rows), 4 rows per
-// thread (x 24 row groups) 73 and 1190 us, 6 rows (2 waves per SIMD) 53 and 874
-// us, 2 columns per wave without LDS 127 and 2740 us; block barriers instead of
-// the flags 50.4 and 801 us against 50.0 and 786.
+// / this / with the reciprocal pairs / with one table entry per power): 2000 x
+// 1000 63.2 / 55 / 50 / 48.9 us, 8192 x 4096 980 / 867 / 786 / 770 us. Three rows
+// per thread fit 128 VGPRs (4 waves per SIMD, two 66 KB blocks per CU). Same
+// boxes, not kept, against 55 and 867 us: 8 columns x 96 rows in 256 threads 58
+// and 1200 us (64-byte rows), 4 rows per thread (x 24 row groups) 73 and 1190
+// us, 6 rows (2 waves per SIMD) 53 and 874 us, 2 columns per wave without LDS
+// 127 and 2740 us; block barriers instead of the flags 50.4 and 801 us against
+// 50.0 and 786; two rows per thread, 64 to 128 rows, 4 to 6 waves per SIMD 64 to
+// 99 us against 48.9 (spills, and twice the LDS traffic per row).
 template <int NW, int NR>
 struct ZTileLds {
   static constexpr int NT = 64 * NW;
