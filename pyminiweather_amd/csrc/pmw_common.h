@@ -118,6 +118,22 @@ __device__ __forceinline__ void recon4(double s0, double s1, double s2,
   d3 = ((s0 * -1.0 + s1 * 3.0) + s2 * -3.0) + s3 * 1.0;
 }
 
+// The power of a face: of any argument, or of 64 <= x < 1024, where `rare` gets
+// the lanes with other arguments (in scalar registers).
+struct PowGamma {
+  __device__ __forceinline__ double operator()(double x) const { return pow_gamma(x); }
+};
+struct PowGammaIn {
+  unsigned long long& rare;
+  __device__ __forceinline__ double operator()(double x) const {
+    double s, l;
+    unsigned k;
+    pow_gamma_entry(x, s, l, k);
+    rare |= __builtin_amdgcn_ballot_w64(k >= 2048u);
+    return s + l;
+  }
+};
+
 // x-direction Euler flux with hyperviscosity (solve/interpolate.py:105-129).
 // The pressure's argument rho * t, t = (rho*theta) / rho, keeps the
 // reference's roundings (a last bit there is a last bit of a 1e5 Pa pressure).
@@ -125,15 +141,17 @@ __device__ __forceinline__ void recon4(double s0, double s1, double s2,
 // of rho * (m / rho), one product per term, and the products that are only
 // added into a flux are not rounded before: fewer roundings than the
 // reference's, which sit far below the pressure's last bit.
+// power: PowGamma, or PowGammaIn where the caller looks at `rare` afterwards.
+template <class Pow>
 __device__ __forceinline__ void flux_x_face(const double val[4],
                                             const double d3[4], double hyr,
                                             double hyt, double hv,
-                                            double F[4]) {
+                                            double F[4], Pow&& power) {
   const double rho = val[0] + hyr;
   const Recip r = recip(rho);
   const double u = quot(val[1], r);
   const double t = quot(val[3] + hyt, r);
-  const double p = kC0 * pow_gamma(rho * t);
+  const double p = kC0 * power(rho * t);
   F[0] = fma(-hv, d3[0], val[1]);
   F[1] = fma(-hv, d3[1], fma(val[1], u, p));
   F[2] = fma(-hv, d3[2], u * val[2]);
@@ -142,16 +160,17 @@ __device__ __forceinline__ void flux_x_face(const double val[4],
 
 // z-direction flux (solve/interpolate.py:153-186); `wall` marks faces k = 0
 // and k = nz, where w and the rho' 3rd difference are zeroed.
+template <class Pow>
 __device__ __forceinline__ void flux_z_face(const double val[4], double d3[4],
                                             double hyr, double hyt,
                                             double hyp, double hv, bool wall,
-                                            double G[4]) {
+                                            double G[4], Pow&& power) {
   const double rho = val[0] + hyr;
   const Recip r = recip(rho);
   const double m = wall ? 0.0 : val[2];  // rho w
   const double w = quot(m, r);
   const double t = quot(val[3] + hyt, r);
-  const double p = kC0 * pow_gamma(rho * t) - hyp;
+  const double p = kC0 * power(rho * t) - hyp;
   const double d0 = wall ? 0.0 : d3[0];
   G[0] = fma(-hv, d0, m);
   G[1] = fma(-hv, d3[1], w * val[1]);
