@@ -61,9 +61,9 @@ namespace {
 // are bound by FP64 issue in the steady state, with the start and the tail of
 // the launch on top (2.5 of 5 waves per SIMD on average). Per launch between
 // events, 512-thread LDS tiles / these waves / with the reciprocal pairs of
-// recip() and tend_of() / with one table entry per power: 2000 x 1000 52.3 /
-// 42.5 / 38.7 / 37.3 us, 8192 x 4096 740 / 599 / 551 / 526 us (4.1 TB/s of reads
-// and writes; a 4 GB copy reaches 4.6). The cheaper power alone took the tiles
+// recip() and tend_of() / with one table entry per power / tested once per wave:
+// 2000 x 1000 52.3 / 42.5 / 38.7 / 37.8 / 37.0 us, 8192 x 4096 740 / 599 / 551 /
+// 526 / 497 us (4.3 TB/s of reads and writes; a 4 GB copy reaches 4.6). The cheaper power alone took the tiles
 // from 51 to 47 us, and they stayed at 42 with the power left out of a timing
 // copy altogether.
 constexpr int kXwWaves = 4;  // waves per block (they share nothing)
