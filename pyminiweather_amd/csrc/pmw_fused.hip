@@ -295,8 +295,7 @@ __device__ __forceinline__ unsigned long long dir_x_run(const DirArgs& a, const 
 // If any argument of the wave lay outside the table: once more, with the power
 // of any argument. Nothing that the wave reads has been written since (a
 // launch's waves write each their own cells, and halo cells with the values they
-// have). The same for the z tiles gained nothing (2000 x 1000 50.2 / 50.3 us,
-// 48 ensemble grids 1535 / 1556): their faces wait for more than issue.
+// have).
 template <int K, bool INFLOW>
 __device__ __forceinline__ void dir_x_wave(const DirArgs& a, const Grid& g, unsigned b,
                                            unsigned E, int rbase, int nrows,
@@ -377,9 +376,11 @@ __global__ __launch_bounds__(64 * kXwWaves)
 // which then meet in one XCD's L2).
 //
 // Measured (between events, one cell per thread with the RK init in registers
-// / this / with the reciprocal pairs / with one table entry per power): 2000 x
-// 1000 63.2 / 55 / 50 / 48.9 us, 8192 x 4096 980 / 867 / 786 / 770 us. Three rows
-// per thread fit 128 VGPRs (4 waves per SIMD, two 66 KB blocks per CU). Same
+// / this / with the reciprocal pairs / with one table entry per power / its range
+// tested once per stage): 2000 x 1000 63.2 / 55 / 50 / 49.2 / 47.6 us, 8192 x 4096
+// 980 / 867 / 786 / 769 / 738 us. (Tested once per tile, with a block barrier and
+// the whole tile run again: no faster than once per face.) Three rows per thread
+// fit 128 VGPRs (4 waves per SIMD, two 66 KB blocks per CU). Same
 // boxes, not kept, against 55 and 867 us: 8 columns x 96 rows in 256 threads 58
 // and 1200 us (64-byte rows), 4 rows per thread (x 24 row groups) 73 and 1190
 // us, 6 rows (2 waves per SIMD) 53 and 874 us, 2 columns per wave without LDS
@@ -389,12 +390,13 @@ __global__ __launch_bounds__(64 * kXwWaves)
 template <int NW, int NR>
 struct ZTileLds {
   static constexpr int NT = 64 * NW;
+  double hz[3][NR];    // rho, rho*theta, p at the rows' lower faces
+  int wf[NW + 2];      // wave phase flags
+  // the large arrays last: every slot within the 64 KB of an offset field
   double lo[kNv][NT];  // each thread's first row,
   double h1[kNv][NT];  // its last row
   double h2[kNv][NT];  // and the one before
   double f0[kNv][NT];  // flux at its first face
-  double hz[3][NR];    // rho, rho*theta, p at the rows' lower faces
-  int wf[NW + 2];      // wave phase flags
 };
 
 constexpr int kZtCols = 16, kZtK = 3;
@@ -533,37 +535,54 @@ __device__ __forceinline__ void dir_zt1_tile(const DirArgs& a, const Grid& g, in
       }
     };
     const int tp = t >= CW ? t - CW : t, tn = t + CW < NT ? t + CW : t;  // rows before, after
-    double b2[4], b1[4], Fp[4];  // the two rows before, the flux behind
-#pragma unroll
-    for (int v = 0; v < kNv; ++v) {
-      b2[v] = sm.h2[v][tp];
-      b1[v] = sm.h1[v][tp];
-    }
-#pragma unroll
-    for (int j = 0; j < K; ++j) {  // face k0+j, then row k0+j-1
-      double v4[4], d3[4], F[4], cur[4];
+    double b1[4], Fp[4];  // the row before, the flux behind
+    // the stage's faces, each followed by the row before it but the last
+    auto faces = [&](auto power) {
+      double b2[4];
 #pragma unroll
       for (int v = 0; v < kNv; ++v) {
-        cur[v] = s[j][v];
-        recon4(b2[v], b1[v], cur[v], j + 1 < K ? s[j + 1 < K ? j + 1 : j][v] : sm.lo[v][tn],
-               v4[v], d3[v]);
+        b2[v] = sm.h2[v][tp];
+        b1[v] = sm.h1[v][tp];
       }
-      const int q = rg * K + j;
-      flux_z_face(v4, d3, sm.hz[0][q], sm.hz[1][q], sm.hz[2][q], a.hv,
-                  k0 + j == 0 || k0 + j == nz, F, PowGamma{});
-      if (j == 0) {
 #pragma unroll
-        for (int v = 0; v < kNv; ++v) sm.f0[v][t] = F[v];
-      } else {
-        update(j - 1, b1, Fp, F);
+      for (int j = 0; j < K; ++j) {  // face k0+j, then row k0+j-1
+        double v4[4], d3[4], F[4], cur[4];
+#pragma unroll
+        for (int v = 0; v < kNv; ++v) {
+          cur[v] = s[j][v];
+          recon4(b2[v], b1[v], cur[v], j + 1 < K ? s[j + 1 < K ? j + 1 : j][v] : sm.lo[v][tn],
+                 v4[v], d3[v]);
+        }
+        const int q = rg * K + j;
+        flux_z_face(v4, d3, sm.hz[0][q], sm.hz[1][q], sm.hz[2][q], a.hv,
+                    k0 + j == 0 || k0 + j == nz, F, power);
+        if (j == 0) {
+#pragma unroll
+          for (int v = 0; v < kNv; ++v) sm.f0[v][t] = F[v];
+        } else {
+          update(j - 1, b1, Fp, F);
+        }
+#pragma unroll
+        for (int v = 0; v < kNv; ++v) {
+          b2[v] = b1[v];
+          b1[v] = cur[v];
+          Fp[v] = F[v];
+        }
+        __builtin_amdgcn_sched_barrier(0);  // one face's values live at a time
       }
+    };
+    unsigned long long rare = 0;
+    faces(PowGammaIn{rare});
+    if (__builtin_expect(rare != 0, 0)) {
+      // an argument outside the table: once more, from the published rows (a
+      // neighbour publishes again only after this wave's flag)
 #pragma unroll
       for (int v = 0; v < kNv; ++v) {
-        b2[v] = b1[v];
-        b1[v] = cur[v];
-        Fp[v] = F[v];
+        s[0][v] = sm.lo[v][t];
+        s[1][v] = sm.h2[v][t];
+        s[2][v] = sm.h1[v][t];
       }
-      __builtin_amdgcn_sched_barrier(0);  // one face's values live at a time
+      faces(PowGamma{});
     }
     wave_phase_done(sm.wf, 2 * stage + 1, t);
     {

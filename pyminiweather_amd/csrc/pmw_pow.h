@@ -316,9 +316,10 @@ PMW_HD double significand(double x) {
 // 4096 1315 / 1277, of 1003 x 517 33.8 / 33.0. With uniform loads (a timing
 // copy, wrong values) 2000 x 1000 takes 75.1.
 //
-// The x waves take the value of the entry alone (PowGammaIn) and look at k once,
-// after their last face: a test and a branch in every face cost 5 % of a large
-// launch (8192 x 4096 523 / 499 us, 2000 x 1000 38.4 / 37.6).
+// The x waves and the large z tiles take the value of the entry alone
+// (PowGammaIn) and look at k once, after a wave's last face (x) or a stage's (z):
+// a test and a branch in every face cost 4 to 5 % of a large launch (8192 x 4096
+// x 523 / 497 us, z 769 / 738; 2000 x 1000 x 38.4 / 37.6, z 49.4 / 47.6).
 
 // x^gamma = (s + l) times 1 for k < 2048, else times the binade's factor.
 PMW_HD void pow_gamma_entry(double x, double& s, double& l, unsigned& k) {
