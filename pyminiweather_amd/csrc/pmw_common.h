@@ -95,8 +95,9 @@ struct Grid {
 // (relative error e below 2^-46), yl = e y the remainder, so that y + yl is
 // 1/b to 2^-92, and a/b = RN(a y + RN(a yl)) is the correctly rounded
 // quotient except with probability ~2^-38: 5 instructions, and 2 per
-// quotient, instead of 10 for an IEEE reciprocal and 3. As with the division
-// by b, 0, infinite and NaN b give NaN quotients here.
+// quotient, instead of 10 for an IEEE reciprocal and 3. Unlike a division, a
+// zero or infinite b gives NaN, and an infinite a gives an infinity or NaN with
+// the sign of yl.
 struct Recip {
   double y, yl;
 };
@@ -187,11 +188,13 @@ __device__ __forceinline__ double tend_of(double f_lo, double f_hi, double id, d
 
 // Value the reference's set_bc_z leaves in z-halo row `prow` (0, 1, nz+2 or
 // nz+3) of variable v, given the same column's value on the adjacent interior
-// edge row (bcs.py:92-148).
+// edge row (bcs.py:92-148). An IEEE division, so that an infinite momentum stays
+// one (quot may make it NaN); only the wall's rows take it, and a step of every
+// size from 100 x 50 to 8192 x 4096 takes as long with quot (+- 0.8 %).
 __device__ __forceinline__ double wall_halo(int v, double edge_val,
                                             double hy_edge, double hy_halo) {
   if (v == 2) return 0.0;
-  if (v == 1) return quot(edge_val, recip(hy_edge)) * hy_halo;
+  if (v == 1) return edge_val / hy_edge * hy_halo;
   return edge_val;
 }
 

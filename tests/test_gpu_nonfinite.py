@@ -1,0 +1,38 @@
+"""Infinite values through the per-function kernels, against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+INF, NAN = float("inf"), float("nan")
+
+
+def _fields(p):
+    from pyminiweather_amd.data import initialize_fields
+    from pyminiweather_amd.ics import init
+    from pyminiweather_amd.mesh import MeshData
+    f = initialize_fields(p)
+    init(f, p, MeshData(p))
+    return f
+
+
+@pytest.mark.parametrize("nz", [4, 5, 6, 7, 8, 9])
+def test_wall_halos_of_non_finite_momenta(nz):
+    """rho*u of the edge rows divided by one density (several, whose reciprocals
+    round up and down) and multiplied by another: infinities keep their sign,
+    and finite values of any size their bits."""
+    from pyminiweather_amd.ics import set_bc_z
+    p = O.make_params(9, nz, "thermal")
+    f = _fields(p)
+    edge = torch.tensor([INF, -INF, NAN, 1.7e308, -1.7e308, 1e-320, -0.0, 3.0, -7.5],
+                        dtype=torch.float64, device="cuda")
+    f.state[1, 2, 2:-2] = edge
+    f.state[1, nz + 1, 2:-2] = edge.flip(0)
+    want = f.state.cpu().numpy()
+    with np.errstate(all="ignore"):
+        O.halo_z(p, {"hy_dens_cell": f.hy_dens_cell.cpu().numpy()}, want)
+    set_bc_z(p, f, f.state, "thermal")
+    np.testing.assert_array_equal(f.state.cpu().numpy(), want)
