@@ -36,3 +36,18 @@ def test_wall_halos_of_non_finite_momenta(nz):
         O.halo_z(p, {"hy_dens_cell": f.hy_dens_cell.cpu().numpy()}, want)
     set_bc_z(p, f, f.state, "thermal")
     np.testing.assert_array_equal(f.state.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("row", [0, 1, 2, 3, 4, 5])
+@pytest.mark.parametrize("value", [INF, -INF, 1e200])
+def test_energy_of_infinite_momentum(row, value):
+    """A cell whose kinetic energy is or overflows to infinity (several rows, so
+    several densities): mass as before, energy +inf, as in the oracle."""
+    from pyminiweather_amd.post import compute_stats
+    p = O.make_params(7, 6, "thermal")
+    f = _fields(p)
+    mass = compute_stats(p, f)[0]
+    for v in (1, 2):
+        f.state[v, row + 2, 4] = value
+        assert compute_stats(p, f) == (mass, INF)
+        f.state[v, row + 2, 4] = 0.0
