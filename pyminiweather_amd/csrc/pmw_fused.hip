@@ -232,9 +232,9 @@ __device__ __forceinline__ unsigned long long dir_x_run(const DirArgs& a, const 
         recon4(b2[v], b1[v], cur[v], j + 1 < K ? s[K - 1][v] : nx1[v], v4[v], d3[v]);
       }
       if constexpr (ANY)
-        flux_x_face(v4, d3, hyr, hyt, a.hv, F, PowGamma{});
+        flux_x_face<false>(v4, d3, hyr, hyt, a.hv, F, PowGamma{});
       else
-        flux_x_face(v4, d3, hyr, hyt, a.hv, F, PowGammaIn{rare});
+        flux_x_face<false>(v4, d3, hyr, hyt, a.hv, F, PowGammaIn{rare});
       if (j == 0) {
 #pragma unroll
         for (int v = 0; v < kNv; ++v) F0[v] = F[v];
@@ -554,8 +554,8 @@ __device__ __forceinline__ void dir_zt1_tile(const DirArgs& a, const Grid& g, in
                  v4[v], d3[v]);
         }
         const int q = rg * K + j;
-        flux_z_face(v4, d3, sm.hz[0][q], sm.hz[1][q], sm.hz[2][q], a.hv,
-                    k0 + j == 0 || k0 + j == nz, F, power);
+        flux_z_face<false>(v4, d3, sm.hz[0][q], sm.hz[1][q], sm.hz[2][q], a.hv,
+                           k0 + j == 0 || k0 + j == nz, F, power);
         if (j == 0) {
 #pragma unroll
           for (int v = 0; v < kNv; ++v) sm.f0[v][t] = F[v];
@@ -729,7 +729,7 @@ __device__ __forceinline__ void dir_z_wave(const DirArgs& a, const Grid& g, int 
       const double b1 = from_prev(s[v]);
       recon4(from_prev(b1), b1, s[v], from_next(s[v]), v4[v], d3[v]);
     }
-    flux_z_face(v4, d3, hyr, hyt, hyp, a.hv, k == 0 || k == nz, F, PowGamma{});
+    flux_z_face<false>(v4, d3, hyr, hyt, hyp, a.hv, k == 0 || k == nz, F, PowGamma{});
     double td[4];
 #pragma unroll
     for (int v = 0; v < kNv; ++v) td[v] = tend_of(F[v], from_next(F[v]), a.id, a.idl);
@@ -867,7 +867,8 @@ __device__ __forceinline__ void dir_z1_tile(const DirArgs& a, const Grid& g, int
 #pragma unroll
       for (int v = 0; v < kNv; ++v)
         recon4(s[v][u - 2 * CW], s[v][u - CW], s[v][u], s[v][u + CW], v4[v], d3[v]);
-      flux_z_face(v4, d3, hz[0][j], hz[1][j], hz[2][j], a.hv, k == 0 || k == nz, G, PowGamma{});
+      flux_z_face<false>(v4, d3, hz[0][j], hz[1][j], hz[2][j], a.hv, k == 0 || k == nz, G,
+                         PowGamma{});
 #pragma unroll
       for (int v = 0; v < kNv; ++v) fl[v][u] = G[v];
     }
@@ -1017,7 +1018,8 @@ __device__ __forceinline__ void dir_z1d_tile(const DirArgs& a, const Grid& g, in
 #pragma unroll
       for (int v = 0; v < kNv; ++v)
         recon4(s[v][u - 2 * CW], s[v][u - CW], s[v][u], s[v][u + CW], v4[v], d3[v]);
-      flux_z_face(v4, d3, hz[0][j], hz[1][j], hz[2][j], a.hv, k == 0 || k == nz, G, PowGamma{});
+      flux_z_face<false>(v4, d3, hz[0][j], hz[1][j], hz[2][j], a.hv, k == 0 || k == nz, G,
+                         PowGamma{});
 #pragma unroll
       for (int v = 0; v < kNv; ++v) fl[v][u] = G[v];
     }

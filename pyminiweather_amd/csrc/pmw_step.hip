@@ -176,7 +176,7 @@ __global__ __launch_bounds__(256) void k_flux_x(
     a[v] = vals[v * pv + o];
     b[v] = d3[v * pv + o];
   }
-  flux_x_face(a, b, hyr[k + kHs], hyt[k + kHs], hv, F, PowGamma{});
+  flux_x_face<true>(a, b, hyr[k + kHs], hyt[k + kHs], hv, F, PowGamma{});
 #pragma unroll
   for (int v = 0; v < kNv; ++v) flux[v * pf + o] = F[v];
 }
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(256) void k_flux_z(
     a[v] = vals[v * pv + idx];
     b[v] = d3[v * pv + idx];
   }
-  flux_z_face(a, b, hyr[k], hyt[k], hyp[k], hv, wall, G, PowGamma{});
+  flux_z_face<true>(a, b, hyr[k], hyt[k], hyp[k], hv, wall, G, PowGamma{});
   if (wall) d3[idx] = 0.0;  // d3_vals_z[rho'] zeroed in place (interpolate.py:172-173)
   const long long o = (long long)k * (g.nx + 1) + i;
 #pragma unroll
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(kXThreads) void k_stage_x(
 #pragma unroll
     for (int v = 0; v < kNv; ++v)
       recon4(sv[v][t], sv[v][t + 1], sv[v][t + 2], sv[v][t + 3], a[v], b[v]);
-    flux_x_face(a, b, hr, ht, hv, F, PowGamma{});
+    flux_x_face<true>(a, b, hr, ht, hv, F, PowGamma{});
 #pragma unroll
     for (int v = 0; v < kNv; ++v) sf[v][t] = F[v];
   }
@@ -417,7 +417,7 @@ __global__ __launch_bounds__(kZtCols* kZtRows) void k_stage_z(
 #pragma unroll
     for (int v = 0; v < kNv; ++v)
       recon4(s[v][t - 2 * CW], s[v][t - CW], s[v][t], s[v][t + CW], a[v], b[v]);
-    flux_z_face(a, b, hr, ht, hp, hv, k == 0 || k == nz, G, PowGamma{});
+    flux_z_face<true>(a, b, hr, ht, hp, hv, k == 0 || k == nz, G, PowGamma{});
 #pragma unroll
     for (int v = 0; v < kNv; ++v) fl[v][t] = G[v];
   }

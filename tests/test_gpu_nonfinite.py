@@ -1,4 +1,4 @@
-"""Infinite values through the per-function kernels, against the oracle."""
+"""Infinite and undefined values through the per-function kernels, against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -51,3 +51,65 @@ def test_energy_of_infinite_momentum(row, value):
         f.state[v, row + 2, 4] = value
         assert compute_stats(p, f) == (mass, INF)
         f.state[v, row + 2, 4] = 0.0
+
+
+@pytest.mark.parametrize("case", ["nan state", "nan profile", "no density"])
+def test_fluxes_are_nan_where_the_oracles_are(case):
+    """A NaN density in a state's edge rows and inside, a NaN or zero row of the
+    background: no flux of such a face is finite, the mass fluxes through the
+    walls and along the row among them."""
+    import pyminiweather_amd.solve as S
+    p = O.make_params(11, 6, "thermal")
+    f = _fields(p)
+    a = O.init_state(p)
+    if case == "nan state":
+        for k, i in ((0, 2), (5, 8), (3, 5)):
+            a["state"][0, k + 2, i + 2] = NAN
+    else:
+        value = NAN if case == "nan profile" else 0.0
+        a["hy_dens_cell"][4] = a["hy_dens_int"][0] = a["hy_dens_int"][3] = value
+    O.halo_x(p, a, a["state"])
+    with np.errstate(all="ignore"):
+        O.halo_z(p, {"hy_dens_cell": np.ones(10)}, a["state"])
+        want_x = O.flux_x(p, a, *O.reconstruct_x(p, a["state"]))
+        want_z = O.flux_z(p, a, *O.reconstruct_z(p, a["state"]))
+    for k in ("state", "hy_dens_cell", "hy_dens_int"):
+        getattr(f, k).copy_(torch.from_numpy(a[k]))
+    S.interpolate_x(p, f)
+    S.compute_flux_x(p, f)
+    got_x = f.flux[:, :-1].cpu().numpy()
+    S.interpolate_z(p, f)
+    S.compute_flux_z(p, f)
+    got_z = f.flux[:, :, :-1].cpu().numpy()
+    for got, want in ((got_x, want_x), (got_z, want_z)):
+        assert np.isnan(want).any() and not np.isnan(want).all()
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+
+
+@pytest.mark.parametrize("nx,nz", [(60, 40), (400, 120), (700, 450)])
+@pytest.mark.parametrize("case", ["nan state", "nan profile", "no density"])
+def test_evolve_spreads_nans_as_the_stages_do(nx, nz, case):
+    """A step of the fused directions leaves NaN where the per-stage kernels do
+    and the same bits elsewhere, in state and state_tmp."""
+    import pyminiweather_amd.solve as S
+    p = O.make_params(nx, nz, "thermal", cfl=0.5)
+    out = []
+    for tuning in ((0, 512, 8096), (1, 512, 8096)):
+        f = _fields(p)
+        if case == "nan state":
+            for k, i in ((0, 2), (nz - 1, nx - 3), (nz // 2, 0)):
+                f.state[0, k + 2, i + 2] = NAN
+        else:
+            value = NAN if case == "nan profile" else 0.0
+            f.hy_dens_cell[nz // 3 + 2] = f.hy_dens_int[nz // 3] = value
+        S.set_tuning(nx, nz, tuning)
+        S.reverse_direction = False
+        try:
+            S.evolve(p, f, None, dt=p["dt"])
+        finally:
+            S._tuning_table.clear()
+            S.reverse_direction = False
+        out.append((f.state.cpu().numpy(), f.state_tmp.cpu().numpy()))
+    for fused, staged in zip(*out):
+        assert np.isnan(staged).any() and not np.isnan(staged).all()
+        np.testing.assert_array_equal(fused, staged)
