@@ -1332,7 +1332,10 @@ ZKernel fused_z_kernel(int seg, long long cells, int min_nz, int max_nx) {
 int launch_dir_x(const DirArgs& a, Grid g, int nt, hipStream_t st, int members) {
   if (members < 1 || members > 65535 || (members > 1 && a.mstride <= 0)) return PMW_EINVAL;
   if (!fused_x_tile_ok(nt) || (a.inj_rows && g.nx < kMinInflowCells)) return PMW_EINVAL;
-  if (nt > 1000 && (long long)g.nz * (g.nx + 12) > (1LL << 30)) return PMW_EINVAL;
+  // the bound of these codes; the inflow, which has always run whatever the code,
+  // has none (the kernels take rows beyond 2^31 slots as further blockIdx.z)
+  if (nt > 1000 && !a.inj_rows && (long long)g.nz * (g.nx + 12) > (1LL << 30))
+    return PMW_EINVAL;
   return fused_x_cells(nt, (long long)g.nx * g.nz * members) == 1
              ? launch_x<1>(a, g, st, members)
              : launch_x<2>(a, g, st, members);
