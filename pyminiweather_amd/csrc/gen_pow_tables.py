@@ -10,11 +10,12 @@ decimal module at 60 digits and rounded to doubles.
   4th entry, 2^(j/64)).
 * gamma: for j = 0..511, c_j = 1/(1 + (j + 1/2)/512) rounded to 10 bits, so
   that r = m*c_j - 1 is exact in one fma for m in [1 + j/512, 1 + (j+1)/512)
-  (|r| <= 2^-9); for the four binades from 2^6, entry 512 o + j: the power
-  (2^(6+o) / c_j)^gamma as a double and a float of its rest, and c_j as a float
-  (kGamQ); and for other binades, whose significands use the entries of binade
-  6 + (e-6) mod 4, 2^(4 (i-258) gamma) for i = 1.. as a double-double (0 for
-  i = 0, times 2^64 for i < 100, up to the largest that is finite, then one NaN).
+  (|r| <= 2^-9); for the sixteen binades from 2^-6, entry 512 o + j: the power
+  (2^(o-6) / c_j)^gamma as a double and a float of its rest, and c_j as a float
+  (kGamQ); and for other binades e, whose significands use the entries of binade
+  (e+6) mod 16 - 6, 2^(16 (i-64) gamma) for i = 0.. as a double-double, times
+  2^64 for i < 36 and 2^-64 for i >= 100, up to the last i with a finite power,
+  then one NaN (kGamE).
 * gamma - 1: c_j^(1-gamma) and c_j (kGamM), and for every biased exponent e of
   a double 2^((e-1023) (gamma-1)) (kGamD).
   gamma is the double nearest to the physical constant.
@@ -63,23 +64,21 @@ def main():
     gamma = Decimal(GAMMA)
     ln2 = Decimal(2).ln()
     gq, gm = [], []
-    for i in range(2048):
+    for i in range(8192):
         o, j = divmod(i, 512)
         c = round_bits(1 / (1 + (Decimal(j) + Decimal("0.5")) / 512), 10)
         for m in (1 + Decimal(j) / 512, 1 + Decimal(j + 1) / 512):
             assert abs(m * c - 1) <= Decimal(2) ** -9
-        lx = (6 + o) * ln2 - c.ln()
+        lx = (o - 6) * ln2 - c.ln()
         h, l = dd((gamma * lx).exp())
         gq.append((h, f32(l), f32(c)))
         assert Decimal(f32(c)) == c
         if o == 0:
             gm += [rn(((1 - gamma) * c.ln()).exp()), rn(c)]
     ge, gd = [], []
-    for i in range(513):
-        k = 4 * (i - 258)
-        if k * gamma < 1024:
-            lift = 64 * ln2 if i < 100 else 0  # clear of subnormal factors
-            ge += dd((k * gamma * ln2 + lift).exp()) if i else (0.0, 0.0)
+    for i in range(111):
+        lift = 64 if i < 36 else -64 if i >= 100 else 0  # clear of subnormals and overflow
+        ge += dd(((16 * (i - 64) * gamma + lift) * ln2).exp())
     for e in range(2048):
         gd.append(rn(((e - 1023) * (gamma - 1) * ln2).exp()))
 
@@ -102,6 +101,7 @@ def main():
     arr("kExpHi", th)
     arr("kExpLo", tl)
     out.append("struct alignas(16) GamQ {\n  double h;\n  float l, c;\n};")
+    out.append(f"constexpr unsigned kGamEntries = {len(gq)};")
     out.append(f"constexpr GamQ kGamQ[{len(gq)}] = {{")
     out.extend("    {%s, %sf, %sf}," % tuple(float.hex(v) for v in q) for q in gq)
     out.append("};")

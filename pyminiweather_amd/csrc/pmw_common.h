@@ -119,7 +119,7 @@ __device__ __forceinline__ void recon4(double s0, double s1, double s2,
   d3 = ((s0 * -1.0 + s1 * 3.0) + s2 * -3.0) + s3 * 1.0;
 }
 
-// The power of a face: of any argument, or of 64 <= x < 1024, where `rare` gets
+// The power of a face: of any argument, or of 2^-6 <= x < 1024, where `rare` gets
 // the lanes with other arguments (in scalar registers).
 struct PowGamma {
   __device__ __forceinline__ double operator()(double x) const { return pow_gamma(x); }
@@ -130,7 +130,7 @@ struct PowGammaIn {
     double s, l;
     unsigned k;
     pow_gamma_entry(x, s, l, k);
-    rare |= __builtin_amdgcn_ballot_w64(k >= 2048u);
+    rare |= __builtin_amdgcn_ballot_w64(k >= powt::kGamEntries);
     return s + l;
   }
 };

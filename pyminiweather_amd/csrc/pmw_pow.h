@@ -27,11 +27,10 @@
 // ~1e-6 of arguments; glibc's pow, which NumPy calls, misses in 8e-4).
 //
 // pow_gamma evaluates the one power of the flux, x^gamma, without a logarithm
-// or an exponential: the exponent is fixed, so c_j^-gamma (m's table value)
-// and 2^((e-1023) gamma) (the binary exponent's) are tables and what is left
-// is (1 + r)^gamma, |r| <= 2^-9, a short binomial series. About 40 VALU
-// instructions and 3 loads, all issued at once, against 131 and two dependent
-// rounds of loads of pow_pos, at pow_pos's accuracy.
+// or an exponential: the exponent is fixed, so (2^e / c_j)^gamma is a table and
+// what is left is (1 + r)^gamma, |r| <= 2^-9, a short binomial series. About 40
+// VALU instructions and one 16-byte load, against 131 and two dependent rounds of
+// loads of pow_pos, at pow_pos's accuracy.
 //
 // pow_pos_near continues a power already evaluated at a nearby argument with
 // the binomial series of (1 + e)^y and returns pow_pos's result bit for bit:
@@ -299,16 +298,24 @@ PMW_HD double significand(double x) {
 
 // x^gamma for gamma = kGamma's double (pmw_common.h), the exponent of the
 // tables. x = 2^(e-1023) m; j = m's first 9 fraction bits; r = m c_j - 1,
-// exact; x^gamma = (2^(e-1023) / c_j)^gamma (1 + r)^gamma. For 64 <= x < 1024
-// (rho*theta of any atmosphere) one 16-byte table entry holds c_j and the first
-// factor as a double and a float; elsewhere the entry of the binade 6 + (e-6)
-// mod 4 is scaled by a second, double-double factor. The linear term of the
-// series is double-double; the quadratic and later terms (< 2^-19.8) are
-// doubles, whose rounding sets the error of the value before the last
-// rounding: all but ~1e-6 of results are the correctly rounded ones. Powers
-// that overflow give inf; other arguments as pow(x, gamma): +-0 -> 0, +-inf ->
-// inf, negative and NaN -> NaN; subnormal arguments, whose power is below the
-// smallest double, give 0.
+// exact; x^gamma = (2^(e-1023) / c_j)^gamma (1 + r)^gamma. For 2^-6 <= x < 1024
+// one 16-byte table entry holds c_j and the first factor as a double and a float;
+// elsewhere the entry of the same significand there is scaled by a second,
+// double-double factor. The linear term of the series is double-double; the
+// quadratic and later terms (< 2^-19.8) are doubles, whose rounding sets the error
+// of the value before the last rounding (2.7e-22 relative): one in 3e6 results is
+// not the correctly rounded one. Powers that overflow give inf; other arguments as
+// pow(x, gamma): +-0 -> 0, +-inf -> inf, negative and NaN -> NaN; subnormal
+// arguments, whose power is below the smallest double, give 0.
+//
+// The range: rho*theta falls with height, over a constant-theta background from
+// 350 at the ground to 65 at 15 km, 25 at 20 km, 0.8 at 28 km and 2^-6 at 30.2 km (at
+// 30.7 km its pressure ends). A row touches the one or two entries near its value,
+// so the rest of the 128 KB costs nothing. With four binades (64 <= x, 32 KB)
+// every row above 15 km was computed twice; step of 2000 x 1000 in us, four / sixteen
+// binades, column of 10 km 76.4 / 76.4, 20 km 132.8 / 76.1, 28 km 133.4 / 76.1;
+// 800 x 400 23.4 / 23.4, 37.9 / 23.4, 38.2 / 23.4; 1003 x 517 with the inflow 32.7 /
+// 32.8, 53.7 / 32.8, 54.2 / 32.8.
 //
 // The entry is a gather, and the flux kernels pay for its bytes. Three loads of
 // 40 bytes a lane (c_j and double-doubles of c_j^-gamma and of every binade's
@@ -321,11 +328,11 @@ PMW_HD double significand(double x) {
 // a test and a branch in every face cost 4 to 5 % of a large launch (8192 x 4096
 // x 523 / 497 us, z 769 / 738; 2000 x 1000 x 38.4 / 37.6, z 49.4 / 47.6).
 
-// x^gamma = (s + l) times 1 for k < 2048, else times the binade's factor.
+// x^gamma = s + l for k < kGamEntries, else s + l times the binade's factor.
 PMW_HD void pow_gamma_entry(double x, double& s, double& l, unsigned& k) {
   using namespace powt;
-  k = (high_word(x) >> 11) - (1029u << 9);           // < 2048: 64 <= x < 1024
-  const GamQ t = kGamQ[k & 2047u];
+  k = (high_word(x) >> 11) - (1017u << 9);           // 2^-6 <= x < 1024: an index
+  const GamQ t = kGamQ[k & (kGamEntries - 1u)];
   const double r = fma(significand(x), (double)t.c, -1.0);  // exact
   const double th = t.h, tl = t.l;
   // c_k = gamma (gamma-1) ... (gamma-k+1) / k!, k = 7..2; c_8 r^8 < 2^-80
@@ -348,14 +355,14 @@ PMW_HD double pow_gamma(double x) {
   double s, l;
   unsigned k;
   pow_gamma_entry(x, s, l, k);
-  if (__builtin_expect(k >= 2048u, 0)) {
+  if (__builtin_expect(k >= kGamEntries, 0)) {
     // the last entry (NaN) serves powers past the largest, NaN and a set sign
-    const unsigned e = ((high_word(x) >> 20) + 3u) >> 2;
+    const unsigned e = ((high_word(x) >> 20) + 7u) >> 4;
     const double* te = kGamE + 2u * (e < kGamELast ? e : kGamELast);
     const double eh = te[0], el = te[1];
     const double h = s * eh;                         // (s + l)(eh + el)
     const double up = h + fma(l, eh, fma(s, el, fma(s, eh, -h)));
-    const double res = e < 100u ? up * 0x1p-64 : up;  // as the table's entries
+    const double res = e < 36u ? up * 0x1p-64 : e < 100u ? up : up * 0x1p64;  // as kGamE
     const double inf = __builtin_inf();
     if (res < inf) return res;
     return x == 0.0 ? 0.0 : (x > 0.0 || x == -inf) ? inf : __builtin_nan("");
