@@ -83,8 +83,23 @@ def valu_from_profile(kernel):
     return None
 
 
+def launched_kernels(tuning, nx, nz):
+    """The x and z kernels (rocprof names) that a fused tuning launches on the
+    grid of the committed summary, 2000 x 1000 (the choices by size of
+    include/pmw.h at that size); None on others, whose launches its counts do
+    not describe."""
+    if (nx, nz) != (2000, 1000):
+        return None, None
+    _, xb, zs = tuning
+    x = "k_dir_x<256>" if xb == 256 else "k_dir_x<512>"
+    z = ("k_dir_z1<32>" if zs <= 64 else "k_dir_z1d<96>" if zs in (18096, 18128) else
+         "k_dir_zt1<8, 96>")
+    return x, z
+
+
 def fused_kernel_names(tuning):
-    """The x and z kernels (rocprof names) that a fused tuning launches."""
+    """The shapes that the tuning codes are named after (codes of one shape have
+    since come to share kernels: launched_kernels)."""
     _, xb, zs = tuning
     x = f"k_dir_xd<{xb - 1000}>" if xb > 1000 else f"k_dir_x<{xb}>"
     if zs == 18128:
@@ -469,7 +484,7 @@ def main():
     if S.tuning_for(nx, nz)[0] == 0:
         names = {0: "k_dir_x (x direction, 3 fused RK stages)",
                  1: "k_dir_z (z direction, 3 fused RK stages)"}
-        prefixes = dict(enumerate(fused_kernel_names(S.tuning_for(nx, nz))))
+        prefixes = dict(enumerate(launched_kernels(S.tuning_for(nx, nz), nx, nz)))
     else:  # per-stage kernels: a direction's three launches summed (no per-launch traffic)
         names = {0: "k_stage_x (x direction, its 3 RK-stage launches summed)",
                  1: "k_stage_z (z direction, its 3 RK-stage launches summed)"}
@@ -530,9 +545,10 @@ def main():
                                   "unit": "G wave64 VALU instructions/s",
                                   "frac": round(dom_valu / dom_avg_s / VALU_ISSUE_PEAK, 4)}
                                  if dom_valu else None),
-                     "binding": ("fp64_valu_issue" if dom_valu and dom_traffic and
-                                 dom_valu / VALU_ISSUE_PEAK > dom_traffic / (HBM_PEAK_GBS * 1e9)
-                                 else "hbm")},
+                     # the resource of which the counted launch uses more
+                     "binding": (("fp64_valu_issue" if dom_valu / VALU_ISSUE_PEAK >
+                                  dom_traffic / (HBM_PEAK_GBS * 1e9) else "hbm")
+                                 if dom_valu and dom_traffic else None)},
         "step_roofline_frac": round(value * BYTES_PER_CELL_STEP / 1e9 / HBM_PEAK_GBS, 4),
         "gpu_ms_per_step": gpu_s / args.steps * 1e3,
         "kernels": kern,
