@@ -18,12 +18,12 @@ from . import _lib
 from . import solve as S
 from ._lib import ptr, stream_of
 
-# x: waves with one (256) or two (1512) cells per lane; the other codes choose
-# between them by size
-X_BLOCKS = (256, 448, 512, 1256, 1512)
-# z: 8..64 one-cell tiles of 32 rows, 18096 / 18128 dense one-cell tiles of 96
-# rows; the other codes choose by size
-Z_SEGMENTS = (8, 16, 24, 32, 48, 64, 8064, 4128, 8096, 8128, 18128, 18096)
+# One code per kernel (include/pmw.h lists the others): of several codes of one
+# kernel the fastest is that kernel's best of several samples, and wins against a
+# faster kernel with one. x: waves with one (256) or two (1512) cells per lane.
+X_BLOCKS = (256, 1512)
+# z: by size (8096), one-cell tiles of 32 rows, dense ones of 96
+Z_SEGMENTS = (8096, 32, 18096)
 
 
 def _time_grid(params, fields, tuning, steps, bufs):
