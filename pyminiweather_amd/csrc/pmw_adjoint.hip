@@ -514,7 +514,7 @@ int launch_adj_x(const AdjDirArgs& a, Grid g, int members, hipStream_t st) {
 // slots outside the domain keep the zero they were loaded with.
 //
 // Bound by the memory's latency and by its own chain of phases: 24 waves per
-// CU (96 B of LDS per slot, 76 VGPRs) move 384 MB in about 100 us at 2000 x
+// CU (96 B of LDS per slot, 66 VGPRs) move 384 MB in about 100 us at 2000 x
 // 1000, with the FP64 pipes a third busy. The wall rows are part of every
 // launch's longest blocks: gathered face by face, with a division per halo row
 // and stage / as corrections of the inside formula (below), a step of the sweep

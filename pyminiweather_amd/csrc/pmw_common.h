@@ -6,7 +6,7 @@
 // -ffp-contract=off, so that they round like the NumPy code they replace. The
 // expected differences from NumPy are fewer roundings in the fluxes' advective
 // and viscous terms (flux_x_face), last-bit differences of the powers
-// (pow_gamma of pmw_pow.h is correctly rounded in all but ~1e-7 of cases,
+// (pow_gamma of pmw_pow.h is correctly rounded in all but one of 3e6 cases,
 // glibc's pow, which NumPy calls, in all but 8e-4) and of exp/cos in the
 // initial conditions.
 #pragma once

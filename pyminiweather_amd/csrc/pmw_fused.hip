@@ -317,7 +317,8 @@ __device__ __forceinline__ void member_offset(DirArgs& a) {
   if (a.s1) a.s1 += off;
 }
 
-// Registers: K = 1 fits 6 waves per SIMD (78 VGPRs), K = 2 five (96).
+// Registers: K = 1 fits 6 waves per SIMD (74 VGPRs), K = 2 five (94; 96 with the
+// inflow, which spills one).
 constexpr int xw_waves_per_simd(int K) { return K == 1 ? 6 : 5; }
 
 __device__ __forceinline__ unsigned xw_wave(int block) {
@@ -1296,10 +1297,14 @@ bool fused_x_tile_ok(int nt) {
 // the slots on wave overlap instead of 23 % and halve the neighbour exchange
 // per cell, but each wave takes twice as long: one cell per lane is faster
 // while all its waves (one per 52 slots) fit the 6 x 1024 the GPU holds at
-// once. Step time in us, one / two cells per lane (x kernel: see above):
-// 400x200 17.9 / 18.7, 800x400 (just over one round of waves) 28.9 / 27.3,
-// 1003x517 39.1 / 40.4, 1200x600 47.7 / 47.9, 1500x750 66.6 / 63.6,
-// 2000x1000 104.8 / 99.2.
+// once. Step time in us, one / two cells per lane: 200x100 10.7 / 11.9, 400x200
+// 12.6 / 12.8, 700x350 21.0 / 21.6, 774x387 23.3 / 23.1, 800x400 (just over one
+// round of waves) 23.9 / 22.9, 900x450 25.3 / 25.1, 1003x517 29.1 / 29.8, 1100x550
+// 32.7 / 33.1, 1200x600 36.9 / 36.6, 1500x750 50.7 / 49.2, 2000x1000 78.4 / 74.9,
+// 4096x2048 367 / 334; with the inflow 400x200 13.4 / 14.5, 800x400 24.7 / 24.5,
+// 1003x517 31.4 / 31.8, 2000x1000 81.9 / 76.9. The cost goes by rounds of waves, so
+// a line by cells is up to 2.5 % off between 500000 and 600000 cells, where one
+// cell per lane fills its second round.
 int fused_x_cells(int nt, long long cells) {
   if (nt == 256 || nt == 1512) return nt == 256 ? 1 : 2;
   return cells <= 300000 ? 1 : 2;
@@ -1315,9 +1320,10 @@ bool fused_z_seg_ok(int seg) {
 // 8 to 64 the small ones; the others go by size. The three-row tiles need
 // edge tiles that reach past their own rows into the grid only (nz >= 46 for
 // their smallest) and 32-bit offsets inside a tile; they win once their blocks
-// fill the GPU. Step time in us, one-cell tiles of 32 rows / three-row tiles of
-// 48: 600x300 18.3 / 20.3, 700x350 22.2 / 21.2, 1000x300 24.8 / 25.9, 800x400
-// 25.4 / 24.6, 2000x200 29.9 / 29.2, 4000x100 31.3 / 30.0, 900x500 31.1 / 29.5.
+// fill the GPU. Step time in us, one-cell tiles of 32 rows / three-row tiles:
+// 800x400 23.3 / 22.9, 900x450 27.8 / 25.1, 1003x517 32.3 / 29.8, 1500x750 57.9 /
+// 49.2, 2000x1000 93.1 / 74.7; below the line, with earlier x kernels, 600x300 18.3 /
+// 20.3, 700x350 22.2 / 21.2, 1000x300 24.8 / 25.9.
 // Against one-cell tiles of 96 rows, which remain for columns and rows outside
 // those bounds: 10000x50 40.1 / 40.1, x60 43.3 / 41.4, x80 45.4 / 42.3, x93
 // 66.4 / 53.0.

@@ -1,12 +1,14 @@
-// pmw_pow.h -- x^y for the pressure p = C0 (rho*theta)^gamma (and dp/dq).
+// pmw_pow.h -- x^gamma for the pressure p = C0 (rho*theta)^gamma, and dp/dq.
 //
-// The flux kernels evaluate one such power per face; the general device pow
-// (about 220 instructions for gfx950, two thirds of the flux arithmetic)
-// also handles negative, zero, infinite and integer-exponent cases that a
-// density times a potential temperature never reaches. pow_pos evaluates
-// x^y = exp(y ln x) for positive finite x with two small tables
-// (pmw_pow_tables.h, generated by gen_pow_tables.py) and double-double
-// arithmetic where the rounding matters. The scheme is Tang's table-driven
+// The kernels evaluate one power per face: pow_gamma in the fluxes, the
+// background and the energy, pow_gamma_minus_one in the adjoint. Both take the
+// fixed exponent into their tables (pmw_pow_tables.h, generated by
+// gen_pow_tables.py). The powers of any exponent before them, pow_pos and its
+// relatives, are what kernels used earlier; no kernel calls them any more, and
+// the host tests hold them and, through them, the tables' generator.
+//
+// pow_pos evaluates x^y = exp(y ln x) for positive finite x with two small tables
+// and double-double arithmetic where the rounding matters. The scheme is Tang's table-driven
 // one (P. T. P. Tang, "Table-driven implementation of the logarithm function
 // in IEEE floating-point arithmetic", ACM TOMS 16(4), 1990, and "... of the
 // exponential function", ACM TOMS 15(2), 1989: reduce with a table entry,
@@ -65,8 +67,8 @@ PMW_HD double two_sum(double a, double b, double& lo) {
 
 // 1/x within an ulp or two for normal x (v_rcp_f64 and two Newton steps,
 // enough from any start better than 2^-13) on the device; RN(1/x) on the
-// host. Only pow_pos_near's reference uses it: pow_pos_near stays equal to
-// pow_pos with rx off by up to ~1e-14 relative (tests/test_pow_host.py;
+// host. The adjoint's quotients by rho are products with it; pow_pos_near stays
+// equal to pow_pos with rx off by up to ~1e-14 relative (tests/test_pow_host.py;
 // at 1e-13 it no longer is, through the e^2 terms evaluated from eh).
 PMW_HD double rcp_approx(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -234,10 +236,8 @@ PMW_HD double pow_pos_near(double x, double y, const PowRef& ref) {
 
 // x^y to within a few 1e-15 relative (measured on the host for x in
 // [1e-3, 1e5]) for positive finite x and 0 < y <= 1.5: the same reductions
-// in plain double arithmetic. For the
-// adjoint's dp/dq = gamma C0 q^(gamma-1), where a derivative needs no last
-// bit; about a third of pow_pos's instructions. Non-positive or non-finite x
-// give NaN.
+// in plain double arithmetic, for a derivative that needs no last bit; about a
+// third of pow_pos's instructions. Non-positive or non-finite x give NaN.
 PMW_HD double pow_pos_fast(double x, double y) {
   using namespace powt;
   const bool fin = x > 0.0 && x < __builtin_inf();
